@@ -275,42 +275,90 @@ __device__ __forceinline__ double lj_energy(double r, const LJPair& p) {
   return 0.0;
 }
 
-// Real-space pair sum over the reference's image range
-// (PotentialEwaldCoul::PairEnergyReal, potential_ewald_coul.cc:134-164).
-__device__ inline double real_pair_ref(const double* a, double qa, const double* b,
-                                       double qb, const Geo& g) {
-  if (qa * qb == 0) return 0.0;
-  double d[3];
-  min_image(a, b, g.L, g.npbc, d);
-  double pref = g.lB * qa * qb;
+// Minimum-image separation b - a in the Ewald box (x, y and, with three
+// periodic dimensions, z), the quotient taken with the reciprocal edge: it
+// differs from min_image only where |d| is half an edge to the last bit, and
+// there both images are in the image sum or both are beyond every cutoff.
+__device__ __forceinline__ void min_image_inv(const double* a, const double* b, const double* L, const double* inv_L,
+                                              int npbc, double* d) {
+#pragma unroll
+  for (int i = 0; i < 3; i++) {
+    double di = b[i] - a[i];
+    if (i < npbc) di -= L[i] * rint(di * inv_L[i]);
+    d[i] = di;
+  }
+}
+
+// Real-space sum of a unit prefactor over the reference's image range
+// (PotentialEwaldCoul::PairEnergyReal, potential_ewald_coul.cc:134-164) at
+// the separation d: sum of erfc(sqrt(alpha) r) / r over the images within rc.
+// Along each dimension only the offsets that can bring that component within
+// rc are visited (the test widened by a rounding margin), in the order of the
+// full loop, so the sum is the full loop's: the others add
+// nothing.  In a box with 2 rc > L (27 images) one or two offsets a dimension
+// remain, and a pair costs its in-range images instead of 27 square roots (the
+// pressure sample of 3,200 beads with r_c = 42 and L = 60, 5.1 million pairs:
+// 824 -> 645 us).
+__device__ inline double real_images(const double* d, const double* L, const double* inv_L, const Geo& g) {
+  const double rcw = g.rc * (1 + 1e-9), rc2w = rcw * rcw;
+  int lo[3], hi[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const double m = rcw + 1e-9 * L[k];
+    lo[k] = max(-g.real_cell[k], (int)ceil((-m - d[k]) * inv_L[k]));
+    hi[k] = min(g.real_cell[k], (int)floor((m - d[k]) * inv_L[k]));
+  }
   double e = 0;
-  for (int i = -g.real_cell[0]; i <= g.real_cell[0]; i++)
-    for (int j = -g.real_cell[1]; j <= g.real_cell[1]; j++)
-      for (int k = -g.real_cell[2]; k <= g.real_cell[2]; k++) {
-        double x = d[0] + i * g.L[0], y = d[1] + j * g.L[1], z = d[2] + k * g.L[2];
-        double r = sqrt(x * x + y * y + z * z);
-        if (r > 0 && r <= g.rc) e += pref * erfc_nodes(g, g.sqrt_alpha * r) / r;
+  for (int i = lo[0]; i <= hi[0]; i++) {
+    const double x = d[0] + i * L[0];
+    for (int j = lo[1]; j <= hi[1]; j++) {
+      const double y = d[1] + j * L[1];
+      const double xy2 = x * x + y * y;
+      if (xy2 > rc2w) continue;
+      for (int k = lo[2]; k <= hi[2]; k++) {
+        const double z = d[2] + k * L[2];
+        const double r = sqrt(xy2 + z * z);
+        if (r > 0 && r <= g.rc) e += erfc_nodes(g, g.sqrt_alpha * r) / r;
       }
+    }
+  }
   return e;
 }
 
-// The same pair sum when only the minimum image can lie within rc: every
-// periodic edge is longer than 2 rc (g.single_image), and along a
+// True when only the image at the minimum-image separation d can lie within
+// rc: every periodic edge is longer than 2 rc (g.single_image), and along a
 // non-periodic z the separation is shorter than the padded period minus rc.
-// It is then the (0, 0, 0) term of the image loop above, equal to that loop
-// bit for bit since every other image falls beyond rc.
-__device__ __forceinline__ double real_pair(const double* a, double qa, const double* b, double qb,
-                                           const Geo& g) {
+__device__ __forceinline__ bool one_image(const double* d, double Lz, const Geo& g) {
+  return g.single_image && (g.npbc == 3 || fabs(d[2]) + g.rc * (1 + 1e-9) < Lz);
+}
+
+// Real-space pair energy of a and b, every image within rc.
+__device__ __forceinline__ double real_pair(const double* a, double qa, const double* b, double qb, const Geo& g) {
   if (qa * qb == 0) return 0.0;
   double d[3];
-  min_image(a, b, g.L, g.npbc, d);
-  if (!g.single_image || (g.npbc < 3 && !(fabs(d[2]) + g.rc * (1 + 1e-9) < g.L[2])))
-    return real_pair_ref(a, qa, b, qb, g);
+  min_image_inv(a, b, g.L, g.inv_L, g.npbc, d);
   const double pref = g.lB * qa * qb;
+  if (!one_image(d, g.L[2], g)) return pref * real_images(d, g.L, g.inv_L, g);
   const double r = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
-  double e = 0;
-  if (r > 0 && r <= g.rc) e += pref * erfc_nodes(g, g.sqrt_alpha * r) / r;
-  return e;
+  return (r > 0 && r <= g.rc) ? pref * erfc_nodes(g, g.sqrt_alpha * r) / r : 0.0;
+}
+
+// LJ (minimum image, BBDist) and real-space energy of one explicit bead pair
+// (charges in .w), w times each added to elj and ere.  Both terms share one
+// separation: x and y have the same period in both, and z is wrapped only
+// with three periodic dimensions, where the Ewald box is the simulation box.
+__device__ __forceinline__ void pair_both(const double4& a, const double4& b, const LJPair& lp, const Geo& g,
+                                          double w, double& elj, double& ere) {
+  const double av[3] = {a.x, a.y, a.z}, bv[3] = {b.x, b.y, b.z};
+  double d[3];
+  min_image_inv(av, bv, g.L, g.inv_L, g.npbc, d);
+  const double r = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+  if (g.use_pair) elj += w * lj_energy(r, lp);
+  const double qq = a.w * b.w;
+  if (!g.use_ewald || qq == 0) return;
+  const double pref = w * g.lB * qq;
+  if (!one_image(d, g.L[2], g)) ere += pref * real_images(d, g.L, g.inv_L, g);
+  else if (r > 0 && r <= g.rc) ere += pref * erfc_nodes(g, g.sqrt_alpha * r) / r;
 }
 
 // PotentialTruncatedLJWall::BeadEnergy (potential_truncated_lj_wall.cc:46-134)

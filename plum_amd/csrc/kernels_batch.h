@@ -958,16 +958,11 @@ __device__ void cross_block(const Geo& g, const Dev& d, const RepCfg& rc, int sp
     const int i = t / np_, j = t - (t / np_) * np_;
     const int si = sq * rc.maxm + i, sj = sp * rc.maxm + j;
     const double4 a0 = d.mv_old[si], a1 = d.mv_new[si], b0 = d.mv_old[sj], b1 = d.mv_new[sj];
-    const double ao[3] = {a0.x, a0.y, a0.z}, an[3] = {a1.x, a1.y, a1.z};
-    const double bo[3] = {b0.x, b0.y, b0.z}, bn[3] = {b1.x, b1.y, b1.z};
-    if (g.use_pair) {
-      const LJPair lp = d.lj[d.mv_type[si] * g.n_types + d.mv_type[sj]];
-      elj = lj_energy(bb_dist(an, bn, g.Lsim, g.npbc), lp) - lj_energy(bb_dist(ao, bn, g.Lsim, g.npbc), lp) -
-            lj_energy(bb_dist(an, bo, g.Lsim, g.npbc), lp) + lj_energy(bb_dist(ao, bo, g.Lsim, g.npbc), lp);
-    }
-    if (g.use_ewald && a0.w * b0.w != 0)
-      ere = real_pair(an, a1.w, bn, b1.w, g) - real_pair(ao, a0.w, bn, b1.w, g) -
-            real_pair(an, a1.w, bo, b0.w, g) + real_pair(ao, a0.w, bo, b0.w, g);
+    const LJPair lp = d.lj[d.mv_type[si] * g.n_types + d.mv_type[sj]];
+    pair_both(a1, b1, lp, g, 1.0, elj, ere);
+    pair_both(a0, b1, lp, g, -1.0, elj, ere);
+    pair_both(a1, b0, lp, g, -1.0, elj, ere);
+    pair_both(a0, b0, lp, g, 1.0, elj, ere);
   }
   const double a = block_sum<kBlock>(elj, sh);
   const double c = block_sum<kBlock>(ere, sh);

@@ -193,13 +193,9 @@ __device__ void mm_block(const Geo& g, const Dev& d, int blk, int nblk, double* 
     long long b = pidx - a * (2LL * nm - a - 1) / 2 + a + 1;
     if (b >= nm) b = nm - 1;
     const double4 na4 = d.mv_new[a], nb4 = d.mv_new[b], oa4 = d.mv_old[a], ob4 = d.mv_old[b];
-    const double na[3] = {na4.x, na4.y, na4.z}, nb[3] = {nb4.x, nb4.y, nb4.z};
-    const double oa[3] = {oa4.x, oa4.y, oa4.z}, ob[3] = {ob4.x, ob4.y, ob4.z};
-    if (g.use_pair) {
-      const LJPair lp = d.lj[d.mv_type[a] * g.n_types + d.mv_type[b]];
-      elj += lj_energy(bb_dist(na, nb, g.Lsim, g.npbc), lp) - lj_energy(bb_dist(oa, ob, g.Lsim, g.npbc), lp);
-    }
-    if (g.use_ewald) ere += real_pair(na, na4.w, nb, nb4.w, g) - real_pair(oa, oa4.w, ob, ob4.w, g);
+    const LJPair lp = d.lj[d.mv_type[a] * g.n_types + d.mv_type[b]];
+    pair_both(na4, nb4, lp, g, 1.0, elj, ere);
+    pair_both(oa4, ob4, lp, g, -1.0, elj, ere);
   }
   const double a = block_sum<kBlock>(elj, sh);
   const double c = block_sum<kBlock>(ere, sh);

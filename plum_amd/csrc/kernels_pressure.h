@@ -41,23 +41,13 @@ __device__ inline double real_pair_stretch(const double* a, double qa, const dou
                                            const Geo& g) {
   if (qa * qb == 0) return 0.0;
   const double Ls[3] = {g.L[0], g.L[1], g.L[2] + kDz};
+  const double inv_Ls[3] = {g.inv_L[0], g.inv_L[1], 1.0 / Ls[2]};
   double d[3];
-  min_image(a, b, Ls, g.npbc, d);
+  min_image_inv(a, b, Ls, inv_Ls, g.npbc, d);
   const double pref = g.lB * qa * qb;
-  double e = 0;
-  if (g.single_image && (g.npbc == 3 || fabs(d[2]) + g.rc * (1 + 1e-9) < Ls[2])) {
-    const double r = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
-    if (r > 0 && r <= g.rc) e += pref * erfc_nodes(g, g.sqrt_alpha * r) / r;
-    return e;
-  }
-  for (int i = -g.real_cell[0]; i <= g.real_cell[0]; i++)
-    for (int j = -g.real_cell[1]; j <= g.real_cell[1]; j++)
-      for (int k = -g.real_cell[2]; k <= g.real_cell[2]; k++) {
-        const double x = d[0] + i * Ls[0], y = d[1] + j * Ls[1], z = d[2] + k * Ls[2];
-        const double r = sqrt(x * x + y * y + z * z);
-        if (r > 0 && r <= g.rc) e += pref * erfc_nodes(g, g.sqrt_alpha * r) / r;
-      }
-  return e;
+  if (!one_image(d, Ls[2], g)) return pref * real_images(d, Ls, inv_Ls, g);
+  const double r = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+  return (r > 0 && r <= g.rc) ? pref * erfc_nodes(g, g.sqrt_alpha * r) / r : 0.0;
 }
 
 // Unordered bead pairs a <= b (bead order is molecule order, so these are the

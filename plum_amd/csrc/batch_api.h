@@ -189,12 +189,13 @@ int batch_upload_state(plum_batch* b) {
     q.nkb_s = c->nkb_s;
     q.nrun = c->nrun;
     q.qfill = b->n_cu * std::min(b->comp_occ, b->tune.blocks_per_cu) * kQWaves;
-    q.nsplit = c->nsplit;
+    q.qmax = query_split(c->cand, kQShare, b->tune.split_div);
+    q.qfine = query_split(c->cand, kQFine, b->tune.split_div);
     q.ncell = c->g.ncell;
     q.pmax = b->tune.pmax;
     q.maxm = c->maxm;
     q.nmmb = c->nmmb;
-    q.rstride = 2 * c->maxm * kMaxQWave;
+    q.rstride = query_blocks(c->maxm, kMaxQBlock) * kQWaves;
     q.xcap = c->xcap;
     q.da = b->da ? 1 : 0;
     q.train = (b->da && r == 0) ? 1 : 0;

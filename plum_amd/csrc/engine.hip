@@ -245,11 +245,16 @@ void set_cell_grid(plum_ctx* c, int div) {
 }
 
 // Expected candidate slots of a real-space query (the cells within the search
-// radius of a point) and the query split it gives.
+// radius of a point) and the query split it gives.  With two periodic
+// dimensions the beads fill the simulation box only, not the padding of the
+// Ewald box (a brush 40 high in a box of 190: 16,600 candidates, not 3,500).
 void set_cand(plum_ctx* c) {
   const Geo& g = c->g;
-  double cand = g.n / c->info.vol_e;
-  for (int k = 0; k < 3; k++) cand *= 2 * g.rs + g.h[k];
+  double cand = g.n;
+  for (int k = 0; k < 3; k++) {
+    const double w = 2 * g.rs + g.h[k];
+    cand *= k < g.npbc ? w / g.L[k] : std::min(1.0, w / g.Lsim[k]);
+  }
   c->cand = cand;
   c->nsplit = split_for(cand, kDefaultSplitDiv);
 }
@@ -457,6 +462,7 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
   g.rs = std::max(g.rc, lj_max);
   if (g.rs <= 0) g.rs = 1.0;
   g.rs2 = g.rs * g.rs;
+  g.lj2_max = lj_max * lj_max * (1 + 1e-12);
 
   // cell grid: edge ~ rs / div
   set_cell_grid(c, p.cell_div > 0 ? p.cell_div : 2);
@@ -572,7 +578,7 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
   ALLOC(d.ctl, 1);
   set_cand(c);
   // room for any split (the batch autotuner may change it)
-  ALLOC(d.part_k, c->nkb); ALLOC(d.part_r, (size_t)kMaxProp * 2 * maxm * kMaxQWave);
+  ALLOC(d.part_k, c->nkb); ALLOC(d.part_r, (size_t)kMaxProp * std::max(query_blocks(maxm, kMaxQBlock) * kQWaves, 2 * maxm * kMaxSplit));
   ALLOC(d.part_mm, (size_t)kMaxProp * c->nmmb);
   ALLOC(d.sk_part, (size_t)c->nchunk * std::max(1, g.n_kh));
   ALLOC(c->epart_k, c->nkb_full);

@@ -38,6 +38,7 @@ struct Geo {
   int n_types;
   double rc;         // real-space cutoff (reference's derived value)
   double rs, rs2;    // search radius = max(rc, largest LJ cutoff)
+  double lj2_max;    // square of the largest LJ cutoff, widened by a rounding margin
   double sqrt_alpha, lB;
   double self_coef;  // -lB sqrt(alpha/kPi)
   double dip_coef;   // lB 2 kPi / V_e
@@ -80,28 +81,43 @@ __device__ __forceinline__ int erfc_node_index(double x) {
   return x < kErfcMax ? max(0, (int)(x * kErfcPerUnit + 0.5)) : 0;
 }
 
+// A constant put into scalar registers where it is used: the compiler
+// otherwise hoists the series' sixteen 64-bit constants out of the pair loops
+// into 32 vector registers and spills others.
+__device__ __forceinline__ double scalar_const(double v) {
+  asm volatile("" : "+s"(v));
+  return v;
+}
+
 // erfc(x) from its node i = erfc_node_index(x) and the node's table entry.
+// With y = -2 x_i t the terms (-1)^n H_n(x_i) t^n regroup by powers of t^2:
+//   sum_n (-1)^n H_n(x_i) t^n / (n+1)! = sum_k (-t^2)^k / k! sum_m y^m / (m! (m + 2k + 1)),
+// the k = 0 sum being (e^y - 1) / y.  |y| <= 1/16 and t^2 <= 1.6e-5, so eight,
+// six and three terms of k = 0, 1, 2 hold what the first eight n hold, in 20
+// operations of which most are fused, instead of 38 by the recurrence for H_n.
 __device__ __forceinline__ double erfc_from_node(double x, int i, double2 node) {
   if (!(x < kErfcMax)) return 0.0;
   const double xi = (double)i * (1.0 / kErfcPerUnit);
   const double t = x - xi;   // exact: x and x_i are within a factor of 2 (or x_i = 0)
-  // q_n = (-1)^n H_n(x_i): q_0 = 1, q_1 = -2 x_i, q_{n+1} = -2 x_i q_n - 2 n q_{n-1};
-  // w_n = t^{n+1} / (n+1)!
-  const double m2x = -2.0 * xi;
-  double qm = 1.0, q = m2x;
-  double w = t;
-  double s = w;
-  w *= t * 0.5;
-  s += q * w;
-#pragma unroll
-  for (int n = 1; n < 7; n++) {
-    const double qn = m2x * q - (2.0 * n) * qm;
-    qm = q;
-    q = qn;
-    w *= t * (1.0 / (n + 2));
-    s += q * w;
-  }
-  return node.x - node.y * s;
+  const double y = -2.0 * xi * t, t2 = t * t;
+  double p0 = scalar_const(1.0 / 40320.0);
+  p0 = fma(p0, y, scalar_const(1.0 / 5040.0));
+  p0 = fma(p0, y, scalar_const(1.0 / 720.0));
+  p0 = fma(p0, y, scalar_const(1.0 / 120.0));
+  p0 = fma(p0, y, scalar_const(1.0 / 24.0));
+  p0 = fma(p0, y, scalar_const(1.0 / 6.0));
+  p0 = fma(p0, y, 0.5);
+  double p1 = scalar_const(1.0 / 960.0);
+  p1 = fma(p1, y, scalar_const(1.0 / 168.0));
+  p1 = fma(p1, y, scalar_const(1.0 / 36.0));
+  p1 = fma(p1, y, scalar_const(0.1));
+  p1 = fma(p1, y, scalar_const(0.25));
+  p1 = fma(p1, y, scalar_const(1.0 / 3.0));
+  double p2 = fma(scalar_const(1.0 / 14.0), y, scalar_const(1.0 / 6.0));
+  p2 = fma(p2, y, scalar_const(0.2));
+  // s / t - 1: the leading 1 is added to t last
+  const double r = fma(t2, fma(0.5 * t2, p2, -p1), p0 * y);
+  return fma(-node.y, fma(t, r, t), node.x);
 }
 
 __device__ __forceinline__ double erfc_nodes(const Geo& g, double x) {
@@ -273,6 +289,25 @@ __device__ __forceinline__ double lj_energy(double r, const LJPair& p) {
     return 4 * p.eps * (r6 * r6 - r6) - p.shift;
   }
   return 0.0;
+}
+
+// r = sqrt(r2) and 1 / r together for r2 > 0 (normal numbers): the hardware
+// estimate, two Goldschmidt steps and a last residual correction of each.
+// Both within an ulp, for about half of what a square root and a division
+// cost one after the other.
+__device__ __forceinline__ void sqrt_rsqrt(double r2, double& r, double& rinv) {
+  const double y = __builtin_amdgcn_rsq(r2);
+  double g = r2 * y, h = 0.5 * y;
+  double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  g = fma(fma(-g, g, r2), h, g);
+  const double z = h + h;
+  r = g;
+  rinv = fma(fma(-g, z, 1.0), z, z);
 }
 
 // Minimum-image separation b - a in the Ewald box (x, y and, with three

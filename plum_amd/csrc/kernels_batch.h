@@ -53,7 +53,7 @@ constexpr int kKSpec = 32;             // k-vector runs per speculative k-space 
 // Per-system launch shape.
 struct RepCfg {
   int nkb_s;    // k-space blocks of kKSpec runs (0 without Ewald)
-  int nsplit;   // blocks per real-space query
+  int qmax, qfine;   // blocks of a real-space query, ordinary and on an idle chip (query_split)
   int ncell;    // cells
   int pmax;     // proposals per batch (<= kMaxProp, <= kMaxScreen with the surrogate)
   int maxm;     // moved-list capacity per proposal (longest molecule)
@@ -70,26 +70,38 @@ struct RepCfg {
 
 // Real-space query blocks of a move of nm beads: one query per cluster of up
 // to kCluster consecutive moved beads at their old and one at their new
-// positions, qw waves per query (each takes a share of the candidate slots),
+// positions, qb blocks per query (each takes a share of the query's cells),
 // kQWaves waves per block.
 constexpr int kQWaves = kBlock / kWave;
-constexpr int kMaxQWave = 4 * kMaxSplit;
-// One wave per split share; a batch with few exact proposals (fewer than 16
-// over all systems) spreads each query over four times as many waves, as its
-// queries alone would leave most of the chip idle, unless the system's own
-// query waves (its exact slots' clusters at old and new positions, times the
-// shares) would then outnumber the waves the chip holds at once (fill).  The
-// plan chooses it per batch from the exact slots it assigned (with delayed
-// acceptance most screened proposals never reach the queries).
-__host__ __device__ __forceinline__ int query_waves(int nsplit, int proposals, int clusters, int fill) {
-  if (nsplit == 1 || proposals >= 16) return nsplit;
-  return (long long)clusters * nsplit * kQWaves <= fill ? kQWaves * nsplit : nsplit;
+constexpr int kMaxQBlock = 8;
+constexpr int kQShare = 1000;  // candidate slots per block of a query at the default split_div
+constexpr int kQFine = 480;    // the same where the queries leave the chip idle
+// Most blocks of a query of `cand` expected candidate slots, `share` slots
+// each at the default split_div.
+__host__ __device__ __forceinline__ int query_split(double cand, int share, int split_div) {
+  const double s = share * (double)split_div / kDefaultSplitDiv;
+  return max(1, min(kMaxQBlock, (int)(cand / s + 0.5)));
+}
+// Blocks per query of a system with `clusters` queries in the batch (its own
+// only: a system's sums do not depend on the systems beside it).  A query wave
+// is a serial chain (cell list, candidate loads, pair drains) that ends the
+// launch when it is long, but each more block of a query repeats its set-up:
+// shares of about kQShare candidates (qmax blocks) are the shortest launches
+// where a batch has its 16 proposals (k_compute_spec of the 40,000-bead system
+// at 500, 1,000 and 2,000 a block: 57, 46 and 46 us; 1,000 beads: 31, 28 and
+// 33), kQFine (qfine blocks) where few proposals leave most of the chip idle
+// (delayed acceptance on the brush: 50 and 35 us).  More query waves than 5/8
+// of what the chip holds at once (fill; the other blocks take the rest) start
+// a second round: a query is spread no further (the brush at 16 and 32 waves a
+// query: 71 and 110 us).
+__host__ __device__ __forceinline__ int query_spread(int qmax, int qfine, int clusters, int fill) {
+  if (clusters < 1) clusters = 1;
+  const int want = 5 * fill / 8 / kQWaves / clusters, idle = fill / 4 / kQWaves / clusters;
+  return max(max(1, min(want, qmax)), min(idle, qfine));
 }
 constexpr int kCluster = 8;   // moved beads per real-space query (cluster)
 __host__ __device__ __forceinline__ int query_clusters(int nm) { return (nm + kCluster - 1) / kCluster; }
-__host__ __device__ __forceinline__ int query_blocks(int nm, int qw) {
-  return (2 * query_clusters(nm) * qw + kQWaves - 1) / kQWaves;
-}
+__host__ __device__ __forceinline__ int query_blocks(int nm, int qb) { return 2 * query_clusters(nm) * qb; }
 
 // k-space blocks per k block: one wave per exact slot.
 __host__ __device__ __forceinline__ int kspace_groups(int ne) { return (ne + kQWaves - 1) / kQWaves; }
@@ -462,17 +474,16 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan_spec(const Geo* __restric
       if (exact >= 0) sm.s_screen[exact] = t;
     }
     wave_sync_lds();
-    // waves per query for this batch's exact slots (the other systems of a
-    // batch taken to have as many), then query and moved-moved blocks per
-    // exact slot, prefixes over the slots
+    // blocks per query for this batch's exact slots, then query and
+    // moved-moved blocks per exact slot, prefixes over the slots
     int ncl = t < ne ? 2 * query_clusters(sm.s_prop[sm.s_screen[t]].n) : 0;
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) ncl += __shfl_xor(ncl, o, kWave);
-    const int qw = query_waves(rc.nsplit, ne * R, ncl, rc.qfill);
+    const int qb = query_spread(rc.qmax, rc.qfine, ncl, rc.qfill);
     int nq = 0, nmb = 0;
     if (t < ne) {
       const int n = sm.s_prop[sm.s_screen[t]].n;
-      nq = n > 0 ? query_blocks(n, qw) : 0;
+      nq = n > 0 ? query_blocks(n, qb) : 0;
       nmb = n > 0 ? nmm_blocks(n) : 0;
       plan->screen_of[t] = sm.s_screen[t];
     }
@@ -490,7 +501,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan_spec(const Geo* __restric
     }
     const int off = ne > 0 ? __shfl(nq, ne - 1, kWave) + __shfl(nmb, ne - 1, kWave) : 0;
     if (t == 0) {
-      plan->qwave = qw;
+      plan->qblk = qb;
       plan->q_off[0] = 0;
       plan->mm_off[0] = 0;
       plan->n_decide = ndec;
@@ -651,107 +662,76 @@ __device__ void kspace_spec_wave(const Geo& g, const Dev& d, const RepCfg& rc, c
 }
 
 // ------------------------------------------------------------ real space
-// Cluster queries, one per wave (kQWaves per block, no block barriers): a wave
-// takes up to kCluster consecutive moved beads of one proposal, all at their
-// old or all at their new positions (the query points), and one share of the
-// candidate slots of the cells within the search radius of the points'
-// bounding box.  The wave lists those cells 64 at a time with a wave prefix
-// over their counts; each lane takes candidate slots lane, lane + 64, ...
-// (bead index, position and type loaded together, one candidate ahead) and
-// tests its candidate against every point, so a candidate's load, cell
-// lookup and image decode serve all the points.  The pairs within the radius
-// go into a per-wave queue in LDS (ballot + lane prefix); each time the queue
-// holds 64 pairs every lane takes one and evaluates its LJ and erfc terms, so
-// the lanes never diverge on the pair arithmetic.  A wave reduction sums the
-// lanes in fixed order.  Same pair terms as real_query.
-constexpr int kQueue = 2 * kWave;   // pair queue of one wave (holds < 2 fills)
+// Cluster queries: a block takes up to kCluster consecutive moved beads of one
+// proposal, all at their old or all at their new positions (the query
+// points), and one share of the cells within the search radius of the points'
+// bounding box.  Its threads list the share's cells together, one each, with a
+// block prefix over their counts, and its waves take 64 candidates in turn, so
+// the four of them end together and a cell is listed once.  Each lane takes a
+// candidate slot (bead index, position and type loaded together, one
+// candidate ahead) and tests it against every point, so a candidate's load,
+// cell lookup and image decode serve all the points.  The charged pairs within
+// the real-space cutoff go into a per-wave queue in LDS (ballot + lane
+// prefix), last in first out; each time it holds 64 pairs every lane takes one
+// and evaluates its erfc term, so the lanes never diverge on the pair
+// arithmetic.  Pairs within the largest LJ cutoff, one in a hundred at r_c =
+// 12, have a queue of their own: in the common one they cost nearly every
+// drain the LJ table load and arithmetic.  A wave reduction sums the lanes in
+// fixed order.  Bound by VALU issue: about 150 instructions per 64 pairs
+// (distance tests of three candidates for each pair in range, queue, erfc).
+constexpr int kQueue = 2 * kWave;   // < 64 left after a drain, one push of up to 64
 static_assert(kCluster <= kWave, "one lane per query point");
 
 template <int P>
 struct QWaveSmem {
-  int s_cell[kWave];
-  int s_img[kWave];
-  int s_end[kWave];
-  double4 s_pt[kCluster];  // query points (the image nearest the first point) and charges
-  int s_ptt[kCluster];     // their types
-  double s_r2[kQueue];     // squared distance of a queued pair
-  double s_qq[kQueue];     // its charge product
-  int s_t[kQueue];         // its LJ pair index | 1 << 24 when LJ applies (no z image in a slab)
-  // P = 1: the queue of pairs at or beyond fp64_below, evaluated in FP32
-  double s_fr2[P ? kQueue : 1];
-  float s_fqq[P ? kQueue : 1];
-  int s_ft[P ? kQueue : 1];
+  double2 s_q[kQueue];     // squared distance and charge product of a queued pair
+  double s_lr[kQueue];     // squared distance of a queued LJ pair
+  int s_lt[kQueue];        // its LJ pair index
+  // P = 1: the queue of charged pairs at or beyond fp64_below, evaluated in FP32
+  float2 s_f[P ? kQueue : 1];
 };
 
-// LJ + real-space terms of one queued pair (squared distance r2 <= rs^2,
-// charge product qq, LJ pair index lji, whether LJ applies), FP64.  Both table
-// entries (LJ pair, erfc node) are loaded before either is used, so that a
-// queue drain waits for memory once rather than twice in a row: the empty asm
-// takes them as inputs, which keeps the loads ahead of both branches.
-__device__ __forceinline__ void pair_terms(const Geo& g, const Dev& d, double r2, double qq, int lji, bool lj_ok,
-                                           double& elj, double& ere) {
-  const double r = sqrt(r2);
-  const double x = g.sqrt_alpha * r;
-  const int ni = erfc_node_index(x);
-  const LJPair lp = d.lj[lji];
-  const double2 node = g.erfc_tab[ni];
-  asm volatile("" ::"v"(lp.sigma), "v"(lp.cut), "v"(node.x));
-  if (lj_ok) elj += lj_energy(r, lp);
-  if (g.use_ewald && qq != 0 && r > 0 && r <= g.rc) ere += g.lB * qq * erfc_from_node(x, ni, node) / r;
-}
-
-// The same in FP32 (the FP32 pair path, pairs at or beyond fp64_below; the
-// cutoff tests compare the FP64 squared distance), added to the FP64 sums.
-__device__ __forceinline__ void pair_terms32(const Geo& g, const Dev& d, double r2, float qq, int lji, bool lj_ok,
-                                             double& elj, double& ere) {
-  const float r2f = (float)r2;
-  const float rf = sqrtf(r2f);
-  const float x = (float)g.sqrt_alpha * rf;
-  const int ni = erfc_node_index32(x);
-  const LJPair32 lp = d.lj32[lji];
-  const float2 node = g.erfc_tab32[ni];
-  asm volatile("" ::"v"(lp.sigma2), "v"(lp.cut), "v"(node.x));
-  if (lj_ok) {
-    if (r2 < (double)lp.cut * (double)lp.cut) {
-      const float s2 = lp.sigma2 / r2f;
-      const float r6 = s2 * s2 * s2;
-      elj += (double)(lp.eps4 * (r6 * r6 - r6) - lp.shift);
-    }
-  }
-  if (g.use_ewald && qq != 0.f && r2 <= g.rc * g.rc) ere += (double)((float)g.lB * qq * erfc_from_node32(x, ni, node) / rf);
-}
+template <int P>
+struct QueryShare {
+  int s_cell[kBlock];      // cells of this share, their images and count prefix
+  int s_img[kBlock];
+  int s_end[kBlock];
+  int s_wsum[kQWaves];
+  double4 s_pt[kCluster];  // query points (the image nearest the first point) and charges
+  int s_ptt[kCluster];     // their types
+  QWaveSmem<P> q[kQWaves];
+};
 
 // LJ + real-space energy of the np points pts[0 .. np) (charges in .w, types
 // ptype[]) against every bead image in the cell list within the search
-// radius, skipping the index range [mlo, mhi] (contig) or the moved flags,
-// one wave taking share `part` of `nparts` of the candidate slots.  Result
-// valid in lane 0.
+// radius, skipping the index range [mlo, mhi] (the device loop's moves are
+// contiguous), over share `part` of `nparts` of the query's cells.  Each
+// wave's part of the result valid in its lane 0.
 template <int P>
 __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4* __restrict__ pts,
-                                      const int* __restrict__ ptype, int np, int contig, int mlo, int mhi, int part,
-                                      int nparts, QWaveSmem<P>& sm) {
-  const int lane = threadIdx.x % kWave;
+                                      const int* __restrict__ ptype, int np, int mlo, int mhi, int part, int nparts,
+                                      QueryShare<P>& sh) {
+  const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
+  QWaveSmem<P>& sm = sh.q[wv];
   // each point as the image nearest the first point's wrapped position (an
   // image of a point has the same pair images within the radius), and the
-  // points' bounding box
+  // points' bounding box; lane l holds point l % kCluster (the last one again
+  // past the end)
   double bl[3], bh[3];
   {
-    const double4 p0 = pts[0];
-    const double p0v[3] = {p0.x, p0.y, p0.z};
+    const int ip = min(lane % kCluster, np - 1);
+    const double4 p0 = pts[0], p = pts[ip];
+    const double p0v[3] = {p0.x, p0.y, p0.z}, pv[3] = {p.x, p.y, p.z};
     double qv[3];
 #pragma unroll
-    for (int k = 0; k < 3; k++) qv[k] = wrap_coord(p0v[k], g.L[k], g.inv_L[k]);
-    if (lane < np) {
-      const double4 p = pts[lane];
-      const double pv[3] = {p.x, p.y, p.z};
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        double dk = pv[k] - p0v[k];
-        dk -= g.L[k] * rint(dk * g.inv_L[k]);
-        qv[k] += dk;
-      }
-      sm.s_pt[lane] = make_double4(qv[0], qv[1], qv[2], p.w);
-      sm.s_ptt[lane] = ptype[lane];
+    for (int k = 0; k < 3; k++) {
+      double dk = pv[k] - p0v[k];
+      dk -= g.L[k] * rint(dk * g.inv_L[k]);
+      qv[k] = wrap_coord(p0v[k], g.L[k], g.inv_L[k]) + dk;
+    }
+    if (threadIdx.x < np) {
+      sh.s_pt[lane] = make_double4(qv[0], qv[1], qv[2], p.w);
+      sh.s_ptt[lane] = ptype[lane];
     }
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -759,7 +739,7 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4*
       bh[k] = qv[k];
     }
 #pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1)
+    for (int o = kCluster / 2; o > 0; o >>= 1)
 #pragma unroll
       for (int k = 0; k < 3; k++) {
         bl[k] = fmin(bl[k], __shfl_xor(bl[k], o, kWave));
@@ -780,41 +760,57 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4*
     nd[k] = hi - lo[k] + 1;
   }
   const int ncq = nd[0] * nd[1] * nd[2];
+  const int mine = (ncq + nparts - 1) / nparts;   // cells of this share, at most
   const int nt = g.n_types;
-  double elj = 0, ere = 0;
-  int qhead = 0, qn = 0;   // queue start and fill (wave-uniform)
-  int fhead = 0, fn = 0;   // the same for the FP32 queue (P = 1)
+  const double rc2 = g.use_ewald ? g.rc * g.rc : -1.0, lj2 = g.use_pair ? g.lj2_max : -1.0;
   const double fp64_b2 = P ? g.fp64_below * g.fp64_below : 0.0;
-  // the pairs queued at qhead .. qhead + count - 1, one per lane
+  double elj = 0, ere = 0;
+  int qn = 0, ln = 0, fn = 0;   // queue fills (wave-uniform)
+  // real-space terms of the pairs at the queue's end, one per lane
   auto drain = [&](int count) {
     wave_sync_lds();
-    if (lane < count) {
-      const int k = (qhead + lane) % kQueue;
-      const int t = sm.s_t[k];
-      pair_terms(g, d, sm.s_r2[k], sm.s_qq[k], t & 0xffffff, (t >> 24) != 0, elj, ere);
-    }
-    qhead = (qhead + count) % kQueue;
     qn -= count;
+    if (lane < count) {
+      const double2 e = sm.s_q[qn + lane];
+      double r, rinv;
+      sqrt_rsqrt(e.x, r, rinv);
+      const double x = g.sqrt_alpha * r;
+      const int ni = erfc_node_index(x);
+      const double u = erfc_from_node(x, ni, g.erfc_tab[ni]) * rinv;
+      if (e.x > 0) ere = fma(e.y, u, ere);
+    }
     wave_sync_lds();
   };
+  // the same in FP32 (pairs at or beyond fp64_below), added to the FP64 sum
   auto drain32 = [&](int count) {
     wave_sync_lds();
-    if (lane < count) {
-      const int k = (fhead + lane) % kQueue;
-      const int t = sm.s_ft[k];
-      pair_terms32(g, d, sm.s_fr2[k], sm.s_fqq[k], t & 0xffffff, (t >> 24) != 0, elj, ere);
-    }
-    fhead = (fhead + count) % kQueue;
     fn -= count;
+    if (lane < count) {
+      const float2 e = sm.s_f[fn + lane];
+      const float rf = sqrtf(e.x);
+      const float x = (float)g.sqrt_alpha * rf;
+      const int ni = erfc_node_index32(x);
+      ere += (double)(e.y * erfc_from_node32(x, ni, g.erfc_tab32[ni]) / rf);
+    }
     wave_sync_lds();
   };
-  wave_sync_lds();   // the points are in LDS
-  for (int base = 0; base < ncq; base += kWave) {
-    const int nloc = min(kWave, ncq - base);
+  auto drain_lj = [&](int count) {
+    wave_sync_lds();
+    ln -= count;
+    if (lane < count) elj += lj_energy(sqrt(sm.s_lr[ln + lane]), d.lj[sm.s_lt[ln + lane]]);
+    wave_sync_lds();
+  };
+  for (int base = 0; base < mine; base += kBlock) {
+    const int nloc = min(kBlock, mine - base);
     int end = 0;
-    if (lane < nloc) {
-      const int c = base + lane;
-      const int cz = c % nd[2], cy = (c / nd[2]) % nd[1], cx = c / (nd[2] * nd[1]);
+    if (threadIdx.x < nloc) {
+      // cell of this share in group `grp` of nparts cells: the shares change
+      // places from group to group (with a fixed place and nparts a multiple
+      // of a grid edge, one share would hold a whole layer of a slab and
+      // another the empty padding)
+      const int grp = base + threadIdx.x;
+      const int c = nparts * grp + (int)((part + (unsigned)grp * 40503u % 8191u) % (unsigned)nparts);
+      const int cyx = c / nd[2], cz = c - cyx * nd[2], cx = cyx / nd[1], cy = cyx - cx * nd[1];
       const int u[3] = {lo[0] + cx, lo[1] + cy, lo[2] + cz};
       int cell = 0, img = 0;
 #pragma unroll
@@ -824,11 +820,11 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4*
         cell = cell * g.nc[k] + w;
         img |= ((qk + 128) & 0xff) << (8 * k);
       }
-      sm.s_cell[lane] = cell;
-      sm.s_img[lane] = img;
+      sh.s_cell[threadIdx.x] = cell;
+      sh.s_img[threadIdx.x] = img;
       // cells whose box (widened by a rounding margin) lies beyond the search
       // radius of the bounding box hold no candidate
-      double dmin2 = 0;
+      double dmin2 = c < ncq ? 0 : 2 * g.rs2 + 1;
 #pragma unroll
       for (int k = 0; k < 3; k++) {
         const double b0 = (double)u[k] * g.h[k] - 1e-9 * g.L[k], b1 = b0 + g.h[k] + 2e-9 * g.L[k];
@@ -842,23 +838,31 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4*
       const int v = __shfl_up(end, o, kWave);
       if (lane >= o) end += v;
     }
-    sm.s_end[lane] = end;
-    const int total = __builtin_amdgcn_readfirstlane(__shfl(end, nloc - 1, kWave));
-    wave_sync_lds();
-    const int stride = nparts * kWave;
-    // candidate it: its cell slot and image (binary search over the wave's
+    if (lane == kWave - 1) sh.s_wsum[wv] = end;
+    __syncthreads();
+    int total = 0;
+#pragma unroll
+    for (int w = 0; w < kQWaves; w++) {
+      const int v = sh.s_wsum[w];
+      if (w < wv) end += v;
+      total += v;
+    }
+    total = __builtin_amdgcn_readfirstlane(total);
+    sh.s_end[threadIdx.x] = end;
+    __syncthreads();
+    // candidate it: its cell slot and image (binary search over the share's
     // cell prefix in LDS)
     auto locate = [&](int it, size_t& si, int& img) {
       int lo_i = 0, hi_i = nloc - 1;
       while (lo_i < hi_i) {
         const int mid = (lo_i + hi_i) >> 1;
-        if (sm.s_end[mid] > it) hi_i = mid;
+        if (sh.s_end[mid] > it) hi_i = mid;
         else lo_i = mid + 1;
       }
-      si = (size_t)sm.s_cell[lo_i] * g.cap + (it - (lo_i ? sm.s_end[lo_i - 1] : 0));
-      img = sm.s_img[lo_i];
+      si = (size_t)sh.s_cell[lo_i] * g.cap + (it - (lo_i ? sh.s_end[lo_i - 1] : 0));
+      img = sh.s_img[lo_i];
     };
-    int it = part * kWave + lane;
+    int it = threadIdx.x;
     int j = -1, tj = 0, img = 0;
     double4 pj = make_double4(0, 0, 0, 0);
     if (it < total) {
@@ -869,9 +873,10 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4*
       tj = d.ctype[si];
     }
     // wave-uniform trip count: the lanes past `total` ride along
-    const int rounds = total > part * kWave ? (total - part * kWave + stride - 1) / stride : 0;
+    const int first = wv * kWave;
+    const int rounds = total > first ? (total - first + kBlock - 1) / kBlock : 0;
     for (int rd = 0; rd < rounds; rd++) {
-      const int it2 = it + stride;
+      const int it2 = it + kBlock;
       int j2 = -1, tj2 = 0, img2 = 0;
       double4 pj2 = make_double4(0, 0, 0, 0);
       if (it2 < total) {
@@ -881,52 +886,49 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4*
         pj2 = d.cpos[si2];
         tj2 = d.ctype[si2];
       }
-      // candidate it (its image position) against every point
-      const bool ok = it < total && j >= 0 && !(contig ? (j >= mlo && j <= mhi) : d.moved[j]);
-      double cx = 0, cy = 0, cz = 0;
-      int tflag = 0;
-      if (ok) {
-        const int iz = ((img >> 16) & 0xff) - 128;
-        const int ix = (img & 0xff) - 128, iy = ((img >> 8) & 0xff) - 128;
-        cx = pj.x + ix * g.L[0];
-        cy = pj.y + iy * g.L[1];
-        cz = pj.z + iz * g.L[2];
-        tflag = (g.use_pair && (g.npbc == 3 || iz == 0)) ? 1 << 24 : 0;
-      }
+      // candidate it (its image position) against every point; a candidate
+      // that does not count is put where every test fails
+      const bool ok = it < total && j >= 0 && !(j >= mlo && j <= mhi);
+      const int iz = ((img >> 16) & 0xff) - 128, ix = (img & 0xff) - 128, iy = ((img >> 8) & 0xff) - 128;
+      const double cx = ok ? pj.x + ix * g.L[0] : 1e30, cy = pj.y + iy * g.L[1], cz = pj.z + iz * g.L[2];
+      const double qj = g.lB * pj.w;
+      const double rcj2 = pj.w != 0 ? rc2 : -1.0;
+      const double ljj2 = (g.npbc == 3 || iz == 0) ? lj2 : -1.0;
 #pragma unroll 1
       for (int i = 0; i < np; i++) {
-        const double4 qp = sm.s_pt[i];
+        const double4 qp = sh.s_pt[i];
         const double dx = cx - qp.x, dy = cy - qp.y, dz = cz - qp.z;
         const double r2 = dx * dx + dy * dy + dz * dz;
-        const bool in = ok && r2 <= g.rs2;
-        // FP64 queue: every pair (P = 0), the close ones (P = 1)
+        // FP64 queue: every charged pair (P = 0), the close ones (P = 1)
+        const bool in = r2 <= rcj2;
         const bool near = in && (P == 0 || r2 < fp64_b2);
         const unsigned long long m = __ballot(near);
         if (m) {
-          if (near) {
-            const int k = (qhead + qn + lanes_below(m)) % kQueue;
-            sm.s_r2[k] = r2;
-            sm.s_qq[k] = qp.w * pj.w;
-            sm.s_t[k] = (sm.s_ptt[i] * nt + tj) | tflag;
-          }
+          if (near) sm.s_q[qn + lanes_below(m)] = make_double2(r2, qp.w * qj);
           qn += __popcll(m);
           if (qn >= kWave) drain(kWave);
         }
         if (P == 1) {
-          // each queue drains 64 pairs of one precision at a time, so the
-          // lanes of a drain never split between the two
+          // each queue drains pairs of one precision at a time, so the lanes
+          // of a drain never split between the two
           const bool far = in && !near;
           const unsigned long long mf = __ballot(far);
           if (mf) {
-            if (far) {
-              const int k = (fhead + fn + lanes_below(mf)) % kQueue;
-              sm.s_fr2[k] = r2;
-              sm.s_fqq[k] = (float)(qp.w * pj.w);
-              sm.s_ft[k] = (sm.s_ptt[i] * nt + tj) | tflag;
-            }
+            if (far) sm.s_f[fn + lanes_below(mf)] = make_float2((float)r2, (float)(qp.w * qj));
             fn += __popcll(mf);
             if (fn >= kWave) drain32(kWave);
           }
+        }
+        const bool lj = r2 < ljj2;
+        const unsigned long long ml = __ballot(lj);
+        if (ml) {
+          if (lj) {
+            const int k = ln + lanes_below(ml);
+            sm.s_lr[k] = r2;
+            sm.s_lt[k] = sh.s_ptt[i] * nt + tj;
+          }
+          ln += __popcll(ml);
+          if (ln >= kWave) drain_lj(kWave);
         }
       }
       it = it2;
@@ -935,10 +937,11 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4*
       img = img2;
       pj = pj2;
     }
-    wave_sync_lds();   // the next chunk rewrites the cell arrays
+    __syncthreads();   // the next chunk rewrites the cell arrays
   }
   if (qn > 0) drain(qn);
   if (P == 1 && fn > 0) drain32(fn);
+  if (ln > 0) drain_lj(ln);
 #pragma unroll
   for (int off = kWave / 2; off > 0; off >>= 1) {
     elj += __shfl_down(elj, off, kWave);
@@ -973,73 +976,104 @@ struct CSpecSmem {
   double sh[kBlock / kWave];
 };
 
+// What a block of k_compute_spec reads of the plan, one array element per
+// lane, every load issued before the first is used: a block finds its slot or
+// pair by one ballot over the prefix it holds instead of walking the prefix
+// with one dependent global read per step (up to 15 steps for a slot and 119
+// for a pair, about half a microsecond each).
+struct PlanLanes {
+  int ne, qb, nn;      // exact slots, blocks per query, near pairs (scalar)
+  int q, mm, scr;      // lane l: q_off[l], mm_off[l] (l <= ne), screen_of[l] (l < ne)
+  int off0, off1;      // pair_off[l], pair_off[l + 64]
+  int pq0, pq1;        // slots of pairs l and l + 64, p | q << 8
+};
+
+__device__ __forceinline__ PlanLanes plan_lanes(const SpecPlan* plan) {
+  const int lane = threadIdx.x % kWave, l16 = min(lane, kMaxProp), l1 = min(lane + kWave, kMaxPairs);
+  PlanLanes L;
+  const int ne = plan->n_exact, qb = plan->qblk, nn = plan->n_near;
+  L.q = plan->q_off[l16];
+  L.mm = plan->mm_off[l16];
+  L.scr = plan->screen_of[min(lane, kMaxProp - 1)];
+  L.off0 = plan->pair_off[lane];
+  L.off1 = plan->pair_off[l1];
+  const int p0 = plan->pair_p[lane], q0 = plan->pair_q[lane];
+  const int l1p = min(l1, kMaxPairs - 1);
+  const int p1 = plan->pair_p[l1p], q1 = plan->pair_q[l1p];
+  L.pq0 = p0 | (q0 << 8);
+  L.pq1 = p1 | (q1 << 8);
+  L.ne = __builtin_amdgcn_readfirstlane(ne);
+  L.qb = __builtin_amdgcn_readfirstlane(qb);
+  L.nn = __builtin_amdgcn_readfirstlane(nn);
+  return L;
+}
+
+// Slot e of prefix value `pre` (lane l: the blocks before slot l) that holds
+// block b, for b below lane ne's value.
+__device__ __forceinline__ int plan_slot(int pre, int ne, int b) {
+  const int lane = threadIdx.x % kWave;
+  return __popcll(__ballot(lane >= 1 && lane < ne && pre <= b));
+}
+
 template <int P>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_compute_spec(
     const Geo* __restrict__ G, const Dev* __restrict__ D, const RepCfg* __restrict__ RC,
     const int* __restrict__ vb_count, int R) {
   __shared__ int s_pre[kMaxReplicas];
-  __shared__ struct U {
-    QWaveSmem<P> q[kQWaves];
-  } sm;
+  __shared__ QueryShare<P> sm;
   __shared__ CSpecSmem cs;
-  for (int r = threadIdx.x; r < R; r += kBlock) s_pre[r] = vb_count[r];
-  __syncthreads();
-  lds_scan(s_pre, R);
-  const int total = s_pre[R - 1];
+  int total;
+  if (R == 1) {
+    total = uload(vb_count);
+  } else {
+    for (int r = threadIdx.x; r < R; r += kBlock) s_pre[r] = vb_count[r];
+    __syncthreads();
+    lds_scan(s_pre, R);
+    total = s_pre[R - 1];
+  }
+  const int lane = threadIdx.x % kWave;
   for (int vb = blockIdx.x; vb < total; vb += gridDim.x) {
-    const int r = __builtin_amdgcn_readfirstlane(find_replica(s_pre, R, vb));
+    const int r = R == 1 ? 0 : __builtin_amdgcn_readfirstlane(find_replica(s_pre, R, vb));
     int b = __builtin_amdgcn_readfirstlane(vb - (r ? s_pre[r - 1] : 0));
     const Geo g = load_const(G, r);
     const Dev d = load_const(D, r);
     const RepCfg rc = load_const(RC, r);
-    const SpecPlan* plan = d.plan;
-    const int ne = uload(&plan->n_exact);
-    const int ngrp = kspace_groups(ne);
+    const PlanLanes L = plan_lanes(d.plan);
+    const int ne = L.ne, ngrp = kspace_groups(ne);
     // longest work first: queries, k space, moved-moved pairs, cross terms
-    const int nqt = uload(&plan->q_off[ne]);
+    const int nqt = __builtin_amdgcn_readlane(L.q, ne), nmt = __builtin_amdgcn_readlane(L.mm, ne);
     if (b < nqt) {
-      int e = 0;
-      while (e + 1 < ne && uload(&plan->q_off[e + 1]) <= b) e++;
-      const int local = b - uload(&plan->q_off[e]);
-      const Dev v = prop_view(g, d, rc, uload(&plan->screen_of[e]), e);
-      const int nm = uload(&v.rec->n_moved);
-      const int qw = uload(&plan->qwave);
-      // wave gw: share gw % qw of query q2 = gw / qw = 2 c + on, cluster c
-      // (moved beads c kCluster ..) at their old (on = 0) or new positions
-      const int w = threadIdx.x / kWave, gw = local * kQWaves + w;
-      if (gw < 2 * query_clusters(nm) * qw) {
-        const int q2 = gw / qw, part = gw - q2 * qw;
-        const int m0 = (q2 >> 1) * kCluster, on = q2 & 1;
-        const double2 eq = real_query_cluster<P>(g, v, (on ? v.mv_new : v.mv_old) + m0, v.mv_type + m0,
-                                                 min(kCluster, nm - m0), v.rec->contig, v.rec->lo, v.rec->hi, part,
-                                                 qw, sm.q[w]);
-        const double sgn = on ? 1.0 : -1.0;
-        if (threadIdx.x % kWave == 0) v.part_r[gw] = make_double2(sgn * eq.x, sgn * eq.y);
-      }
+      const int e = plan_slot(L.q, ne, b);
+      const int local = b - __builtin_amdgcn_readlane(L.q, e);
+      const Dev v = prop_view(g, d, rc, __builtin_amdgcn_readlane(L.scr, e), e);
+      const int nm = uload(&v.rec->n_moved), lo = uload(&v.rec->lo), hi = uload(&v.rec->hi);
+      // share local % qb of query q2 = local / qb = 2 c + on, cluster c (moved
+      // beads c kCluster ..) at their old (on = 0) or new positions
+      const int q2 = local / L.qb, part = local - q2 * L.qb;
+      const int m0 = (q2 >> 1) * kCluster, on = q2 & 1;
+      const double2 eq = real_query_cluster<P>(g, v, (on ? v.mv_new : v.mv_old) + m0, v.mv_type + m0,
+                                               min(kCluster, nm - m0), lo, hi, part, L.qb, sm);
+      const double sgn = on ? 1.0 : -1.0;
+      if (lane == 0) v.part_r[local * kQWaves + threadIdx.x / kWave] = make_double2(sgn * eq.x, sgn * eq.y);
     } else if ((b -= nqt) < rc.nkb_s * ngrp) {
       // k block b / ngrp, exact slots kQWaves (b % ngrp) + wave
       const int kb = b / ngrp, e = (b - kb * ngrp) * kQWaves + threadIdx.x / kWave;
-      if (e < ne) kspace_spec_wave(g, d, rc, plan, kb, e);
+      if (e < ne) kspace_spec_wave(g, d, rc, d.plan, kb, e);
+    } else if ((b -= rc.nkb_s * ngrp) < nmt) {
+      const int e = plan_slot(L.mm, ne, b);
+      const Dev v = prop_view(g, d, rc, __builtin_amdgcn_readlane(L.scr, e), e);
+      const int nm = uload(&v.rec->n_moved);
+      mm_block(g, v, b - __builtin_amdgcn_readlane(L.mm, e), nmm_blocks(nm), cs.sh);
     } else {
-      b -= rc.nkb_s * ngrp;
-      const int nmt = uload(&plan->mm_off[ne]);
-      if (b < nmt) {
-        int e = 0;
-        while (e + 1 < ne && uload(&plan->mm_off[e + 1]) <= b) e++;
-        const Dev v = prop_view(g, d, rc, uload(&plan->screen_of[e]), e);
-        const int nm = uload(&v.rec->n_moved);
-        mm_block(g, v, b - uload(&plan->mm_off[e]), nmm_blocks(nm), cs.sh);
-      } else {
-        b -= nmt;
-        const int nn = uload(&plan->n_near);
-        int j = 0;
-        while (j + 1 < nn && uload(&plan->pair_off[j + 1]) <= b) j++;
-        const int off = uload(&plan->pair_off[j]);
-        const int sp = uload(&plan->screen_of[uload(&plan->pair_p[j])]);
-        const int sq = uload(&plan->screen_of[uload(&plan->pair_q[j])]);
-        const int np_ = uload(&d.recs[sp].n_moved), nq = uload(&d.recs[sq].n_moved);
-        cross_block(g, d, rc, sp, sq, np_, nq, b - off, cs.sh, d.part_x + b);
-      }
+      b -= nmt;
+      // pair j of the near list: pair_off is increasing, entry 0 is 0
+      const int j = __popcll(__ballot(lane >= 1 && lane < L.nn && L.off0 <= b)) +
+                    __popcll(__ballot(lane + kWave < L.nn && L.off1 <= b));
+      const int off = j < kWave ? __builtin_amdgcn_readlane(L.off0, j) : __builtin_amdgcn_readlane(L.off1, j - kWave);
+      const int pq = j < kWave ? __builtin_amdgcn_readlane(L.pq0, j) : __builtin_amdgcn_readlane(L.pq1, j - kWave);
+      const int sp = __builtin_amdgcn_readlane(L.scr, pq & 0xff), sq = __builtin_amdgcn_readlane(L.scr, pq >> 8);
+      const int np_ = uload(&d.recs[sp].n_moved), nq = uload(&d.recs[sq].n_moved);
+      cross_block(g, d, rc, sp, sq, np_, nq, b - off, cs.sh, d.part_x + b);
     }
     __syncthreads();  // the LDS is reused by the next virtual block
   }
@@ -1095,7 +1129,7 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce_spec(const Geo* __res
     if (e >= ne) return;
     const int nm = d.recs[plan->screen_of[e]].n_moved;
     if (nm == 0) return;
-    const int nreal = 2 * query_clusters(nm) * plan->qwave, nmm = nmm_blocks(nm);
+    const int nreal = query_blocks(nm, plan->qblk) * kQWaves, nmm = nmm_blocks(nm);
     const double2* pr = d.part_r + (size_t)e * rc.rstride;
     const double2* pm = d.part_mm + (size_t)e * rc.nmmb;
     double lj = 0, re = 0;

@@ -38,3 +38,23 @@ def test_pair_images_when_the_cutoff_passes_the_box(L, alpha, cells):
     eng.finalize(False)
     for k in E.TERMS:
         assert abs(d[k] - d_ref[k]) <= 1e-10 * max(abs(d_ref[k]), 1e-2), (k, d[k], d_ref[k])
+
+
+@pytest.mark.parametrize("chain_len", [3, 8, 9, 17])
+@pytest.mark.parametrize("split_div,cell_div", [(16, 4), (384, 1), (4000, 2)])
+def test_query_shares_and_partial_clusters(chain_len, split_div, cell_div):
+    """Real-space queries of one to eight blocks, clusters with one, seven and
+    eight beads, cell lists from a few to over 256 cells per share; a fifth of
+    the beads uncharged, so that pairs without an Ewald term occur too."""
+    L = 15.0
+    sd = systems.config("tiny")
+    xyz, q, ty, ms = systems.build_bulk(6, chain_len, 6 * chain_len, L, 3 + chain_len)
+    q = np.where(np.arange(len(q)) % 5 == 2, 0.0, q)
+    sd.update(xyz=xyz, q=q, type=ty, mol_start=ms, box=[L, L, L], alpha=0.25)
+    eng = E.Engine(sd, cell_div=cell_div)
+    eng.set_tuning(split_div=split_div, cell_div=cell_div)
+    eng.mc_record(200)
+    eng.mc_run(120, sd["move_prob"], move_size=1.0, seed=chain_len)
+    recs, _ = eng.mc_records(200)
+    assert len(recs) >= 100
+    replay(sd, recs, 1e-10)

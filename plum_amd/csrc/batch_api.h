@@ -187,7 +187,6 @@ int batch_upload_state(plum_batch* b) {
     D[r] = c->d;
     RepCfg& q = RCv[r];
     q.nkb_s = c->nkb_s;
-    q.nrun = c->nrun;
     q.qfill = b->n_cu * std::min(b->comp_occ, b->tune.blocks_per_cu) * kQWaves;
     q.qmax = query_split(c->cand, kQShare, b->tune.split_div);
     q.qfine = query_split(c->cand, kQFine, b->tune.split_div);

@@ -60,8 +60,7 @@ struct plum_ctx {
   double cand = 0;       // expected candidate pair-images per query
   int cell_div = 2;      // cells per search radius and dimension
   int grid_gen = 0;      // bumped by every re-grid (batches re-upload their copies)
-  int nkb_s = 0;         // k-space blocks of the speculative loop
-  int nrun = 0;          // k-vector runs of the speculative k-space (Dev::krun)
+  int nkb_s = 0;         // k-space tiles of the speculative loop
   int xcap = 0;          // cross-term partial capacity
   plum_batch* self = nullptr;  // this system as a batch of one (device loop)
   SurHost* sur = nullptr;      // delayed-acceptance surrogate (null when off)
@@ -495,18 +494,23 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
   }
   g.n_kh = (int)kl.size();
   info.n_k_half = g.n_kh;
-  // runs of up to kKRun k vectors with one (l_x, l_y) and consecutive l_z
-  // (the list has l_z fastest), one lane each in the speculative k-space
-  std::vector<int2> krun;
+  // rows of one (l_x, l_y) with their l_z from -m to m (the l_x = l_y = 0 row:
+  // 1 to m; the list has l_z fastest and the cutoff takes both signs), longest
+  // first so that the 16 rows of a tile need about the same l_z, and the tiles
+  // of the speculative k-space
+  std::vector<int4> krow;
   for (int k = 0; k < g.n_kh;) {
-    int len = 1;
-    while (len < kKRun && k + len < g.n_kh && kl[k + len].x == kl[k].x && kl[k + len].y == kl[k].y &&
-           kl[k + len].z == kl[k].z + len)
-      len++;
-    krun.push_back(make_int2(k, len));
-    k += len;
+    int e = k;
+    while (e < g.n_kh && kl[e].x == kl[k].x && kl[e].y == kl[k].y) e++;
+    krow.push_back(make_int4(kl[k].x, kl[k].y, k, kl[e - 1].z));
+    k = e;
   }
-  c->nrun = (int)krun.size();
+  std::stable_sort(krow.begin(), krow.end(), [](const int4& a, const int4& b) { return a.w > b.w; });
+  while (krow.size() % kKTile) krow.push_back(make_int4(0, 0, 0, -1));
+  std::vector<int2> ktile;
+  for (size_t r = 0; r < krow.size(); r += kKTile)
+    for (int z = 0; z <= krow[r].w; z += kKTile) ktile.push_back(make_int2((int)r, z));
+  c->nkb_s = p.use_ewald ? (int)ktile.size() : 0;
   c->nkb = std::max(1, (g.n_kh + kKPerBlock - 1) / kKPerBlock);
   c->nkb_full = std::max(1, (g.n_kh + kBlock - 1) / kBlock);
 
@@ -554,7 +558,7 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
   ALLOC(d.mv_type, (size_t)kMaxProp * maxm);
   ALLOC(d.recs, kMaxScreen); ALLOC(d.smv_idx, (size_t)kMaxProp * maxm);
   ALLOC(d.prop, kMaxScreen); ALLOC(d.plan, 1);
-  ALLOC(d.krun, std::max(1, c->nrun));
+  ALLOC(d.krow, krow.size()); ALLOC(d.ktile, ktile.size());
   // erfc nodes {erfc(x_i), (2 / sqrt(pi)) exp(-x_i^2)}, x_i = i / kErfcPerUnit,
   // each rounded once from long double (erfc_nodes)
   std::vector<double2> erfc_h(kErfcNodes);
@@ -571,8 +575,7 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
   float2* erfc32_d = nullptr;
   ALLOC(erfc32_d, kErfcNodes);
   g.erfc_tab32 = erfc32_d;
-  c->nkb_s = (g.use_ewald && g.n_kh > 0) ? (c->nrun + kKSpec - 1) / kKSpec : 0;
-  ALLOC(d.part_ks, (size_t)kKVals * std::max(1, c->nkb_s));
+  ALLOC(d.part_ks, (size_t)kMaxProp * std::max(1, c->nkb_s) * kQWaves);
   c->xcap = kMaxPairs * cross_blocks(maxm, maxm);
   ALLOC(d.part_x, c->xcap);
   ALLOC(d.ctl, 1);
@@ -608,7 +611,8 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
       (rc = up(d.type, type, sizeof(int) * n)) || (rc = up(d.mol_of, mol_of.data(), sizeof(int) * n)) ||
       (rc = up(d.mol_start, ms, sizeof(int) * (n_mols + 1))) ||
       (rc = up(d.kl, kl.data(), sizeof(int4) * kl.size())) ||
-      (rc = up(d.krun, krun.data(), sizeof(int2) * krun.size())) ||
+      (rc = up(d.krow, krow.data(), sizeof(int4) * krow.size())) ||
+      (rc = up(d.ktile, ktile.data(), sizeof(int2) * ktile.size())) ||
       (rc = up(d.ck, ck.data(), sizeof(double) * ck.size())) ||
       (rc = up(d.lj, lj.data(), sizeof(LJPair) * lj.size())) ||
       (rc = up(d.lj32, lj32.data(), sizeof(LJPair32) * lj32.size())) ||

@@ -121,7 +121,8 @@ struct Dev {
   int* ctype;
   // k space
   int4* kl;
-  int2* krun;             // runs of k vectors: (first, count), one (l_x, l_y), consecutive l_z
+  int4* krow;             // rows of the k list: (l_x, l_y, first k, largest l_z), longest first, whole tiles
+  int2* ktile;            // speculative k-space tiles: (first row, first l_z)
   double* ck;
   double2 *Sk, *dS;
   double2* tab;           // phase tables
@@ -152,7 +153,7 @@ struct Dev {
   int* smv_idx;
   PropInfo* prop;
   SpecPlan* plan;
-  double* part_ks;        // [kKVals][k blocks]
+  double* part_ks;        // [kMaxProp][k tiles][waves]
   double2* part_x;        // cross-term block partials
   // delayed acceptance (null without the surrogate): descriptor rows and
   // network outputs of every proposal (row (2 s + on) * maxm + m, on = 0 old

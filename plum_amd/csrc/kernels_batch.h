@@ -20,8 +20,8 @@
 //                    beside it, the proposals' phase tables in chunks of rows
 //                    and the fold of the previous batch's accepted dS(k) into
 //                    S(k).
-//   k_compute_spec   all systems' k-space waves (dS_e(k) of every exact slot
-//                    and its dE_k per k block), real-space query blocks
+//   k_compute_spec   all systems' k-space blocks (dS_e(k) of every exact slot
+//                    and its dE_k per k tile), real-space query blocks
 //                    (cluster queries by waves) and moved-moved blocks per
 //                    slot, and cross blocks (LJ + real pairs between two
 //                    slots' moved beads, old/new combinations), spread over
@@ -48,11 +48,11 @@ namespace plum {
 constexpr int kMaxReplicas = 1024;
 constexpr int kMaxSplit = 8;           // most blocks per real-space query
 constexpr int kDefaultSplitDiv = 384;   // candidate slots per query share
-constexpr int kKSpec = 32;             // k-vector runs per speculative k-space wave
+constexpr int kKTile = 16;             // rows and l_z of a speculative k-space tile
 
 // Per-system launch shape.
 struct RepCfg {
-  int nkb_s;    // k-space blocks of kKSpec runs (0 without Ewald)
+  int nkb_s;    // k-space tiles (0 without Ewald)
   int qmax, qfine;   // blocks of a real-space query, ordinary and on an idle chip (query_split)
   int ncell;    // cells
   int pmax;     // proposals per batch (<= kMaxProp, <= kMaxScreen with the surrogate)
@@ -64,7 +64,6 @@ struct RepCfg {
   int fill;     // exact slots given to first-stage rejections (training data)
   float r_d;    // descriptor radius of the surrogate
   int train;    // this system feeds the surrogate's training ring
-  int nrun;     // k-vector runs (Dev::krun)
   int qfill;    // waves of k_compute_spec resident on the chip at once
 };
 
@@ -74,7 +73,7 @@ struct RepCfg {
 // kQWaves waves per block.
 constexpr int kQWaves = kBlock / kWave;
 constexpr int kMaxQBlock = 8;
-constexpr int kQShare = 1000;  // candidate slots per block of a query at the default split_div
+constexpr int kQShare = 800;   // candidate slots per block of a query at the default split_div
 constexpr int kQFine = 480;    // the same where the queries leave the chip idle
 // Most blocks of a query of `cand` expected candidate slots, `share` slots
 // each at the default split_div.
@@ -88,8 +87,8 @@ __host__ __device__ __forceinline__ int query_split(double cand, int share, int 
 // launch when it is long, but each more block of a query repeats its set-up:
 // shares of about kQShare candidates (qmax blocks) are the shortest launches
 // where a batch has its 16 proposals (k_compute_spec of the 40,000-bead system
-// at 500, 1,000 and 2,000 a block: 57, 46 and 46 us; 1,000 beads: 31, 28 and
-// 33), kQFine (qfine blocks) where few proposals leave most of the chip idle
+// at 330, 650 and 1,000 a block: 45, 32 and 36 us; 1,000 beads at 1,000 and
+// 1,600: 28 and 33), kQFine (qfine blocks) where few proposals leave most of the chip idle
 // (delayed acceptance on the brush: 50 and 35 us).  More query waves than 5/8
 // of what the chip holds at once (fill; the other blocks take the rest) start
 // a second round: a query is spread no further (the brush at 16 and 32 waves a
@@ -102,9 +101,6 @@ __host__ __device__ __forceinline__ int query_spread(int qmax, int qfine, int cl
 constexpr int kCluster = 8;   // moved beads per real-space query (cluster)
 __host__ __device__ __forceinline__ int query_clusters(int nm) { return (nm + kCluster - 1) / kCluster; }
 __host__ __device__ __forceinline__ int query_blocks(int nm, int qb) { return 2 * query_clusters(nm) * qb; }
-
-// k-space blocks per k block: one wave per exact slot.
-__host__ __device__ __forceinline__ int kspace_groups(int ne) { return (ne + kQWaves - 1) / kQWaves; }
 
 // Moved-moved pair blocks: 256 pairs each, independent of the launch size.
 __host__ __device__ __forceinline__ int nmm_blocks(int nm) {
@@ -563,102 +559,102 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan_spec(const Geo* __restric
   }
   if (t == kWave - 1) {
     plan->n_near = cs;
-    // k-space blocks: one wave per exact slot and k block
-    vb_count[r] = (np > 0 && ne > 0) ? rc.nkb_s * kspace_groups(ne) + sm.s_off + bs : 0;
+    // k-space blocks: one per exact slot and k tile
+    vb_count[r] = (np > 0 && ne > 0) ? rc.nkb_s * ne + sm.s_off + bs : 0;
   }
 }
 
 // ------------------------------------------------------------ k space
-// One wave per (k block, exact slot), kQWaves slots per block, no block
-// barriers.  A k block is kKSpec runs; a run is up to kKRun k vectors of one
-// (l_x, l_y) row with consecutive l_z.  Lane (run kk, bead group grp) reads
-// the x, y and first z phase and e^{i theta_z} of each of its moved beads at
-// both positions from the tables and advances the z phase by multiplication
-// (e^{i (l+1) theta} = e^{i l theta} e^{i theta}, conjugated rows included):
-// four table reads for up to four k vectors instead of three each.  The bead
-// groups of a run meet by wave shuffles; the run's lane writes dS_e(k) and the
-// wave sums the slot's dE_e = sum_k c_k (2 Re(S* dS_e) + |dS_e|^2) over the
-// block's k vectors (S(k) with the previous batch's acceptances folded in by
-// the plan).  The cross sums 2 sum_k c_k Re(dS_p* dS_q) are formed from the
-// dS rows by k_reduce_spec.
-constexpr int kKRun = 4;
-constexpr int kKGrp = kWave / kKSpec;   // bead groups per wave
-static_assert(kKSpec * kKGrp == kWave, "a wave is the runs x bead groups of one slot");
+// One block per (k tile, exact slot).  A tile is 16 rows (l_x, l_y) of the
+// half-space list by 16 consecutive l_z >= 0, and both signs of l_z: with
+// a = q e^{i (l_x theta_x + l_y theta_y)} and z = e^{i l_z theta_z} of a moved
+// bead at its new (+) or old (-) position,
+//   dS(+-l_z) = sum (Re a Re z -+ Im a Im z) + i (Im a Re z +- Re a Im z),
+// four real products of a 16 x 2n by a 2n x 16 matrix on
+// v_mfma_f64_16x16x4f64: lane l supplies row l % 16 (column l % 16) of the
+// left (right) operand at inner index l / 16 and receives rows 4 v + l / 16 of
+// column l % 16 in its value v.  Inner index 2 m + on is row 2 m + on of the
+// slot's phase tables, so a step of four takes two beads; the block's waves
+// take the steps in turn and meet in LDS, where wave w sums value v = w.  The
+// waves then write dS_e(k) and sum the slot's dE_e = sum_k c_k (2 Re(S* dS_e)
+// + |dS_e|^2) over their k vectors (S(k) with the previous batch's acceptances
+// folded in by the plan).  The cross sums 2 sum_k c_k Re(dS_p* dS_q) are
+// formed from the dS rows by k_reduce_spec.
+// Bound by the latency of the table loads, hence four waves a tile (one wave
+// per tile: 30 us for 100 beads).  The vector form (one lane per run of four
+// k vectors, the z phase advanced by multiplication) spent 110 vector
+// instructions a bead on 32 runs, 6.6 million wave instructions per batch of
+// the 40,000-bead system, half of the launch; here a step is 4 matrix
+// instructions for 512 k vectors' terms and some 12 vector instructions, and
+// the z phase comes from the table without the multiplications' rounding.
 static_assert(kMaxProp <= 32, "exact slots are bits of one mask");
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-__device__ void kspace_spec_wave(const Geo& g, const Dev& d, const RepCfg& rc, const SpecPlan* plan, int kb, int e) {
-  const int lane = threadIdx.x % kWave;
-  const int kk = lane % kKSpec, grp = lane / kKSpec;
-  const int s = uload(&plan->screen_of[e]);
+struct KTileSmem {
+  double s_acc[kQWaves][4][4][kWave];   // [wave][value][product][lane]
+};
+static_assert(kQWaves == 4, "wave w of a k tile sums value w");
+
+__device__ void kspace_spec_block(const Geo& g, const Dev& d, const RepCfg& rc, int s, int tile, int e,
+                                  KTileSmem& sm) {
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
   const int n = uload(&d.recs[s].n_moved);
-  const int r = kb * kKSpec + kk;
-  const int2 run = r < rc.nrun ? d.krun[r] : make_int2(0, 0);
-  const int k0 = run.x, len = run.y;
-  TabIdx ti = {0, 0, 0, false, false};
-  if (len > 0) ti = tab_index(g, d.kl[k0]);
-  const int z1 = g.nkx + 1 + g.nky + 1 + 1;
-  double2 acc[kKRun];
-#pragma unroll
-  for (int i = 0; i < kKRun; i++) acc[i] = make_double2(0, 0);
-  if (len > 0) {
+  const int2 tl = load_const(d.ktile, tile);   // first row, first l_z
+  const int col = lane % kKTile, sub = lane / kKTile;
+  const int4 row = d.krow[tl.x + col];         // l_x, l_y, first k of the row, largest l_z (-1: no row)
+  const int lz = tl.y + col;
+  // the rows this lane finishes (value w): row 4 w + sub of the tile
+  const int4 mine = d.krow[tl.x + 4 * w + sub];
+  f64x4 rr = {0, 0, 0, 0}, ii = rr, ri = rr, ir = rr;
+  if (n > 0) {
     const double4* mo = d.mv_old + s * rc.maxm;
-    const double2* base = d.tab + (size_t)s * rc.maxm * 2 * g.tab_w;
-    for (int m = grp; m < n; m += kKGrp) {
-      const double qm = mo[m].w;
-      const double2* to = base + (size_t)(2 * m) * g.tab_w;
-      const double2* tn = to + g.tab_w;
-      // the eight table reads of both positions first, then new minus old
-      double2 ox_n = tn[ti.ox], oy_n = tn[ti.oy], oz_n = tn[ti.oz], b_n = tn[z1];
-      double2 ox_o = to[ti.ox], oy_o = to[ti.oy], oz_o = to[ti.oz], b_o = to[z1];
-      {
-        if (ti.ny) oy_n.y = -oy_n.y;
-        if (ti.nz) oz_n.y = -oz_n.y;
-        const double2 xy = cmul(ox_n, oy_n);
-        double2 z = oz_n;
-#pragma unroll
-        for (int i = 0; i < kKRun; i++) {
-          if (i) z = cmul(z, b_n);
-          const double2 ph = cmul(xy, z);
-          acc[i].x += qm * ph.x;
-          acc[i].y += qm * ph.y;
-        }
-      }
-      {
-        if (ti.ny) oy_o.y = -oy_o.y;
-        if (ti.nz) oz_o.y = -oz_o.y;
-        const double2 xy = cmul(ox_o, oy_o);
-        double2 z = oz_o;
-#pragma unroll
-        for (int i = 0; i < kKRun; i++) {
-          if (i) z = cmul(z, b_o);
-          const double2 ph = cmul(xy, z);
-          acc[i].x -= qm * ph.x;
-          acc[i].y -= qm * ph.y;
-        }
-      }
+    const double2* tab = d.tab + (size_t)s * rc.maxm * 2 * g.tab_w;
+    const int ox = row.x, oy = g.nkx + 1 + abs(row.y), oz = g.nkx + 1 + g.nky + 1 + min(lz, g.nkz);
+    const double sy = row.y < 0 ? -1.0 : 1.0, sq = (sub & 1) ? 1.0 : -1.0;
+    const int last = 2 * n - 1;
+#pragma unroll 2
+    for (int i0 = 4 * w; i0 <= last; i0 += 4 * kQWaves) {
+      const int i = min(i0 + sub, last);   // past the end: the last row again, with no charge
+      const double2* t = tab + (size_t)i * g.tab_w;
+      const double2 X = t[ox], Y = t[oy], Z = t[oz];
+      const double q = i0 + sub <= last ? sq * mo[i >> 1].w : 0.0;
+      const double yr = q * Y.x, yi = q * sy * Y.y;
+      const double ar = X.x * yr - X.y * yi, ai = X.x * yi + X.y * yr;
+      rr = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, Z.x, rr, 0, 0, 0);
+      ii = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, Z.y, ii, 0, 0, 0);
+      ri = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, Z.y, ri, 0, 0, 0);
+      ir = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, Z.x, ir, 0, 0, 0);
     }
   }
-  // the bead groups of run kk sit in lanes kk, kk + kKSpec, ...; a butterfly
-  // leaves their sum in each of them
 #pragma unroll
-  for (int o = kKSpec; o < kWave; o <<= 1)
+  for (int v = 0; v < 4; v++) {
+    sm.s_acc[w][v][0][lane] = rr[v];
+    sm.s_acc[w][v][1][lane] = ii[v];
+    sm.s_acc[w][v][2][lane] = ri[v];
+    sm.s_acc[w][v][3][lane] = ir[v];
+  }
+  __syncthreads();
+  double t4[4] = {0, 0, 0, 0};
 #pragma unroll
-    for (int i = 0; i < kKRun; i++) {
-      acc[i].x += __shfl_xor(acc[i].x, o, kWave);
-      acc[i].y += __shfl_xor(acc[i].y, o, kWave);
-    }
+  for (int u = 0; u < kQWaves; u++)
+#pragma unroll
+    for (int p = 0; p < 4; p++) t4[p] += sm.s_acc[u][w][p][lane];
   double part = 0;
-  if (grp == 0) {
-#pragma unroll
-    for (int i = 0; i < kKRun; i++)
-      if (i < len) {
-        const double2 v = acc[i], S = d.Sk[k0 + i];
-        d.dS[(size_t)e * g.n_kh + k0 + i] = v;
-        part += d.ck[k0 + i] * (2.0 * (S.x * v.x + S.y * v.y) + v.x * v.x + v.y * v.y);
-      }
+  double2* dS = d.dS + (size_t)e * g.n_kh;
+  auto put = [&](int k, double x, double y) {
+    const double2 S = d.Sk[k];
+    dS[k] = make_double2(x, y);
+    part += d.ck[k] * (2.0 * (S.x * x + S.y * y) + x * x + y * y);
+  };
+  if (lz <= mine.w) {
+    // the l_x = l_y = 0 row holds l_z > 0 only
+    const bool xy = (mine.x | mine.y) != 0;
+    const int k0 = xy ? mine.z + mine.w : mine.z - 1;
+    if (xy || lz > 0) put(k0 + lz, t4[0] - t4[1], t4[2] + t4[3]);
+    if (xy && lz > 0) put(k0 - lz, t4[0] + t4[1], t4[3] - t4[2]);
   }
   part = wave_sum(part);
-  if (lane == 0) d.part_ks[(size_t)e * rc.nkb_s + kb] = part;
+  if (lane == 0) d.part_ks[((size_t)e * rc.nkb_s + tile) * kQWaves + w] = part;
 }
 
 // ------------------------------------------------------------ real space
@@ -1020,7 +1016,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     const Geo* __restrict__ G, const Dev* __restrict__ D, const RepCfg* __restrict__ RC,
     const int* __restrict__ vb_count, int R) {
   __shared__ int s_pre[kMaxReplicas];
-  __shared__ QueryShare<P> sm;
+  __shared__ union {
+    QueryShare<P> q;
+    KTileSmem k;
+  } sm;
   __shared__ CSpecSmem cs;
   int total;
   if (R == 1) {
@@ -1039,7 +1038,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     const Dev d = load_const(D, r);
     const RepCfg rc = load_const(RC, r);
     const PlanLanes L = plan_lanes(d.plan);
-    const int ne = L.ne, ngrp = kspace_groups(ne);
+    const int ne = L.ne;
     // longest work first: queries, k space, moved-moved pairs, cross terms
     const int nqt = __builtin_amdgcn_readlane(L.q, ne), nmt = __builtin_amdgcn_readlane(L.mm, ne);
     if (b < nqt) {
@@ -1052,14 +1051,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
       const int q2 = local / L.qb, part = local - q2 * L.qb;
       const int m0 = (q2 >> 1) * kCluster, on = q2 & 1;
       const double2 eq = real_query_cluster<P>(g, v, (on ? v.mv_new : v.mv_old) + m0, v.mv_type + m0,
-                                               min(kCluster, nm - m0), lo, hi, part, L.qb, sm);
+                                               min(kCluster, nm - m0), lo, hi, part, L.qb, sm.q);
       const double sgn = on ? 1.0 : -1.0;
       if (lane == 0) v.part_r[local * kQWaves + threadIdx.x / kWave] = make_double2(sgn * eq.x, sgn * eq.y);
-    } else if ((b -= nqt) < rc.nkb_s * ngrp) {
-      // k block b / ngrp, exact slots kQWaves (b % ngrp) + wave
-      const int kb = b / ngrp, e = (b - kb * ngrp) * kQWaves + threadIdx.x / kWave;
-      if (e < ne) kspace_spec_wave(g, d, rc, d.plan, kb, e);
-    } else if ((b -= rc.nkb_s * ngrp) < nmt) {
+    } else if ((b -= nqt) < rc.nkb_s * ne) {
+      // k tile b / ne, exact slot b % ne
+      const int kt = b / ne, e = b - kt * ne;
+      kspace_spec_block(g, d, rc, __builtin_amdgcn_readlane(L.scr, e), kt, e, sm.k);
+    } else if ((b -= rc.nkb_s * ne) < nmt) {
       const int e = plan_slot(L.mm, ne, b);
       const Dev v = prop_view(g, d, rc, __builtin_amdgcn_readlane(L.scr, e), e);
       const int nm = uload(&v.rec->n_moved);
@@ -1082,7 +1081,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 constexpr int kReduceThreads = 1024;
 
 // Sums of a batch, one block per (sum, system), fixed order: blockIdx.x in
-// [0, kMaxProp) the k-space dE per exact slot (the k blocks' partials), then
+// [0, kMaxProp) the k-space dE per exact slot (the k tiles' partials), then
 // kMaxPairs k-space cross sums 2 sum_k c_k Re(dS_p* dS_q) of the slot pairs
 // p < q (pair_index order) from the dS rows, then kMaxProp (LJ, real) sums per
 // exact slot (real-space query blocks + moved-moved blocks), then kMaxPairs
@@ -1102,7 +1101,8 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce_spec(const Geo* __res
   if (j < kMaxProp) {
     if (j >= ne) return;
     double s = 0;
-    for (int i = t; i < rc.nkb_s; i += kReduceThreads) s += d.part_ks[(size_t)j * rc.nkb_s + i];
+    const int np = rc.nkb_s * kQWaves;
+    for (int i = t; i < np; i += kReduceThreads) s += d.part_ks[(size_t)j * np + i];
     s = block_sum<kReduceThreads>(s, sh);
     if (t == 0) plan->ksum[j] = s;
   } else if (j < kKVals) {

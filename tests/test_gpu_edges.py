@@ -58,3 +58,21 @@ def test_query_shares_and_partial_clusters(chain_len, split_div, cell_div):
     recs, _ = eng.mc_records(200)
     assert len(recs) >= 100
     replay(sd, recs, 1e-10)
+
+
+@pytest.mark.parametrize("box,alpha,chain_len", [
+    ([14.0, 14.0, 14.0], 0.02, 2),     # a handful of rows: one tile, mostly padding
+    ([14.0, 14.0, 14.0], 0.9, 5),      # |l_z| on both sides of a tile edge
+    ([9.0, 21.0, 14.0], 1.3, 3),       # unequal extents, two l_z groups in some rows only
+    ([20.0, 8.0, 9.0], 0.5, 33),       # moved counts past a multiple of the four-step
+])
+def test_kspace_tiles(box, alpha, chain_len):
+    """dS(k) of the speculative loop by tiles of 16 rows and 16 l_z."""
+    sd = systems.config("tiny")
+    xyz, q, ty, ms = systems.build_bulk(3, chain_len, 3 * chain_len, None, 21, box=box)
+    sd.update(xyz=xyz, q=q, type=ty, mol_start=ms, box=box, alpha=alpha)
+    eng, _, recs, _ = record_run(sd, 80, 16, seed=8)
+    print("k extents", list(eng.info().repl_cell), "vectors", eng.info().n_k_half)
+    replay(sd, recs, 1e-10)
+    run, full = eng.totals(), eng.energy_full()
+    assert abs(run["kspace"] - full["kspace"]) <= 1e-10 * max(1.0, abs(full["kspace"]))

@@ -24,7 +24,6 @@ struct plum_batch {
   int2* d_status = nullptr;
   int2* h_status = nullptr;   // pinned
   int total_cells = 0;
-  int max_nkb_full = 1;
   int n_cu = 0;
   int descr_occ = 1;    // resident k_descr_spec blocks per CU
   int comp_occ = 1;     // resident k_compute_spec blocks per CU
@@ -177,7 +176,6 @@ int batch_upload_state(plum_batch* b) {
   std::vector<Geo> G(b->R);
   std::vector<Dev> D(b->R);
   std::vector<RepCfg> RCv(b->R);
-  b->max_nkb_full = 1;
   b->da = b->reps[0]->sur && b->reps[0]->sur->on;
   if (b->da) CHK(batch_setup_da(b));
   for (int r = 0; r < b->R; r++) {
@@ -204,7 +202,6 @@ int batch_upload_state(plum_batch* b) {
       D[r].sur_x = b->sx + (size_t)r * b->sx_rows * kDescr;
       D[r].sur_f = b->sf + (size_t)r * b->sx_rows;
     }
-    b->max_nkb_full = std::max(b->max_nkb_full, c->nkb_full);
   }
   HIPCHK(hipMemcpyAsync(b->dG, G.data(), sizeof(Geo) * b->R, hipMemcpyHostToDevice, b->st));
   HIPCHK(hipMemcpyAsync(b->dD, D.data(), sizeof(Dev) * b->R, hipMemcpyHostToDevice, b->st));
@@ -270,9 +267,12 @@ void launch_batch(plum_batch* b, hipEvent_t* ev = nullptr) {
   if (ev) (void)hipEventRecord(ev[7], b->st);
 }
 
-void launch_tail(plum_batch* b) {
-  hipLaunchKernelGGL(k_compact_batch, dim3((b->total_cells + kBlock - 1) / kBlock), dim3(kBlock), 0, b->st, b->dG,
+void launch_compact(plum_batch* b) {
+  hipLaunchKernelGGL(k_compact_batch, dim3((b->total_cells + kQWaves - 1) / kQWaves), dim3(kBlock), 0, b->st, b->dG,
                      b->dD, b->d_cell_off, b->R);
+}
+
+void launch_status(plum_batch* b) {
   hipLaunchKernelGGL(k_batch_status, dim3((b->R + kBlock - 1) / kBlock), dim3(kBlock), 0, b->st, b->dD, b->dMC, b->R,
                      b->d_status);
 }
@@ -301,9 +301,10 @@ bool graph_stale(const plum_batch* b, int nb) {
          b->g_sf != (b->da ? (const void*)b->sf : nullptr);
 }
 
-// `nb` batches of every system, then compaction and the status gather.  With
-// profiling, direct launches bracketed by events (per-kernel device times).
-int batch_replay(plum_batch* b, int nb, bool use_graph, plum_ctx* prof) {
+// `nb` batches of every system, then (compact) the cell compaction and the
+// status gather.  With profiling, direct launches bracketed by events
+// (per-kernel device times).
+int batch_replay(plum_batch* b, int nb, bool compact, bool use_graph, plum_ctx* prof) {
   if (prof) {
     std::vector<hipEvent_t> ev(kSpecKernels + 1);
     for (auto& e : ev) HIPCHK(hipEventCreate(&e));
@@ -319,8 +320,7 @@ int batch_replay(plum_batch* b, int nb, bool use_graph, plum_ctx* prof) {
         }
       }
       // stop once every system has made its moves (no idle batches timed)
-      hipLaunchKernelGGL(k_batch_status, dim3((b->R + kBlock - 1) / kBlock), dim3(kBlock), 0, b->st, b->dD, b->dMC,
-                         b->R, b->d_status);
+      launch_status(b);
       HIPCHK(hipMemcpyAsync(b->h_status, b->d_status, sizeof(int2) * b->R, hipMemcpyDeviceToHost, b->st));
       HIPCHK(hipStreamSynchronize(b->st));
       bool busy = false;
@@ -328,13 +328,15 @@ int batch_replay(plum_batch* b, int nb, bool use_graph, plum_ctx* prof) {
       if (!busy) break;
     }
     for (auto& e : ev) (void)hipEventDestroy(e);
-    launch_tail(b);
+    if (compact) launch_compact(b);
+    launch_status(b);
     HIPCHK(hipGetLastError());
     return PLUM_OK;
   }
   if (!use_graph) {
     for (int i = 0; i < nb; i++) launch_batch(b);
-    launch_tail(b);
+    if (compact) launch_compact(b);
+    launch_status(b);
     HIPCHK(hipGetLastError());
     return PLUM_OK;
   }
@@ -342,7 +344,8 @@ int batch_replay(plum_batch* b, int nb, bool use_graph, plum_ctx* prof) {
     batch_drop_graph(b);
     HIPCHK(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
     for (int i = 0; i < nb; i++) launch_batch(b);
-    launch_tail(b);
+    launch_compact(b);
+    launch_status(b);
     hipGraph_t gr = nullptr;
     HIPCHK(hipStreamEndCapture(b->st, &gr));
     b->graph = gr;
@@ -360,9 +363,7 @@ int batch_replay(plum_batch* b, int nb, bool use_graph, plum_ctx* prof) {
 
 // Pending S(k) of every system folded in (end of a run, before a rebuild).
 int batch_flush(plum_batch* b) {
-  hipLaunchKernelGGL(k_flush_spec, dim3(std::min(b->max_nkb_full, 64), b->R), dim3(kBlock), 0, b->st, b->dG, b->dD,
-                     b->R);
-  hipLaunchKernelGGL(k_clear_mask, dim3((b->R + kBlock - 1) / kBlock), dim3(kBlock), 0, b->st, b->dD, b->R);
+  hipLaunchKernelGGL(k_flush_spec, dim3(b->R), dim3(kFlushThreads), 0, b->st, b->dG, b->dD);
   HIPCHK(hipGetLastError());
   return PLUM_OK;
 }
@@ -496,8 +497,30 @@ int batch_run(plum_batch* b, const plum_mc_params* mcp, long long n_moves, bool 
   std::vector<long long> credited(R, 0);   // skipped moves already given back
   const auto t0 = std::chrono::steady_clock::now();
   long long since_resync = 0, rebuilds = 0;
+  // Batches per replay: a whole graph (batches_per_graph batches, compaction,
+  // status) while the moves left fill it, else as many batches as they need,
+  // launched one by one (a launch costs the host some 3 us, less than the
+  // kernels take) instead of idle batches, some 12 us each: a run of 10 moves
+  // spent 31 idle batches of 32.  The cell compaction keeps its period of
+  // batches_per_graph batches whatever the replays, so the slots a batch sees
+  // depend on its number alone.  With online training a replay is a training
+  // period and stays whole.
+  const int period = b->tune.batches_per_graph;
+  const bool whole = prof || (b->da && b->reps[0]->sur->p.train_every > 0);
+  long long left = n_moves, did = 0, batches = 0;
+  int phase = 0;   // batches since the last compaction
   for (;;) {
-    CHK(batch_replay(b, b->tune.batches_per_graph, use_graph, prof));
+    int nb = period;
+    if (!whole) {
+      // 1.1 batches per pmax moves at first (an accepted proposal may end a
+      // batch early), then the rate seen so far
+      const double rate = did > 0 ? (double)did / (double)batches : b->tune.pmax / 1.1;
+      nb = (int)std::min<double>(period - phase, std::max(1.0, std::ceil((double)left / std::max(rate, 0.25))));
+    }
+    const bool compact = phase + nb == period;
+    CHK(batch_replay(b, nb, compact, use_graph && nb == period, prof));
+    phase = compact ? 0 : phase + nb;
+    batches += nb;
     HIPCHK(hipMemcpyAsync(b->h_status, b->d_status, sizeof(int2) * R, hipMemcpyDeviceToHost, b->st));
     if (b->da) HIPCHK(hipMemcpyAsync(b->reps[0]->sur->h_ctl, b->reps[0]->sur->tr_ctl, 2 * sizeof(int),
                                      hipMemcpyDeviceToHost, b->st));
@@ -508,13 +531,17 @@ int batch_run(plum_batch* b, const plum_mc_params* mcp, long long n_moves, bool 
       if (su->p.train_every > 0 && su->h_ctl[0] >= su->p.train_samples)
         CHK(sur_train_step(b->reps[0], b->st, su->p.train_samples, true, true, false));
     }
-    since_resync += (long long)b->tune.batches_per_graph * b->tune.pmax;
+    since_resync += (long long)nb * b->tune.pmax;
     bool busy = false, fix = false;
+    long long most = 0;
     for (int r = 0; r < R; r++) {
       busy |= b->h_status[r].y > 0;
       fix |= b->h_status[r].x != 0;
+      most = std::max<long long>(most, b->h_status[r].y);
     }
-    const bool resync = resync_every > 0 && since_resync >= resync_every && busy;
+    did = n_moves - most;   // moves of the slowest system
+    left = most;
+    const bool resync = resync_every > 0 && since_resync >= resync_every && busy && phase == 0;
     if (fix || resync) {
       CHK(batch_flush(b));
       HIPCHK(hipStreamSynchronize(b->st));
@@ -544,8 +571,7 @@ int batch_run(plum_batch* b, const plum_mc_params* mcp, long long n_moves, bool 
     if (!busy) break;
   }
   CHK(batch_flush(b));
-  hipLaunchKernelGGL(k_compact_batch, dim3((b->total_cells + kBlock - 1) / kBlock), dim3(kBlock), 0, b->st, b->dG,
-                     b->dD, b->d_cell_off, b->R);
+  if (phase > 0) launch_compact(b);
   HIPCHK(hipGetLastError());
   for (int r = 0; r < R; r++) CHK(read_ctl(b->reps[r], b->st));
   HIPCHK(hipStreamSynchronize(b->st));

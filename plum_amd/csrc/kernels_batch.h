@@ -130,11 +130,6 @@ __device__ __forceinline__ double uniform_double(double v) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// Set bits of m below this lane.
-__device__ __forceinline__ int lanes_below(unsigned long long m) {
-  return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-}
-
 // System r owning virtual block v: first r with pre[r] > v (inclusive prefix).
 __device__ __forceinline__ int find_replica(const int* pre, int R, int v) {
   int lo = 0, hi = R - 1;
@@ -1544,16 +1539,16 @@ __global__ __launch_bounds__(kBlock) void k_resolve_spec(const Geo* __restrict__
   }
 }
 
-// Folds the pending accepted dS_e(k) into S(k) (end of a run); one block row
-// per system, grid-stride over its k vectors.
-__global__ void k_flush_spec(const Geo* __restrict__ G, const Dev* __restrict__ D, int R) {
-  const int r = blockIdx.y;
-  if (r >= R) return;
+// Folds the pending accepted dS_e(k) into S(k) (end of a run) and clears the
+// mask, one block per system.
+constexpr int kFlushThreads = 1024;
+__global__ __launch_bounds__(kFlushThreads) void k_flush_spec(const Geo* __restrict__ G, const Dev* __restrict__ D) {
+  const int r = blockIdx.x;
   const Geo& g = G[r];
   const Dev& d = D[r];
   const unsigned mask = d.plan->acc_mask;
   if (!mask) return;
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < g.n_kh; k += gridDim.x * blockDim.x) {
+  for (int k = threadIdx.x; k < g.n_kh; k += kFlushThreads) {
     double2 s = d.Sk[k];
     for (int e = 0; e < kMaxProp; e++)
       if (mask & (1u << e)) {
@@ -1563,18 +1558,18 @@ __global__ void k_flush_spec(const Geo* __restrict__ G, const Dev* __restrict__ 
       }
     d.Sk[k] = s;
   }
+  __syncthreads();
+  if (threadIdx.x == 0) d.plan->acc_mask = 0;
 }
 
-__global__ void k_clear_mask(const Dev* __restrict__ D, int R) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < R) D[r].plan->acc_mask = 0;
-}
-
-// Tombstone compaction of every system's cells; cell_off is the exclusive
-// prefix of the cell counts (R + 1 entries).
-__global__ void k_compact_batch(const Geo* __restrict__ G, const Dev* __restrict__ D,
-                                const int* __restrict__ cell_off, int R) {
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+// Tombstone compaction of every system's cells, one wave per cell; cell_off
+// is the exclusive prefix of the cell counts (R + 1 entries).  A cell is a
+// chain of dependent reads (count, slots, their contents): by one thread, slot
+// after slot, 50 to 130 us a launch whatever the number of cells (longest
+// where few cells hold many beads); by a wave, 64 slots at a time.
+__global__ __launch_bounds__(kBlock) void k_compact_batch(const Geo* __restrict__ G, const Dev* __restrict__ D,
+                                                          const int* __restrict__ cell_off, int R) {
+  const int gid = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
   if (gid >= cell_off[R]) return;
   int lo = 0, hi = R - 1;
   while (lo < hi) {
@@ -1582,7 +1577,7 @@ __global__ void k_compact_batch(const Geo* __restrict__ G, const Dev* __restrict
     if (cell_off[mid] <= gid) lo = mid;
     else hi = mid - 1;
   }
-  compact_cell(G[lo], D[lo], gid - cell_off[lo]);
+  compact_cell_wave(G[lo], D[lo], gid - cell_off[lo]);
 }
 
 // Per system: overflow flag and moves still to propose (read by the host

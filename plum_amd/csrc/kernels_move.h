@@ -464,6 +464,40 @@ __device__ void compact_cell(const Geo& g, const Dev& d, int cell) {
   d.ccount[cell] = w;
 }
 
+// Set bits of m below this lane.
+__device__ __forceinline__ int lanes_below(unsigned long long m) {
+  return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+}
+
+// The same by one wave, 64 slots at a time.  The live slots of a chunk move to
+// places at or before their own, all of its reads before its writes.
+__device__ void compact_cell_wave(const Geo& g, const Dev& d, int cell) {
+  const int lane = threadIdx.x % kWave;
+  const int cnt = d.ccount[cell];
+  const size_t c0 = (size_t)cell * g.cap;
+  int w = 0;
+  for (int base = 0; base < cnt; base += kWave) {
+    const int s = base + lane;
+    const int j = s < cnt ? d.cbead[c0 + s] : -1;
+    const unsigned long long live = __ballot(j >= 0);
+    const int to = w + lanes_below(live);
+    if (j >= 0 && to != s) {
+      const double4 p = d.cpos[c0 + s];
+      const float4 p32 = d.cpos32[c0 + s];
+      const int t = d.ctype[c0 + s];
+      d.cbead[c0 + to] = j;
+      d.cpos[c0 + to] = p;
+      d.cpos32[c0 + to] = p32;
+      d.ctype[c0 + to] = t;
+      d.bslot[j] = to;
+    }
+    w += __popcll(live);
+  }
+  if (w == cnt) return;
+  for (int s = w + lane; s < cnt; s += kWave) d.cbead[c0 + s] = -1;
+  if (lane == 0) d.ccount[cell] = w;
+}
+
 // The moved beads of one commit: item k's trial position and bead index.
 struct MoveItems {
   const double4* mv_new;
@@ -746,13 +780,6 @@ __global__ __launch_bounds__(kBlock) void k_epilogue(Geo g, Dev d, int nkb, int 
 __global__ __launch_bounds__(kBlock) void k_commit(Geo g, Dev d, int accept) {
   __shared__ CommitSmem cs;
   commit_block(g, d, accept && d.rec->valid, cs);
-}
-
-// Removes tombstones cell by cell, keeping slot order.
-__global__ void k_compact(Geo g, Dev d) {
-  const int cell = blockIdx.x * blockDim.x + threadIdx.x;
-  if (cell >= g.ncell) return;
-  compact_cell(g, d, cell);
 }
 
 // ------------------------------------------------------------ proposals

@@ -55,7 +55,8 @@ struct plum_ctx {
   int nmmb = 1;          // blocks of the moved-moved pair work
   int nchunk = 1;        // bead chunks of the S(k) build
   int chunk = 512;
-  int nrealb = 1;        // blocks of the full real-space kernel
+  int full_groups = 1, full_parts = 1;   // slot groups and cell shares of the full real-space kernel
+  size_t fpart_cap = 0;  // its partials allocated
   int nsplit = 1;        // blocks per real-space query
   double cand = 0;       // expected candidate pair-images per query
   int cell_div = 2;      // cells per search radius and dimension
@@ -67,10 +68,9 @@ struct plum_ctx {
   CbmcHost* cbmc = nullptr;    // configurational-bias trial buffers
   VpHost* vp = nullptr;        // volume-perturbation pressure buffers
   int screen_cap = kMaxProp;   // proposal slots allocated
-  double* epart_k = nullptr;
+  double *epart_k = nullptr, *opart = nullptr;   // from-scratch k-space / springs, walls, self, dipole partials
+  int *d_max = nullptr, *h_max = nullptr;        // largest cell count (device, pinned host)
   std::vector<int> mol_start;
-  std::vector<int> type_h;
-  std::vector<double> q_h;
   char* h_in = nullptr;  // pinned staging of the move record
   Ctl* h_ctl = nullptr;  // pinned copy of the control block
   size_t in_bytes = 0, off_xyz = 0;
@@ -146,44 +146,21 @@ void derive_cutoffs(const plum_params& p, plum_info& info) {
   for (int i = 0; i < 3; i++) info.repl_cell[i] = (int)ceil(sqrt(repl_cutoff) * box[i] / (2 * kPi));
 }
 
-// Same expressions as wrap_coord / cell_coord on the device.
-double host_wrap(double x, double L, double invL) {
-  double w = x - L * floor(x * invL);
-  if (w >= L) w -= L;
-  if (w < 0) w += L;
-  return w;
-}
-
-int host_cell(double xw, double inv_h, int n) {
-  int c = (int)floor(xw * inv_h);
-  return c < 0 ? 0 : (c >= n ? n - 1 : c);
-}
-
-// Builds the cell list from the current device positions (host counting
-// sort in bead order: deterministic slot order) and uploads it.
+// Builds the cell list from the current device positions, each cell's beads in
+// index order (k_cell_*).  The largest count comes back to the host, which
+// sizes the slots.
 int build_cells(plum_ctx* c, int min_cap) {
   const Geo& g = c->g;
-  const int n = g.n;
-  std::vector<double> x(n), y(n), z(n);
-  HIPCHK(hipMemcpyAsync(x.data(), c->d.x, sizeof(double) * n, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipMemcpyAsync(y.data(), c->d.y, sizeof(double) * n, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipMemcpyAsync(z.data(), c->d.z, sizeof(double) * n, hipMemcpyDeviceToHost, c->st));
+  const int nb = (g.n + kBlock - 1) / kBlock;
+  HIPCHK(hipMemsetAsync(c->d.ccount, 0, sizeof(int) * g.ncell, c->st));
+  HIPCHK(hipMemsetAsync(c->d_max, 0, sizeof(int), c->st));
+  hipLaunchKernelGGL(k_cell_count, dim3(nb), dim3(kBlock), 0, c->st, g, c->d);
+  hipLaunchKernelGGL(k_cell_max, dim3(std::min(64, (g.ncell + kBlock - 1) / kBlock)), dim3(kBlock), 0, c->st, g,
+                     c->d, c->d_max);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipMemcpyAsync(c->h_max, c->d_max, sizeof(int), hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
-  std::vector<int> cell(n), count(g.ncell, 0);
-  std::vector<double> w(3 * (size_t)n);
-  std::vector<int> cc3(3 * (size_t)n);
-  for (int i = 0; i < n; i++) {
-    const double p[3] = {x[i], y[i], z[i]};
-    int cc = 0;
-    for (int k = 0; k < 3; k++) {
-      w[3 * (size_t)i + k] = host_wrap(p[k], g.L[k], g.inv_L[k]);
-      cc3[3 * (size_t)i + k] = host_cell(w[3 * (size_t)i + k], g.inv_h[k], g.nc[k]);
-      cc = cc * g.nc[k] + cc3[3 * (size_t)i + k];
-    }
-    cell[i] = cc;
-    count[cc]++;
-  }
-  const int maxc = *std::max_element(count.begin(), count.end());
+  const int maxc = *c->h_max;
   const int cap = std::max(std::max(16, min_cap), ((maxc * 2 + 8 + 7) / 8) * 8);
   const size_t slots = (size_t)g.ncell * cap;
   if (cap != c->g.cap || c->d.cbead == nullptr) {
@@ -192,33 +169,23 @@ int build_cells(plum_ctx* c, int min_cap) {
     CHK(dalloc(c, &c->d.cpos32, slots));
     CHK(dalloc(c, &c->d.ctype, slots));
     c->g.cap = cap;
-    c->nrealb = (int)((slots + kBlock - 1) / kBlock);
-    CHK(dalloc(c, &c->d.fpart, 2 * (size_t)c->nrealb));
   }
-  std::vector<int> cbead(slots, -1), ctype(slots, 0), bslot(n);
-  std::vector<double4> cpos(slots, make_double4(0, 0, 0, 0));
-  std::vector<float4> cpos32(slots, make_float4(0, 0, 0, 0));
-  std::fill(count.begin(), count.end(), 0);
-  for (int i = 0; i < n; i++) {
-    const int cc = cell[i];
-    const int s = count[cc]++;
-    const size_t si = (size_t)cc * cap + s;
-    const double* wi = &w[3 * (size_t)i];
-    const int* ci = &cc3[3 * (size_t)i];
-    cbead[si] = i;
-    ctype[si] = c->type_h[i];
-    cpos[si] = make_double4(wi[0], wi[1], wi[2], c->q_h[i]);
-    cpos32[si] = make_float4((float)(wi[0] - ci[0] * g.h[0]), (float)(wi[1] - ci[1] * g.h[1]),
-                             (float)(wi[2] - ci[2] * g.h[2]), (float)c->q_h[i]);
-    bslot[i] = s;
+  // from-scratch real space: block (cell, group of kCluster slots, share of
+  // the query's cells).  Groups for the counts the list holds now (a fuller
+  // cell's blocks take several), shares where few cells hold many beads
+  c->full_groups = std::max(1, std::min((maxc + kCluster - 1) / kCluster, 65535));
+  const long long blocks = (long long)g.ncell * c->full_groups;
+  c->full_parts = (int)std::max(1LL, std::min<long long>(kMaxQBlock, std::min<long long>(
+                      1024 / blocks, (long long)(c->cand / kQShare))));
+  const size_t fp = (size_t)blocks * c->full_parts * kQWaves;
+  if (fp > c->fpart_cap) {
+    CHK(dalloc(c, &c->d.fpart, fp));
+    c->fpart_cap = fp;
   }
-  HIPCHK(hipMemcpyAsync(c->d.ccount, count.data(), sizeof(int) * g.ncell, hipMemcpyHostToDevice, c->st));
-  HIPCHK(hipMemcpyAsync(c->d.cbead, cbead.data(), sizeof(int) * slots, hipMemcpyHostToDevice, c->st));
-  HIPCHK(hipMemcpyAsync(c->d.ctype, ctype.data(), sizeof(int) * slots, hipMemcpyHostToDevice, c->st));
-  HIPCHK(hipMemcpyAsync(c->d.cpos, cpos.data(), sizeof(double4) * slots, hipMemcpyHostToDevice, c->st));
-  HIPCHK(hipMemcpyAsync(c->d.cpos32, cpos32.data(), sizeof(float4) * slots, hipMemcpyHostToDevice, c->st));
-  HIPCHK(hipMemcpyAsync(c->d.bcell, cell.data(), sizeof(int) * n, hipMemcpyHostToDevice, c->st));
-  HIPCHK(hipMemcpyAsync(c->d.bslot, bslot.data(), sizeof(int) * n, hipMemcpyHostToDevice, c->st));
+  HIPCHK(hipMemsetAsync(c->d.ccount, 0, sizeof(int) * g.ncell, c->st));
+  hipLaunchKernelGGL(k_cell_fill, dim3(nb), dim3(kBlock), 0, c->st, g, c->d);
+  hipLaunchKernelGGL(k_cell_order, dim3(g.ncell), dim3(kBlock), 0, c->st, g, c->d);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(c->st));
   c->info.cell_cap = cap;
   return PLUM_OK;
@@ -267,25 +234,35 @@ int regrid_cells(plum_ctx* c, int div) {
   set_cell_grid(c, div);
   if (c->g.ncell != old_ncell) CHK(dalloc(c, &c->d.ccount, c->g.ncell));
   c->d.cbead = nullptr;   // slot arrays sized for the new grid
-  CHK(build_cells(c, 0));
   set_cand(c);
+  CHK(build_cells(c, 0));
   c->grid_gen++;
   return PLUM_OK;
 }
+
+constexpr int kFullSmall = 128;   // blocks of k_full_small
 
 // From-scratch energy on the device; with set_running the running totals,
 // dipole state and the per-molecule spring cache are reset to it.
 int run_full(plum_ctx* c, int set_running, double out[8]) {
   const Geo& g = c->g;
-  hipLaunchKernelGGL(k_full_real, dim3(c->nrealb), dim3(kBlock), 0, c->st, g, c->d);
-  if (g.use_ewald && g.n_kh > 0) {
-    hipLaunchKernelGGL(k_full_sk_part, dim3(c->nkb_full, c->nchunk), dim3(kBlock), 0, c->st, g, c->d,
-                       c->chunk);
+  hipLaunchKernelGGL(k_full_real, dim3(g.ncell, c->full_groups, c->full_parts), dim3(kBlock), 0, c->st, g, c->d,
+                     c->full_parts);
+  const bool ksp = g.use_ewald && g.n_kh > 0;
+  if (ksp) {
+    // by tiles where a step of four beads' tables fits the LDS stage
+    if (sk_sub(g.tab_w) >= 4)
+      hipLaunchKernelGGL(k_full_sk_tile, dim3((c->nkb_s + kQWaves - 1) / kQWaves, c->nchunk), dim3(kBlock), 0, c->st,
+                         g, c->d, c->chunk, c->nkb_s);
+    else
+      hipLaunchKernelGGL(k_full_sk_part, dim3(c->nkb_full, c->nchunk), dim3(kBlock), 0, c->st, g, c->d, c->chunk);
     hipLaunchKernelGGL(k_full_sk_reduce, dim3(c->nkb_full), dim3(kBlock), 0, c->st, g, c->d, c->nchunk,
                        c->epart_k);
   }
-  hipLaunchKernelGGL(k_full_small, dim3(1), dim3(kBlock), 0, c->st, g, c->d, c->nrealb,
-                     (g.use_ewald && g.n_kh > 0) ? c->nkb_full : 0, c->epart_k, set_running);
+  hipLaunchKernelGGL(k_full_small, dim3(kFullSmall), dim3(kBlock), 0, c->st, g, c->d, c->opart);
+  hipLaunchKernelGGL(k_full_final, dim3(1), dim3(kFinalThreads), 0, c->st, g, c->d,
+                     g.ncell * c->full_groups * c->full_parts * kQWaves, ksp ? c->nkb_full : 0, kFullSmall,
+                     c->epart_k, c->opart, set_running);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(c->h_ctl, c->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
@@ -515,8 +492,6 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
   c->nkb_full = std::max(1, (g.n_kh + kBlock - 1) / kBlock);
 
   c->mol_start.assign(ms, ms + n_mols + 1);
-  c->type_h.assign(type, type + n);
-  c->q_h.assign(q, q + n);
   int maxm = 1;
   for (int m = 0; m < n_mols; m++) maxm = std::max(maxm, ms[m + 1] - ms[m]);
   c->maxm = maxm;
@@ -524,6 +499,12 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
   info.n_mols = n_mols;
   info.max_mol_len = maxm;
   c->nmmb = nmm_blocks(maxm);
+  // bead chunks of the S(k) build: about 512 blocks over the groups of four
+  // tiles, 64 to 512 beads each
+  {
+    const int groups = std::max(1, (c->nkb_s + kQWaves - 1) / kQWaves), want = std::max(1, 512 / groups);
+    c->chunk = std::max(64, std::min(512, ((n + want - 1) / want + 63) / 64 * 64));
+  }
   c->nchunk = (n + c->chunk - 1) / c->chunk;
 
   if (hipGetDevice(&c->device) != hipSuccess || hipStreamCreate(&c->st) != hipSuccess) {
@@ -584,7 +565,7 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
   ALLOC(d.part_k, c->nkb); ALLOC(d.part_r, (size_t)kMaxProp * std::max(query_blocks(maxm, kMaxQBlock) * kQWaves, 2 * maxm * kMaxSplit));
   ALLOC(d.part_mm, (size_t)kMaxProp * c->nmmb);
   ALLOC(d.sk_part, (size_t)c->nchunk * std::max(1, g.n_kh));
-  ALLOC(c->epart_k, c->nkb_full);
+  ALLOC(c->epart_k, c->nkb_full); ALLOC(c->opart, 4 * kFullSmall); ALLOC(c->d_max, 1);
   ALLOC(d.chain_ids, n_mols); ALLOC(d.ion_ids, n_mols);
   // move record: header + idx[maxm] + pad + xyz[3 maxm], contiguous
   c->off_xyz = sizeof(MoveRec) + sizeof(int) * maxm + ((sizeof(int) * maxm) % 8);
@@ -599,6 +580,7 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
   }
 #undef ALLOC
   if (hipHostMalloc((void**)&c->h_in, c->in_bytes, hipHostMallocDefault) != hipSuccess ||
+      hipHostMalloc((void**)&c->h_max, sizeof(int), hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc((void**)&c->h_ctl, sizeof(Ctl), hipHostMallocDefault) != hipSuccess)
     return bail(fail(PLUM_E_NOMEM, "hipHostMalloc failed"));
   auto up = [&](void* dst, const void* src, size_t bytes) -> int {
@@ -652,6 +634,7 @@ int plum_destroy(plum_ctx* c) {
   for (void* p : c->dev_allocs) (void)hipFree(p);
   if (c->h_in) (void)hipHostFree(c->h_in);
   if (c->h_ctl) (void)hipHostFree(c->h_ctl);
+  if (c->h_max) (void)hipHostFree(c->h_max);
   if (c->ev_idle) (void)hipEventDestroy(c->ev_idle);
   if (c->st) (void)hipStreamDestroy(c->st);
   delete c;

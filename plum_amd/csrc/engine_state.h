@@ -143,7 +143,7 @@ struct Dev {
   double2* part_r;
   double2* part_mm;
   double2* sk_part;
-  double* fpart;
+  double2* fpart;         // from-scratch real-space partials, one per wave
   // device Monte Carlo
   int *chain_ids, *ion_ids;
   // speculative batches: proposal s's moved beads at s * maxm in mv_old /

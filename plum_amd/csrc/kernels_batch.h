@@ -130,6 +130,14 @@ __device__ __forceinline__ double uniform_double(double v) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// Lane `lane`'s value, in every lane.
+__device__ __forceinline__ double lane_double(double v, int lane) {
+  const unsigned long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, lane);
+  const unsigned hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), lane);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 // System r owning virtual block v: first r with pre[r] > v (inclusive prefix).
 __device__ __forceinline__ int find_replica(const int* pre, int R, int v) {
   int lo = 0, hi = R - 1;
@@ -690,39 +698,45 @@ struct QueryShare {
   int s_wsum[kQWaves];
   double4 s_pt[kCluster];  // query points (the image nearest the first point) and charges
   int s_ptt[kCluster];     // their types
+  int s_own[kCluster];     // their bead indices (ALL)
   QWaveSmem<P> q[kQWaves];
 };
 
-// LJ + real-space energy of the np points pts[0 .. np) (charges in .w, types
-// ptype[]) against every bead image in the cell list within the search
-// radius, skipping the index range [mlo, mhi] (the device loop's moves are
-// contiguous), over share `part` of `nparts` of the query's cells.  Each
-// wave's part of the result valid in its lane 0.
-template <int P>
-__device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4* __restrict__ pts,
-                                      const int* __restrict__ ptype, int np, int mlo, int mhi, int part, int nparts,
-                                      QueryShare<P>& sh) {
+// LJ + real-space energy of up to kCluster points (lane l holds point
+// l % kCluster: position and charge, type, whether it counts; at least one
+// does) against every bead image in the cell list within the search radius,
+// skipping the index range [mlo, mhi] (the device loop's moves are
+// contiguous), over share `part` of `nparts` of the query's cells.  ALL: the
+// points are beads of the list themselves, own their indices, and a point has
+// no LJ term with itself (its images lie beyond the LJ cutoff).  Each wave's
+// part of the result valid in its lane 0.
+template <int P, bool ALL>
+__device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4& p, int type, bool valid, int own,
+                                      int mlo, int mhi, int part, int nparts, QueryShare<P>& sh) {
   const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
   QWaveSmem<P>& sm = sh.q[wv];
   // each point as the image nearest the first point's wrapped position (an
   // image of a point has the same pair images within the radius), and the
-  // points' bounding box; lane l holds point l % kCluster (the last one again
-  // past the end)
+  // points' bounding box
+  const unsigned vm = (unsigned)__ballot(valid) & ((1u << kCluster) - 1u);
+  const int np = ALL ? kCluster : __popc(vm);
+  const int ref = __builtin_ctz(vm);
   double bl[3], bh[3];
   {
-    const int ip = min(lane % kCluster, np - 1);
-    const double4 p0 = pts[0], p = pts[ip];
-    const double p0v[3] = {p0.x, p0.y, p0.z}, pv[3] = {p.x, p.y, p.z};
+    const double p0v[3] = {lane_double(p.x, ref), lane_double(p.y, ref), lane_double(p.z, ref)};
+    const double pv[3] = {p.x, p.y, p.z};
     double qv[3];
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-      double dk = pv[k] - p0v[k];
+      double dk = valid ? pv[k] - p0v[k] : 0.0;
       dk -= g.L[k] * rint(dk * g.inv_L[k]);
       qv[k] = wrap_coord(p0v[k], g.L[k], g.inv_L[k]) + dk;
     }
-    if (threadIdx.x < np) {
-      sh.s_pt[lane] = make_double4(qv[0], qv[1], qv[2], p.w);
-      sh.s_ptt[lane] = ptype[lane];
+    if (threadIdx.x < kCluster) {
+      // (a point that does not count is out of every candidate's reach)
+      sh.s_pt[lane] = make_double4(valid ? qv[0] : -1e30, qv[1], qv[2], p.w);
+      sh.s_ptt[lane] = type;
+      sh.s_own[lane] = own;
     }
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -891,7 +905,9 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4*
         const double dx = cx - qp.x, dy = cy - qp.y, dz = cz - qp.z;
         const double r2 = dx * dx + dy * dy + dz * dz;
         // FP64 queue: every charged pair (P = 0), the close ones (P = 1)
-        const bool in = r2 <= rcj2;
+        // (a bead against itself: zero up to the rounding of the point's image)
+        const bool self = ALL && j == sh.s_own[i];
+        const bool in = r2 <= rcj2 && !(self && r2 < 1e-6);
         const bool near = in && (P == 0 || r2 < fp64_b2);
         const unsigned long long m = __ballot(near);
         if (m) {
@@ -910,7 +926,7 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4*
             if (fn >= kWave) drain32(kWave);
           }
         }
-        const bool lj = r2 < ljj2;
+        const bool lj = r2 < ljj2 && !self;
         const unsigned long long ml = __ballot(lj);
         if (ml) {
           if (lj) {
@@ -1045,8 +1061,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
       // beads c kCluster ..) at their old (on = 0) or new positions
       const int q2 = local / L.qb, part = local - q2 * L.qb;
       const int m0 = (q2 >> 1) * kCluster, on = q2 & 1;
-      const double2 eq = real_query_cluster<P>(g, v, (on ? v.mv_new : v.mv_old) + m0, v.mv_type + m0,
-                                               min(kCluster, nm - m0), lo, hi, part, L.qb, sm.q);
+      const int li = lane % kCluster, np = min(kCluster, nm - m0), pi = m0 + min(li, np - 1);
+      const double4 pt = (on ? v.mv_new : v.mv_old)[pi];
+      const double2 eq = real_query_cluster<P, false>(g, v, pt, v.mv_type[pi], li < np, 0, lo, hi, part, L.qb, sm.q);
       const double sgn = on ? 1.0 : -1.0;
       if (lane == 0) v.part_r[local * kQWaves + threadIdx.x / kWave] = make_double2(sgn * eq.x, sgn * eq.y);
     } else if ((b -= nqt) < rc.nkb_s * ne) {
@@ -1195,13 +1212,6 @@ struct ResSmem {
 };
 
 static_assert(kMaxScreen <= kWave, "one lane per proposal in the decision wave");
-
-__device__ __forceinline__ double lane_double(double v, int lane) {
-  const unsigned long long b = __double_as_longlong(v);
-  const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, lane);
-  const unsigned hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), lane);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
 
 // The reference's sequential Metropolis chain over the batch
 // (simulation.cc:241-355), one wave, one lane per proposal.  A pass

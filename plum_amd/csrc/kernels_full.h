@@ -1,73 +1,116 @@
-// From-scratch energy kernels: real space + LJ over all pairs through the
-// cell list, S(k) by direct summation, springs / wall / self / dipole, and the
-// reduction into the control block.
+// From-scratch kernels: the cell list, and the energy -- real space + LJ over
+// all pairs through the cell list, S(k) by direct summation, springs / wall /
+// self / dipole, and the reduction into the control block.
 #pragma once
-#include "kernels_move.h"
+#include "kernels_batch.h"
 
 namespace plum {
 
-// ============================================================ from scratch
-// Real space + LJ over all pairs: one thread per occupied cell slot; each
-// pair (and each self image, weight 1/2) is counted from its lower index.
-__global__ __launch_bounds__(kBlock) void k_full_real(Geo g, Dev d) {
-  __shared__ double sh[kBlock / kWave];
-  const long long gid = blockIdx.x * (long long)kBlock + threadIdx.x;
-  double elj = 0, ere = 0;
-  if (gid < (long long)g.ncell * g.cap) {
-    const int cell = (int)(gid / g.cap), slot = (int)(gid % g.cap);
-    const size_t si = (size_t)cell * g.cap + slot;
-    const int i = slot < d.ccount[cell] ? d.cbead[si] : -1;
-    if (i >= 0) {
-      const double4 p = d.cpos[si];
-      const LJPair* ljrow = d.lj + d.ctype[si] * g.n_types;
-      const double pw[3] = {p.x, p.y, p.z};
-      int lo[3], hi[3];
-      for (int k = 0; k < 3; k++) {
-        lo[k] = (int)floor((pw[k] - g.rs) * g.inv_h[k]);
-        hi[k] = (int)floor((pw[k] + g.rs) * g.inv_h[k]);
-      }
-      for (int ux = lo[0]; ux <= hi[0]; ux++) {
-        const int qx = floordiv(ux, g.nc[0]), wx = ux - qx * g.nc[0];
-        for (int uy = lo[1]; uy <= hi[1]; uy++) {
-          const int qy = floordiv(uy, g.nc[1]), wy = uy - qy * g.nc[1];
-          for (int uz = lo[2]; uz <= hi[2]; uz++) {
-            const int qz = floordiv(uz, g.nc[2]), wz = uz - qz * g.nc[2];
-            const int c2 = (wx * g.nc[1] + wy) * g.nc[2] + wz;
-            const int cnt = d.ccount[c2];
-            for (int s2 = 0; s2 < cnt; s2++) {
-              const size_t sj = (size_t)c2 * g.cap + s2;
-              const int j = d.cbead[sj];
-              if (j < i) continue;  // also skips tombstones (-1)
-              const double4 pj = d.cpos[sj];
-              const double dx = pj.x + qx * g.L[0] - pw[0];
-              const double dy = pj.y + qy * g.L[1] - pw[1];
-              const double dz = pj.z + qz * g.L[2] - pw[2];
-              const double r2 = dx * dx + dy * dy + dz * dz;
-              if (r2 > g.rs2) continue;
-              const double r = sqrt(r2);
-              if (j > i && g.use_pair && (g.npbc == 3 || qz == 0)) elj += lj_energy(r, ljrow[d.ctype[sj]]);
-              if (g.use_ewald) {
-                const double qq = p.w * pj.w;
-                if (qq != 0 && r > 0 && r <= g.rc) {
-                  const double e = g.lB * qq * erfc_nodes(g, g.sqrt_alpha * r) / r;
-                  ere += (j == i) ? 0.5 * e : e;
-                }
-              }
-            }
-          }
-        }
-      }
+// ============================================================ cell list
+// Built on the device in bead order: counts, then slots by atomics in any
+// order, then each cell's beads put in order of their index by rank (the slot
+// order a host counting sort gives).  On the host (download, sort, upload of
+// every slot array) the list of 40,000 beads took 2.2 ms.
+__global__ void k_cell_count(Geo g, Dev d) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= g.n) return;
+  const double xw = wrap_coord(d.x[i], g.L[0], g.inv_L[0]);
+  const double yw = wrap_coord(d.y[i], g.L[1], g.inv_L[1]);
+  const double zw = wrap_coord(d.z[i], g.L[2], g.inv_L[2]);
+  const int c = (cell_coord(xw, g.inv_h[0], g.nc[0]) * g.nc[1] + cell_coord(yw, g.inv_h[1], g.nc[1])) * g.nc[2] +
+                cell_coord(zw, g.inv_h[2], g.nc[2]);
+  d.bcell[i] = c;
+  atomicAdd(&d.ccount[c], 1);
+}
+
+// Largest cell count into *out (zeroed by the caller).
+__global__ __launch_bounds__(kBlock) void k_cell_max(Geo g, Dev d, int* out) {
+  int m = 0;
+  for (int c = blockIdx.x * kBlock + threadIdx.x; c < g.ncell; c += gridDim.x * kBlock) m = max(m, d.ccount[c]);
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, kWave));
+  if (threadIdx.x % kWave == 0) atomicMax(out, m);
+}
+
+// Bead i takes some slot of its cell (counts zeroed by the caller and counted
+// again here); ctype holds the bead index until k_cell_order.
+__global__ void k_cell_fill(Geo g, Dev d) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= g.n) return;
+  const int c = d.bcell[i];
+  d.ctype[(size_t)c * g.cap + atomicAdd(&d.ccount[c], 1)] = i;
+}
+
+// One block per cell: the bead of rank s among the cell's indices goes to
+// slot s; the slots past the count are empty.
+__global__ __launch_bounds__(kBlock) void k_cell_order(Geo g, Dev d) {
+  __shared__ int s_idx[kBlock];
+  const int c = blockIdx.x;
+  const int cnt = d.ccount[c];
+  const size_t c0 = (size_t)c * g.cap;
+  for (int s0 = 0; s0 < cnt; s0 += kBlock) {
+    const int s = s0 + threadIdx.x;
+    const int j = s < cnt ? d.ctype[c0 + s] : 0;
+    int rank = 0;
+    for (int t0 = 0; t0 < cnt; t0 += kBlock) {
+      __syncthreads();
+      if (t0 + threadIdx.x < cnt) s_idx[threadIdx.x] = d.ctype[c0 + t0 + threadIdx.x];
+      __syncthreads();
+      const int m = min(kBlock, cnt - t0);
+      for (int t = 0; t < m; t++) rank += s_idx[t] < j;
     }
+    if (s < cnt) d.cbead[c0 + rank] = j;
   }
-  const double a = block_sum<kBlock>(elj, sh);
-  const double c = block_sum<kBlock>(ere, sh);
-  if (threadIdx.x == 0) {
-    d.fpart[2 * blockIdx.x] = a;
-    d.fpart[2 * blockIdx.x + 1] = c;
+  for (int s = cnt + threadIdx.x; s < g.cap; s += kBlock) d.cbead[c0 + s] = -1;
+  __syncthreads();   // the cell's slots are written, and its index copies read
+  const int cx = c / (g.nc[1] * g.nc[2]), cy = (c / g.nc[2]) % g.nc[1], cz = c % g.nc[2];
+  for (int s = threadIdx.x; s < cnt; s += kBlock) {
+    const int j = d.cbead[c0 + s];
+    const double xw = wrap_coord(d.x[j], g.L[0], g.inv_L[0]);
+    const double yw = wrap_coord(d.y[j], g.L[1], g.inv_L[1]);
+    const double zw = wrap_coord(d.z[j], g.L[2], g.inv_L[2]);
+    const double q = d.q[j];
+    d.cpos[c0 + s] = make_double4(xw, yw, zw, q);
+    d.cpos32[c0 + s] = make_float4((float)(xw - cx * g.h[0]), (float)(yw - cy * g.h[1]), (float)(zw - cz * g.h[2]),
+                                   (float)q);
+    d.ctype[c0 + s] = d.type[j];
+    d.bslot[j] = s;
   }
 }
 
-// S(k) from scratch, bead chunk `blockIdx.y`: direct FP64 sincos per (k, bead)
+// ============================================================ from scratch
+// Real space + LJ over all pairs: the cluster queries of the device loop with
+// the beads of a cell, kCluster slots at a time, as the points.  Every ordered
+// pair is visited, half of each counted (a bead's own images have weight 1/2
+// as it is), which costs half as many pair terms again as one thread per slot
+// that walks the cells around it, and none of its waits: 2.6 ms for 40,000
+// beads, and 8.5 ms for 3,200 beads in a box of 1.4 r_c, that way.
+// Block (cell, slot group, share of the query's cells).
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_full_real(Geo g, Dev d,
+                                                                                              int nparts) {
+  __shared__ QueryShare<0> sm;
+  const int cell = blockIdx.x, part = blockIdx.z, lane = threadIdx.x % kWave;
+  const int cnt = d.ccount[cell];
+  double elj = 0, ere = 0;
+  for (int s0 = blockIdx.y * kCluster; s0 < cnt; s0 += gridDim.y * kCluster) {
+    const int s = s0 + lane % kCluster;
+    const size_t si = (size_t)cell * g.cap + min(s, cnt - 1);
+    const int own = s < cnt ? d.cbead[si] : -1;
+    if (!__ballot(own >= 0)) continue;
+    const double2 e = real_query_cluster<0, true>(g, d, d.cpos[si], d.ctype[si], own >= 0, own, 0, -1, part, nparts,
+                                                  sm);
+    elj += e.x;
+    ere += e.y;
+    __syncthreads();   // the next group rewrites the points
+  }
+  if (lane == 0) {
+    const size_t b = ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    d.fpart[b * kQWaves + threadIdx.x / kWave] = make_double2(0.5 * elj, 0.5 * ere);
+  }
+}
+
+// S(k) from scratch, bead chunk `blockIdx.y`: direct FP64 sincos per (k,
+// bead), for phase tables that do not fit the LDS of k_full_sk_tile.
 __global__ __launch_bounds__(kBlock) void k_full_sk_part(Geo g, Dev d, int chunk) {
   const int k = blockIdx.x * kBlock + threadIdx.x;
   if (k >= g.n_kh) return;
@@ -91,6 +134,72 @@ __global__ __launch_bounds__(kBlock) void k_full_sk_part(Geo g, Dev d, int chunk
   d.sk_part[(size_t)blockIdx.y * g.n_kh + k] = make_double2(sr, si);
 }
 
+// The same on the matrix cores: block (four k tiles, bead chunk), a wave per
+// tile.  The chunk's phase tables are built in LDS, `sub` beads at a time
+// (tables_row, one thread per bead and dimension), and each wave adds its
+// tile's products over them (kspace_spec_block's form, one position per bead).
+// 40,000 beads and 10,683 vectors: 1.49 ms by sincos, 427 million of them.
+constexpr int kSkStage = 3072;   // LDS table entries (48 KB)
+__host__ __device__ __forceinline__ int sk_sub(int tab_w) { return min(kBlock / 4, kSkStage / (tab_w | 1)) / 4 * 4; }
+
+__global__ __launch_bounds__(kBlock) void k_full_sk_tile(Geo g, Dev d, int chunk, int ntile) {
+  __shared__ double2 s_tab[kSkStage];
+  __shared__ double s_q[kBlock / 4];
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+  const int tile = blockIdx.x * kQWaves + w;
+  const int ws = g.tab_w | 1, nsub = sk_sub(g.tab_w);
+  const int col = lane % kKTile, sub = lane / kKTile;
+  int4 row = make_int4(0, 0, 0, -1);
+  int lz = 0;
+  if (tile < ntile) {
+    const int2 tl = d.ktile[tile];
+    row = d.krow[tl.x + col];
+    lz = tl.y + col;
+  }
+  const int ox = row.x, oy = g.nkx + 1 + abs(row.y), oz = g.nkx + 1 + g.nky + 1 + min(lz, g.nkz);
+  const double sy = row.y < 0 ? -1.0 : 1.0;
+  f64x4 rr = {0, 0, 0, 0}, ii = rr, ri = rr, ir = rr;
+  const int j0 = blockIdx.y * chunk, j1 = min(g.n, j0 + chunk);
+  for (int b0 = j0; b0 < j1; b0 += nsub) {
+    const int nb = min(nsub, j1 - b0);
+    __syncthreads();   // the last sub-chunk's tables are read
+    for (int t = threadIdx.x; t < 3 * nsub; t += kBlock) {
+      const int m = t / 3, dim = t - 3 * m;
+      // (a place past the chunk repeats its last bead, with no charge)
+      const int j = b0 + min(m, nb - 1);
+      tables_row(g, dim, dim == 0 ? d.x[j] : (dim == 1 ? d.y[j] : d.z[j]), s_tab + (size_t)m * ws);
+      if (dim == 0) s_q[m] = m < nb ? d.q[j] : 0.0;
+    }
+    __syncthreads();
+    if (tile < ntile)
+#pragma unroll 2
+      for (int i0 = 0; i0 < nsub; i0 += 4) {
+        const double2* t = s_tab + (size_t)(i0 + sub) * ws;
+        const double2 X = t[ox], Y = t[oy], Z = t[oz];
+        const double q = s_q[i0 + sub];
+        const double yr = q * Y.x, yi = q * sy * Y.y;
+        const double ar = X.x * yr - X.y * yi, ai = X.x * yi + X.y * yr;
+        rr = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, Z.x, rr, 0, 0, 0);
+        ii = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, Z.y, ii, 0, 0, 0);
+        ri = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, Z.y, ri, 0, 0, 0);
+        ir = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, Z.x, ir, 0, 0, 0);
+      }
+  }
+  if (tile >= ntile) return;
+  double2* out = d.sk_part + (size_t)blockIdx.y * g.n_kh;
+#pragma unroll
+  for (int v = 0; v < 4; v++) {
+    const int src = 4 * v + sub;
+    const int first = __shfl(row.z, src, kWave), m = __shfl(row.w, src, kWave);
+    const int xy = __shfl(row.x | row.y, src, kWave);   // 0: the l_x = l_y = 0 row, which holds l_z > 0 only
+    if (lz <= m) {
+      const int k0 = xy ? first + m : first - 1;
+      if (xy || lz > 0) out[k0 + lz] = make_double2(rr[v] - ii[v], ri[v] + ir[v]);
+      if (xy && lz > 0) out[k0 - lz] = make_double2(rr[v] + ii[v], ir[v] - ri[v]);
+    }
+  }
+}
+
 __global__ __launch_bounds__(kBlock) void k_full_sk_reduce(Geo g, Dev d, int nchunk,
                                                            double* epart) {
   __shared__ double sh[kBlock / kWave];
@@ -98,6 +207,7 @@ __global__ __launch_bounds__(kBlock) void k_full_sk_reduce(Geo g, Dev d, int nch
   double e = 0;
   if (k < g.n_kh) {
     double2 s = make_double2(0, 0);
+#pragma unroll 8
     for (int c = 0; c < nchunk; c++) {
       const double2 v = d.sk_part[(size_t)c * g.n_kh + k];
       s.x += v.x;
@@ -110,40 +220,85 @@ __global__ __launch_bounds__(kBlock) void k_full_sk_reduce(Geo g, Dev d, int nch
   if (threadIdx.x == 0) epart[blockIdx.x] = r;
 }
 
-// Per-molecule springs, wall, self energy and the dipole moment; then the
-// final reduction of all from-scratch partials into the control block.
-__global__ __launch_bounds__(kBlock) void k_full_small(Geo g, Dev d, int nrealb, int nkb,
-                                                       const double* epart_k, int set_running) {
-  __shared__ double sh[kBlock / kWave];
-  __shared__ double sbuf[kBlock];
-  Ctl* C = d.ctl;
-  double eb_all = 0;
-  if (g.use_bond) {
-    for (int m = 0; m < g.n_mols; m++) {
+// Spring energy of a molecule at its current coordinates by one wave: the
+// per-bond terms and the order of their sum are molecule_spring's (waves of
+// 64 bonds, then the waves of a block in order, then the blocks), so the bits
+// are the same.  Valid in lane 0.
+__device__ double molecule_spring_wave(const Geo& g, const Dev& d, int a, int b) {
+  const int lane = threadIdx.x % kWave;
+  double acc = 0;
+  for (int base = a; base < b - 1; base += kBlock) {
+    double blk = 0;
+    for (int w0 = base; w0 < min(base + kBlock, b - 1); w0 += kWave) {
+      const int i = w0 + lane;
       double e = 0;
-      if (d.mol_start[m + 1] - d.mol_start[m] > 1) e = molecule_spring(g, d, m, false, sbuf);
-      if (threadIdx.x == 0) {
+      if (i < b - 1) {
+        const double dx = d.x[i] - d.x[i + 1], dy = d.y[i] - d.y[i + 1], dz = d.z[i] - d.z[i + 1];
+        e = spring_energy(g, dx, dy, dz);
+      }
+      blk += wave_sum(e);
+    }
+    acc += blk;
+  }
+  return acc;
+}
+
+// Springs per molecule (a wave each, grid-stride) and wall, self and dipole
+// sums over the beads: block partials opart[4 b ..] = springs, wall, self,
+// M_z.  (One block over all molecules in turn: 3.7 ms for 20,200 molecules.)
+__global__ __launch_bounds__(kBlock) void k_full_small(Geo g, Dev d, double* opart) {
+  __shared__ double sh[kBlock / kWave];
+  const int lane = threadIdx.x % kWave;
+  double eb = 0;
+  if (g.use_bond)
+    for (int m = blockIdx.x * kQWaves + threadIdx.x / kWave; m < g.n_mols; m += gridDim.x * kQWaves) {
+      const int a = d.mol_start[m], b = d.mol_start[m + 1];
+      const double e = b - a > 1 ? molecule_spring_wave(g, d, a, b) : 0.0;
+      if (lane == 0) {
         d.bond_cur[m] = e;
-        eb_all += e;
+        eb += e;
       }
     }
-  }
   double ew = 0, es = 0, mz = 0;
-  for (int i = threadIdx.x; i < g.n; i += kBlock) {
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < g.n; i += gridDim.x * kBlock) {
     const double qi = d.q[i];
     if (g.use_ext) ew += wall_energy(d.z[i], d.wall[d.type[i]], g);
     es += g.self_coef * qi * qi;
     mz += qi * d.z[i];
   }
-  double vl = 0, vr = 0, vk = 0;
-  for (int b = threadIdx.x; b < nrealb; b += kBlock) { vl += d.fpart[2 * b]; vr += d.fpart[2 * b + 1]; }
-  for (int b = threadIdx.x; b < nkb; b += kBlock) vk += epart_k[b];
-  const double ewt = block_sum<kBlock>(ew, sh);
-  const double est = block_sum<kBlock>(es, sh);
-  const double mzt = block_sum<kBlock>(mz, sh);
-  const double lt = block_sum<kBlock>(vl, sh);
-  const double rt = block_sum<kBlock>(vr, sh);
-  const double kt = block_sum<kBlock>(vk, sh);
+  const double v4[4] = {eb, ew, es, mz};
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const double t = block_sum<kBlock>(v4[k], sh);
+    if (threadIdx.x == 0) opart[4 * blockIdx.x + k] = t;
+  }
+}
+
+// The final reduction of all from-scratch partials into the control block.
+constexpr int kFinalThreads = 1024;
+__global__ __launch_bounds__(kFinalThreads) void k_full_final(Geo g, Dev d, int nrealp, int nkb, int nob,
+                                                              const double* epart_k, const double* opart,
+                                                              int set_running) {
+  __shared__ double sh[kFinalThreads / kWave];
+  Ctl* C = d.ctl;
+  double vl = 0, vr = 0, vk = 0, vo[4] = {0, 0, 0, 0};
+#pragma unroll 4
+  for (int b = threadIdx.x; b < nrealp; b += kFinalThreads) {
+    const double2 e = d.fpart[b];
+    vl += e.x;
+    vr += e.y;
+  }
+  for (int b = threadIdx.x; b < nkb; b += kFinalThreads) vk += epart_k[b];
+  for (int b = threadIdx.x; b < nob; b += kFinalThreads)
+#pragma unroll
+    for (int k = 0; k < 4; k++) vo[k] += opart[4 * b + k];
+  const double ebt = block_sum<kFinalThreads>(vo[0], sh);
+  const double ewt = block_sum<kFinalThreads>(vo[1], sh);
+  const double est = block_sum<kFinalThreads>(vo[2], sh);
+  const double mzt = block_sum<kFinalThreads>(vo[3], sh);
+  const double lt = block_sum<kFinalThreads>(vl, sh);
+  const double rt = block_sum<kFinalThreads>(vr, sh);
+  const double kt = block_sum<kFinalThreads>(vk, sh);
   if (threadIdx.x == 0) {
     double f[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (g.use_pair) f[T_LJ] = lt;
@@ -153,7 +308,7 @@ __global__ __launch_bounds__(kBlock) void k_full_small(Geo g, Dev d, int nrealb,
       f[T_SELF] = est;
       if (g.dipole) f[T_DIPOLE] = dipole_energy(g.dip_coef, mzt);
     }
-    if (g.use_bond) f[T_BOND] = eb_all;
+    if (g.use_bond) f[T_BOND] = ebt;
     if (g.use_ext) f[T_WALL] = ewt;
     for (int k = 0; k < 8; k++) C->full[k] = f[k];
     if (set_running) {

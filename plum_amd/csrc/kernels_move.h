@@ -392,6 +392,14 @@ __global__ __launch_bounds__(kBlock) void k_compute(Geo g, Dev d, int nkb, int n
 }
 
 // ------------------------------------------------------------ epilogue
+// One spring (potential_spring.cc:33-41).  No product is fused with a later
+// sum, so every kernel that evaluates a bond gets the same bits.
+__device__ __forceinline__ double spring_energy(const Geo& g, double dx, double dy, double dz) {
+#pragma clang fp contract(off)
+  const double u = sqrt(dx * dx + dy * dy + dz * dz) - g.r0;
+  return 0.5 * g.k_bond * u * u;
+}
+
 // Spring energy of molecule `mol` (potential_spring.cc:22-47: consecutive
 // beads, no PBC).  Per-bond terms are summed by a fixed-order block tree, so
 // the same bits come out whichever kernel evaluates the molecule.
@@ -410,8 +418,7 @@ __device__ double molecule_spring(const Geo& g, const Dev& d, int mol, bool tria
         if (s1 >= 0) { const double4 v = d.mv_new[s1]; p1[0] = v.x; p1[1] = v.y; p1[2] = v.z; }
       }
       const double dx = p0[0] - p1[0], dy = p0[1] - p1[1], dz = p0[2] - p1[2];
-      const double r = sqrt(dx * dx + dy * dy + dz * dz);
-      e = 0.5 * g.k_bond * (r - g.r0) * (r - g.r0);
+      e = spring_energy(g, dx, dy, dz);
     }
     acc += block_sum<kBlock>(e, sbuf);
   }
@@ -434,8 +441,7 @@ __device__ double molecule_spring_range(const Geo& g, const Dev& d, int mol, int
       if (i >= lo && i <= hi) { const double4 v = mv_new[i - lo]; p0[0] = v.x; p0[1] = v.y; p0[2] = v.z; }
       if (i + 1 >= lo && i + 1 <= hi) { const double4 v = mv_new[i + 1 - lo]; p1[0] = v.x; p1[1] = v.y; p1[2] = v.z; }
       const double dx = p0[0] - p1[0], dy = p0[1] - p1[1], dz = p0[2] - p1[2];
-      const double r = sqrt(dx * dx + dy * dy + dz * dz);
-      e = 0.5 * g.k_bond * (r - g.r0) * (r - g.r0);
+      e = spring_energy(g, dx, dy, dz);
     }
     acc += block_sum<kBlock>(e, sbuf);
   }

@@ -76,3 +76,56 @@ def test_kspace_tiles(box, alpha, chain_len):
     replay(sd, recs, 1e-10)
     run, full = eng.totals(), eng.energy_full()
     assert abs(run["kspace"] - full["kspace"]) <= 1e-10 * max(1.0, abs(full["kspace"]))
+
+
+def _full_matches(eng, orc, rel=1e-10):
+    got, ref = eng.energy_full(), orc.energy_full()
+    for k in E.TERMS:
+        assert abs(got[k] - ref[k]) <= rel * max(abs(ref[k]), 1e-2), (k, got[k], ref[k])
+
+
+@pytest.mark.parametrize("n_chains,chain_len,salt,L,alpha,cell_div", [
+    (1, 2, 0, 12.0, 0.2, 1),        # four beads, most cells empty
+    (2, 3, 1, 6.0, 0.05, 2),        # three image shells, one pair of ions
+    (7, 9, 11, 16.0, 0.3, 3),       # odd counts
+    (3, 100, 40, 14.0, 0.1, 1),     # one cell of 680 beads
+])
+def test_from_scratch_energy_and_cell_order(n_chains, chain_len, salt, L, alpha, cell_div):
+    """The device-built cell list and the from-scratch sums (cluster queries,
+    S(k) tiles, springs by waves), fresh, after moves that leave tombstones,
+    and after a resync."""
+    sd = systems.config("tiny")
+    from plum_amd import host
+    xyz, q, ty, ms = host.synth_system(n_chains, chain_len, n_chains * chain_len, salt, [L, L, L], 5)
+    q = np.where(np.arange(len(q)) % 7 == 3, 0.0, q)
+    sd.update(xyz=xyz, q=q, type=ty, mol_start=ms, box=[L, L, L], alpha=alpha)
+    eng = E.Engine(sd, cell_div=cell_div)
+    _full_matches(eng, O.Oracle(sd))
+    rng = np.random.default_rng(1)
+    for k in range(6):
+        idx = np.arange(ms[k % n_chains], ms[k % n_chains + 1], dtype=np.int32)
+        eng.delta(k % n_chains, idx, eng.positions()[idx] + rng.uniform(-2, 2, 3))
+        eng.finalize(True)
+    orc = O.Oracle(dict(sd, xyz=eng.positions()))
+    _full_matches(eng, orc)
+    run = eng.totals()
+    drift = eng.resync()
+    after = eng.totals()
+    for k in E.TERMS:
+        assert abs(run[k] - after[k] - drift[k]) <= 1e-12 * max(1.0, abs(run[k]))
+    _full_matches(eng, orc)
+
+
+def test_spring_energy_has_one_set_of_bits():
+    """The molecule springs of the from-scratch pass equal the trial path's
+    bit for bit: a move that changes nothing has a spring dE of exactly 0."""
+    sd = systems.config("tiny")
+    from plum_amd import host
+    xyz, q, ty, ms = host.synth_system(2, 700, 0, 0, [40.0, 40.0, 40.0], 9, bead_q=0.0)
+    sd.update(xyz=xyz, q=q, type=ty, mol_start=ms, box=[40.0, 40.0, 40.0], alpha=0.05)
+    eng = E.Engine(sd)
+    for mol in (0, 1):
+        idx = np.arange(ms[mol], ms[mol + 1], dtype=np.int32)
+        _, d = eng.delta(mol, idx, xyz[idx])
+        eng.finalize(False)
+        assert d["bond"] == 0.0

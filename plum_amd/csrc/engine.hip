@@ -176,7 +176,7 @@ int build_cells(plum_ctx* c, int min_cap) {
   c->full_groups = std::max(1, std::min((maxc + kCluster - 1) / kCluster, 65535));
   const long long blocks = (long long)g.ncell * c->full_groups;
   c->full_parts = (int)std::max(1LL, std::min<long long>(kMaxQBlock, std::min<long long>(
-                      1024 / blocks, (long long)(c->cand / kQShare))));
+                      4096 / blocks, (long long)(c->cand / kQShare))));
   const size_t fp = (size_t)blocks * c->full_parts * kQWaves;
   if (fp > c->fpart_cap) {
     CHK(dalloc(c, &c->d.fpart, fp));

@@ -681,16 +681,41 @@ __device__ void kspace_spec_block(const Geo& g, const Dev& d, const RepCfg& rc, 
 constexpr int kQueue = 2 * kWave;   // < 64 left after a drain, one push of up to 64
 static_assert(kCluster <= kWave, "one lane per query point");
 
-template <int P>
+// What a cluster query sums: the moved beads of a proposal against the rest;
+// every bead of the list against all (from scratch); the same as the change
+// under the stretch of a volume perturbation.
+enum QueryMode { Q_MOVED = 0, Q_ALL = 1, Q_STRETCH = 2 };
+
+// Stretched configuration of a volume perturbation: per bead the displacement
+// of the image that the cell list holds, the displacement of one period, the
+// number of surface-site molecules.
+struct StretchArgs {
+  const double* dw;
+  const int* mol_of;
+  double dz;
+  int phantom;
+};
+
+// Class of a molecule in the pair rule of a volume perturbation: mobile 0,
+// first / second half of the surface sites 1 / 2; pairs 0-0, 0-1 and 1-2 count
+// (pressure.cc:271-272: a site pairs only from the first half of the list).
+__device__ __forceinline__ int stretch_class(int mol, int phantom) {
+  return mol >= phantom ? 0 : (mol < phantom / 2 ? 1 : 2);
+}
+__device__ __forceinline__ bool stretch_pair(int a, int b) { return a + b <= 1 || (a != b && a > 0 && b > 0); }
+
+template <int P, int MODE>
 struct QWaveSmem {
   double2 s_q[kQueue];     // squared distance and charge product of a queued pair
   double s_lr[kQueue];     // squared distance of a queued LJ pair
   int s_lt[kQueue];        // its LJ pair index
   // P = 1: the queue of charged pairs at or beyond fp64_below, evaluated in FP32
   float2 s_f[P ? kQueue : 1];
+  // Q_STRETCH: the stretched squared distances of the queued pairs
+  double s_qn[MODE == Q_STRETCH ? kQueue : 1], s_ln[MODE == Q_STRETCH ? kQueue : 1];
 };
 
-template <int P>
+template <int P, int MODE>
 struct QueryShare {
   int s_cell[kBlock];      // cells of this share, their images and count prefix
   int s_img[kBlock];
@@ -698,23 +723,33 @@ struct QueryShare {
   int s_wsum[kQWaves];
   double4 s_pt[kCluster];  // query points (the image nearest the first point) and charges
   int s_ptt[kCluster];     // their types
-  int s_own[kCluster];     // their bead indices (ALL)
-  QWaveSmem<P> q[kQWaves];
+  int s_own[kCluster];     // their bead indices (not Q_MOVED)
+  double s_ptd[kCluster];  // their displacements and classes (Q_STRETCH)
+  int s_cls[kCluster];
+  QWaveSmem<P, MODE> q[kQWaves];
 };
 
 // LJ + real-space energy of up to kCluster points (lane l holds point
 // l % kCluster: position and charge, type, whether it counts; at least one
 // does) against every bead image in the cell list within the search radius,
 // skipping the index range [mlo, mhi] (the device loop's moves are
-// contiguous), over share `part` of `nparts` of the query's cells.  ALL: the
-// points are beads of the list themselves, own their indices, and a point has
-// no LJ term with itself (its images lie beyond the LJ cutoff).  Each wave's
-// part of the result valid in its lane 0.
-template <int P, bool ALL>
+// contiguous), over share `part` of `nparts` of the query's cells.  Not
+// Q_MOVED: the points are beads of the list themselves, own their indices, and
+// each pair counts once (LJ needs no self images: they lie beyond its cutoff).
+// Q_STRETCH: each pair's stretched minus current energy, over the pairs within
+// the cutoff in either (the search reaches kStretchMargin further, more than
+// a separation changes).  Each wave's part of the result valid in its lane 0.
+constexpr double kStretchMargin = 1e-3;
+
+template <int P, int MODE>
 __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4& p, int type, bool valid, int own,
-                                      int mlo, int mhi, int part, int nparts, QueryShare<P>& sh) {
+                                      int mlo, int mhi, int part, int nparts, QueryShare<P, MODE>& sh,
+                                      const StretchArgs& st = StretchArgs{nullptr, nullptr, 0, 0}) {
+  constexpr bool ALL = MODE != Q_MOVED;
+  constexpr bool STR = MODE == Q_STRETCH;
   const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
-  QWaveSmem<P>& sm = sh.q[wv];
+  const double rs = STR ? g.rs + kStretchMargin : g.rs, rs2 = STR ? rs * rs : g.rs2;
+  QWaveSmem<P, MODE>& sm = sh.q[wv];
   // each point as the image nearest the first point's wrapped position (an
   // image of a point has the same pair images within the radius), and the
   // points' bounding box
@@ -737,6 +772,12 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
       sh.s_pt[lane] = make_double4(valid ? qv[0] : -1e30, qv[1], qv[2], p.w);
       sh.s_ptt[lane] = type;
       sh.s_own[lane] = own;
+      if constexpr (STR) {
+        // the point's image is p's own: qv is p wrapped near the reference
+        const int jo = valid ? own : 0;
+        sh.s_ptd[lane] = valid ? st.dw[jo] + rint((qv[2] - p.z) * g.inv_L[2]) * st.dz : 0.0;
+        sh.s_cls[lane] = stretch_class(st.mol_of[jo], st.phantom);
+      }
     }
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -760,14 +801,20 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
   int lo[3], nd[3];
 #pragma unroll
   for (int k = 0; k < 3; k++) {
-    lo[k] = (int)floor((bl[k] - g.rs) * g.inv_h[k]);
-    const int hi = (int)floor((bh[k] + g.rs) * g.inv_h[k]);
+    lo[k] = (int)floor((bl[k] - rs) * g.inv_h[k]);
+    const int hi = (int)floor((bh[k] + rs) * g.inv_h[k]);
     nd[k] = hi - lo[k] + 1;
   }
   const int ncq = nd[0] * nd[1] * nd[2];
   const int mine = (ncq + nparts - 1) / nparts;   // cells of this share, at most
   const int nt = g.n_types;
-  const double rc2 = g.use_ewald ? g.rc * g.rc : -1.0, lj2 = g.use_pair ? g.lj2_max : -1.0;
+  const double rcs = STR ? g.rc + kStretchMargin : g.rc;
+  const double rc2 = g.use_ewald ? rcs * rcs : -1.0;
+  double lj2 = g.use_pair ? g.lj2_max : -1.0;
+  if (STR && g.use_pair) {
+    const double c = sqrt(g.lj2_max) + kStretchMargin;
+    lj2 = c * c;
+  }
   const double fp64_b2 = P ? g.fp64_below * g.fp64_below : 0.0;
   double elj = 0, ere = 0;
   int qn = 0, ln = 0, fn = 0;   // queue fills (wave-uniform)
@@ -782,7 +829,17 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
       const double x = g.sqrt_alpha * r;
       const int ni = erfc_node_index(x);
       const double u = erfc_from_node(x, ni, g.erfc_tab[ni]) * rinv;
-      if (e.x > 0) ere = fma(e.y, u, ere);
+      if constexpr (!STR) {
+        if (e.x > 0) ere = fma(e.y, u, ere);
+      } else {
+        const double n2 = sm.s_qn[qn + lane];
+        double rn, rninv;
+        sqrt_rsqrt(n2, rn, rninv);
+        const double xn = g.sqrt_alpha * rn;
+        const int nn = erfc_node_index(xn);
+        const double un = erfc_from_node(xn, nn, g.erfc_tab[nn]) * rninv;
+        ere += e.y * ((n2 > 0 && rn <= g.rc ? un : 0.0) - (e.x > 0 && r <= g.rc ? u : 0.0));
+      }
     }
     wave_sync_lds();
   };
@@ -802,7 +859,11 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
   auto drain_lj = [&](int count) {
     wave_sync_lds();
     ln -= count;
-    if (lane < count) elj += lj_energy(sqrt(sm.s_lr[ln + lane]), d.lj[sm.s_lt[ln + lane]]);
+    if (lane < count) {
+      const LJPair lp = d.lj[sm.s_lt[ln + lane]];
+      const double u = lj_energy(sqrt(sm.s_lr[ln + lane]), lp);
+      elj += STR ? lj_energy(sqrt(sm.s_ln[ln + lane]), lp) - u : u;
+    }
     wave_sync_lds();
   };
   for (int base = 0; base < mine; base += kBlock) {
@@ -829,14 +890,14 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
       sh.s_img[threadIdx.x] = img;
       // cells whose box (widened by a rounding margin) lies beyond the search
       // radius of the bounding box hold no candidate
-      double dmin2 = c < ncq ? 0 : 2 * g.rs2 + 1;
+      double dmin2 = c < ncq ? 0 : 2 * rs2 + 1;
 #pragma unroll
       for (int k = 0; k < 3; k++) {
         const double b0 = (double)u[k] * g.h[k] - 1e-9 * g.L[k], b1 = b0 + g.h[k] + 2e-9 * g.L[k];
         const double dd = fmax(0.0, fmax(b0 - bh[k], bl[k] - b1));
         dmin2 += dd * dd;
       }
-      end = dmin2 > g.rs2 ? 0 : d.ccount[cell];
+      end = dmin2 > rs2 ? 0 : d.ccount[cell];
     }
 #pragma unroll
     for (int o = 1; o < kWave; o <<= 1) {
@@ -898,20 +959,39 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
       const double cx = ok ? pj.x + ix * g.L[0] : 1e30, cy = pj.y + iy * g.L[1], cz = pj.z + iz * g.L[2];
       const double qj = g.lB * pj.w;
       const double rcj2 = pj.w != 0 ? rc2 : -1.0;
-      const double ljj2 = (g.npbc == 3 || iz == 0) ? lj2 : -1.0;
+      double ljj2 = (g.npbc == 3 || iz == 0) ? lj2 : -1.0;
+      double cd = 0;   // displacement of the candidate's image, its class
+      int cj = 0;
+      if constexpr (STR) {
+        cd = (ok ? st.dw[j] : 0.0) + iz * st.dz;
+        cj = ok ? stretch_class(st.mol_of[j], st.phantom) : 0;
+        if (cj) ljj2 = -1.0;   // LJ between mobile beads only
+      }
 #pragma unroll 1
       for (int i = 0; i < np; i++) {
         const double4 qp = sh.s_pt[i];
         const double dx = cx - qp.x, dy = cy - qp.y, dz = cz - qp.z;
         const double r2 = dx * dx + dy * dy + dz * dz;
+        double n2 = 0;
+        if constexpr (STR) {
+          // the same rounding of dz in both separations
+          const double dn = dz + (cd - sh.s_ptd[i]);
+          n2 = dx * dx + dy * dy + dn * dn;
+        }
         // FP64 queue: every charged pair (P = 0), the close ones (P = 1)
-        // (a bead against itself: zero up to the rounding of the point's image)
-        const bool self = ALL && j == sh.s_own[i];
-        const bool in = r2 <= rcj2 && !(self && r2 < 1e-6);
+        // ALL: a pair counts from its lower index, a bead's own images by half
+        // (the bead itself is at zero, up to the rounding of the point's image)
+        const int own = ALL ? sh.s_own[i] : -1;
+        const bool self = ALL && j == own;
+        const bool in = r2 <= rcj2 && (!ALL || j > own || (self && r2 > 1e-6)) &&
+                        (!STR || stretch_pair(sh.s_cls[i], cj));
         const bool near = in && (P == 0 || r2 < fp64_b2);
         const unsigned long long m = __ballot(near);
         if (m) {
-          if (near) sm.s_q[qn + lanes_below(m)] = make_double2(r2, qp.w * qj);
+          if (near) {
+            sm.s_q[qn + lanes_below(m)] = make_double2(r2, self ? 0.5 * (qp.w * qj) : qp.w * qj);
+            if constexpr (STR) sm.s_qn[qn + lanes_below(m)] = n2;
+          }
           qn += __popcll(m);
           if (qn >= kWave) drain(kWave);
         }
@@ -926,12 +1006,13 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
             if (fn >= kWave) drain32(kWave);
           }
         }
-        const bool lj = r2 < ljj2 && !self;
+        const bool lj = r2 < ljj2 && (!ALL || j > own) && (!STR || sh.s_cls[i] == 0);
         const unsigned long long ml = __ballot(lj);
         if (ml) {
           if (lj) {
             const int k = ln + lanes_below(ml);
             sm.s_lr[k] = r2;
+            if constexpr (STR) sm.s_ln[k] = n2;
             sm.s_lt[k] = sh.s_ptt[i] * nt + tj;
           }
           ln += __popcll(ml);
@@ -1028,7 +1109,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     const int* __restrict__ vb_count, int R) {
   __shared__ int s_pre[kMaxReplicas];
   __shared__ union {
-    QueryShare<P> q;
+    QueryShare<P, Q_MOVED> q;
     KTileSmem k;
   } sm;
   __shared__ CSpecSmem cs;
@@ -1063,7 +1144,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
       const int m0 = (q2 >> 1) * kCluster, on = q2 & 1;
       const int li = lane % kCluster, np = min(kCluster, nm - m0), pi = m0 + min(li, np - 1);
       const double4 pt = (on ? v.mv_new : v.mv_old)[pi];
-      const double2 eq = real_query_cluster<P, false>(g, v, pt, v.mv_type[pi], li < np, 0, lo, hi, part, L.qb, sm.q);
+      const double2 eq = real_query_cluster<P, Q_MOVED>(g, v, pt, v.mv_type[pi], li < np, 0, lo, hi, part, L.qb, sm.q);
       const double sgn = on ? 1.0 : -1.0;
       if (lane == 0) v.part_r[local * kQWaves + threadIdx.x / kWave] = make_double2(sgn * eq.x, sgn * eq.y);
     } else if ((b -= nqt) < rc.nkb_s * ne) {

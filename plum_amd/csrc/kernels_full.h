@@ -81,14 +81,14 @@ __global__ __launch_bounds__(kBlock) void k_cell_order(Geo g, Dev d) {
 // ============================================================ from scratch
 // Real space + LJ over all pairs: the cluster queries of the device loop with
 // the beads of a cell, kCluster slots at a time, as the points.  Every ordered
-// pair is visited, half of each counted (a bead's own images have weight 1/2
-// as it is), which costs half as many pair terms again as one thread per slot
+// pair is tested and a pair counted from its lower index (a bead's own images
+// with weight 1/2), which costs more distance tests than one thread per slot
 // that walks the cells around it, and none of its waits: 2.6 ms for 40,000
 // beads, and 8.5 ms for 3,200 beads in a box of 1.4 r_c, that way.
 // Block (cell, slot group, share of the query's cells).
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_full_real(Geo g, Dev d,
                                                                                               int nparts) {
-  __shared__ QueryShare<0> sm;
+  __shared__ QueryShare<0, Q_ALL> sm;
   const int cell = blockIdx.x, part = blockIdx.z, lane = threadIdx.x % kWave;
   const int cnt = d.ccount[cell];
   double elj = 0, ere = 0;
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     const size_t si = (size_t)cell * g.cap + min(s, cnt - 1);
     const int own = s < cnt ? d.cbead[si] : -1;
     if (!__ballot(own >= 0)) continue;
-    const double2 e = real_query_cluster<0, true>(g, d, d.cpos[si], d.ctype[si], own >= 0, own, 0, -1, part, nparts,
+    const double2 e = real_query_cluster<0, Q_ALL>(g, d, d.cpos[si], d.ctype[si], own >= 0, own, 0, -1, part, nparts,
                                                   sm);
     elj += e.x;
     ere += e.y;
@@ -105,7 +105,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
   }
   if (lane == 0) {
     const size_t b = ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
-    d.fpart[b * kQWaves + threadIdx.x / kWave] = make_double2(0.5 * elj, 0.5 * ere);
+    d.fpart[b * kQWaves + threadIdx.x / kWave] = make_double2(elj, ere);
   }
 }
 

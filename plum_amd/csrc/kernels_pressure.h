@@ -2,97 +2,74 @@
 // along z by kDz (ForceField::CalcPressureVolScalingHSELSlit,
 // pressure.cc:187-387).  Beads' z are scaled by 1 + kDz/Lz (with the spring
 // potential; grafted "L" beads stay, "R" beads move by kDz) or each molecule
-// is shifted by kDz com_z / Lz (without it).  The pair part runs over all
-// bead pairs once, new minus old per pair as the reference does, so the
-// difference keeps its precision; the k-space part is summed per k vector from
-// the change of S(k) and of c_k (k_vp_dsk).
+// is shifted by kDz com_z / Lz (without it).  The pair part is summed new minus
+// old per pair as the reference does, so the difference keeps its precision;
+// the k-space part is summed per k vector from the change of S(k) and of c_k
+// (k_vp_dsk).
 #pragma once
-#include "kernels_move.h"
+#include "kernels_full.h"
 
 namespace plum {
 
 constexpr double kDz = 0.00001;   // utilities/constants.h:55
-constexpr int kVpChunk = 512;     // beads per S(k) partial
 
-// Stretched z of every bead.  One thread per molecule: the centre of mass in
-// the reference's bead order, then the molecule's beads.
-__global__ void k_vp_scale(Geo g, Dev d, double* zs) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= g.n_mols) return;
-  const int a = d.mol_start[m], b = d.mol_start[m + 1];
-  const double Lz = g.Lsim[2];
-  double com = 0;
-  for (int j = a; j < b; j++) com += d.z[j];
-  com /= (b - a);
-  double dcz = kDz * (com / Lz);
-  const int k0 = d.wall[d.type[a]].kind;
-  if (k0 == 2) dcz = kDz;
-  else if (k0 == 1) dcz = 0;
-  for (int j = a; j < b; j++) {
-    const int kind = d.wall[d.type[j]].kind;
-    zs[j] = (g.use_bond && kind == 0) ? d.z[j] * (1.0 + kDz / Lz) : d.z[j] + dcz;
+// Stretched z of every bead (zs), its displacement (dz), and the displacement
+// of the image the cell list holds (dw).  A bead that moves with its molecule
+// sums the molecule's centre of mass itself, in the reference's bead order
+// (beads of the spring potential do not: the common case is one pass over the
+// beads).
+__global__ void k_vp_scale(Geo g, Dev d, double* zs, double* dz, double* dw) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= g.n) return;
+  const double Lz = g.Lsim[2], z = d.z[j];
+  double zn;
+  if (g.use_bond && d.wall[d.type[j]].kind == 0) {
+    zn = z * (1.0 + kDz / Lz);
+  } else {
+    const int m = d.mol_of[j], a = d.mol_start[m], b = d.mol_start[m + 1];
+    const int k0 = d.wall[d.type[a]].kind;
+    double dcz = k0 == 2 ? kDz : 0.0;
+    if (k0 == 0) {
+      double com = 0;
+      for (int i = a; i < b; i++) com += d.z[i];
+      com /= (b - a);
+      dcz = kDz * (com / Lz);
+    }
+    zn = z + dcz;
   }
+  // the displacement of the rounded z', exactly: z and z' are close
+  const double disp = zn - z;
+  zs[j] = zn;
+  dz[j] = disp;
+  dw[j] = disp - rint((z - wrap_coord(z, g.L[2], g.inv_L[2])) * g.inv_L[2]) * kDz;
 }
 
-// PotentialEwaldCoul::PairEnergyRealForP (potential_ewald_coul.cc:167-196):
-// the image sum in the box stretched along z, minimum image taken in that
-// box; the single-image shortcut where no other image can reach rc.
-__device__ inline double real_pair_stretch(const double* a, double qa, const double* b, double qb,
-                                           const Geo& g) {
-  if (qa * qb == 0) return 0.0;
-  const double Ls[3] = {g.L[0], g.L[1], g.L[2] + kDz};
-  const double inv_Ls[3] = {g.inv_L[0], g.inv_L[1], 1.0 / Ls[2]};
-  double d[3];
-  min_image_inv(a, b, Ls, inv_Ls, g.npbc, d);
-  const double pref = g.lB * qa * qb;
-  if (!one_image(d, Ls[2], g)) return pref * real_images(d, Ls, inv_Ls, g);
-  const double r = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
-  return (r > 0 && r <= g.rc) ? pref * erfc_nodes(g, g.sqrt_alpha * r) / r : 0.0;
-}
-
-// Unordered bead pairs a <= b (bead order is molecule order, so these are the
-// reference's (i, j) <= (k, l) pairs), grid-stride over the triangular index;
-// Ewald real-space and LJ new minus old per pair.  Pairs of phantom surface
-// sites count only from the first half of the site list (pressure.cc:271-272).
-__global__ __launch_bounds__(kBlock) void k_vp_pairs(Geo g, Dev d, const double* __restrict__ zs, int phantom,
-                                                     long long npair, double* part) {
-  __shared__ double sh[kBlock / kWave];
-  const int n = g.n;
-  const double Ls[3] = {g.Lsim[0], g.Lsim[1], g.Lsim[2] + kDz};
-  double del = 0, dlj = 0;
-  for (long long p = blockIdx.x * (long long)kBlock + threadIdx.x; p < npair; p += (long long)gridDim.x * kBlock) {
-    // row a holds the pairs (a, a..n-1): offset a n - a (a - 1) / 2
-    const double tn = 2.0 * n + 1;
-    long long a = (long long)floor((tn - sqrt(tn * tn - 8.0 * (double)p)) / 2);
-    if (a < 0) a = 0;
-    if (a > n - 1) a = n - 1;
-    while (a > 0 && a * n - a * (a - 1) / 2 > p) a--;
-    while (a < n - 1 && (a + 1) * n - (a + 1) * a / 2 <= p) a++;
-    const long long b = a + (p - (a * n - a * (a - 1) / 2));
-    const int ia = (int)a, ib = (int)b;
-    const int ma = d.mol_of[ia], mb = d.mol_of[ib];
-    if (!(ma >= phantom || (ma < phantom / 2 && mb >= phantom / 2))) continue;
-    const double ca[3] = {d.x[ia], d.y[ia], d.z[ia]}, cb[3] = {d.x[ib], d.y[ib], d.z[ib]};
-    const double ta[3] = {ca[0], ca[1], zs[ia]}, tb[3] = {cb[0], cb[1], zs[ib]};
-    if (g.use_ewald) {
-      const double qa = d.q[ia], qb = d.q[ib];
-      double o = real_pair(ca, qa, cb, qb, g), w = real_pair_stretch(ta, qa, tb, qb, g);
-      if (ia == ib) {
-        o *= 0.5;
-        w *= 0.5;
-      }
-      del += w - o;
-    }
-    if (g.use_pair && ma >= phantom && mb >= phantom && ia != ib) {
-      const LJPair lp = d.lj[d.type[ia] * g.n_types + d.type[ib]];
-      dlj += lj_energy(bb_dist(ta, tb, Ls, g.npbc), lp) - lj_energy(bb_dist(ca, cb, g.Lsim, g.npbc), lp);
-    }
+// Ewald real-space and LJ pairs, stretched minus current: the from-scratch
+// cluster queries (k_full_real) with both separations of each pair.  3,200
+// beads with r_c = 42 and L = 60: 143 us, and linear in N; over all N (N + 1) /
+// 2 bead pairs, the pair index decoded per pair and both image sums explicit,
+// 250 us (432 us with all 27 images), quadratic in N.
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_vp_pairs(
+    Geo g, Dev d, const double* __restrict__ dw, int phantom, int nparts, double2* part_out) {
+  __shared__ QueryShare<0, Q_STRETCH> sm;
+  const StretchArgs st = {dw, d.mol_of, kDz, phantom};
+  const int cell = blockIdx.x, part = blockIdx.z, lane = threadIdx.x % kWave;
+  const int cnt = d.ccount[cell];
+  double dlj = 0, del = 0;
+  for (int s0 = blockIdx.y * kCluster; s0 < cnt; s0 += gridDim.y * kCluster) {
+    const int s = s0 + lane % kCluster;
+    const size_t si = (size_t)cell * g.cap + min(s, cnt - 1);
+    const int own = s < cnt ? d.cbead[si] : -1;
+    if (!__ballot(own >= 0)) continue;
+    const double2 e = real_query_cluster<0, Q_STRETCH>(g, d, d.cpos[si], d.ctype[si], own >= 0, own, 0, -1, part,
+                                                       nparts, sm, st);
+    dlj += e.x;
+    del += e.y;
+    __syncthreads();   // the next group rewrites the points
   }
-  const double s1 = block_sum<kBlock>(del, sh);
-  const double s2 = block_sum<kBlock>(dlj, sh);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = s1;
-    part[2 * blockIdx.x + 1] = s2;
+  if (lane == 0) {
+    const size_t b = ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    part_out[b * kQWaves + threadIdx.x / kWave] = make_double2(dlj, del);
   }
 }
 
@@ -105,8 +82,21 @@ __global__ __launch_bounds__(kBlock) void k_vp_pairs(Geo g, Dev d, const double*
 // current box and the same image is used in the stretched box), so dE_k
 // keeps its precision instead of being a difference of two totals.
 // Bead chunk blockIdx.y.
+// `ncls` is 3 with surface sites, else 1.  The half phase change d/2 is at most
+// l pi kDz / L, so its sine and cosine are the first terms of their series
+// (below 1e-3 the next ones are under 1e-25) and a bead costs one sincos, not
+// three; chunks are short, as a chunk is a serial chain (512 beads a chunk:
+// 372 us for 3,200 beads on seven blocks).
+__device__ __forceinline__ void half_phase(double h, double& sn, double& cs) {
+  const double h2 = h * h;
+  sn = h * (1.0 + h2 * (-1.0 / 6.0 + h2 * (1.0 / 120.0 - h2 * (1.0 / 5040.0))));
+  cs = 1.0 + h2 * (-0.5 + h2 * (1.0 / 24.0 - h2 * (1.0 / 720.0)));
+}
+
+template <int NCLS>
 __global__ __launch_bounds__(kBlock) void k_vp_dsk(Geo g, Dev d, const int4* __restrict__ kl, int nk,
-                                                   const double* __restrict__ zs, int phantom, double2* part) {
+                                                   const double* __restrict__ zs, int phantom, int chunk,
+                                                   double2* part) {
   const int k = blockIdx.x * kBlock + threadIdx.x;
   if (k >= nk) return;
   const int4 l = kl[k];
@@ -115,34 +105,38 @@ __global__ __launch_bounds__(kBlock) void k_vp_dsk(Geo g, Dev d, const int4* __r
   const double kz = (double)(l.z * 2) * kPi / g.L[2];
   const double Ls = g.L[2] + kDz;
   const double kzs = (double)(l.z * 2) * kPi / Ls;
-  const int j0 = blockIdx.y * kVpChunk, j1 = min(g.n, j0 + kVpChunk);
-  double2 S[3] = {make_double2(0, 0), make_double2(0, 0), make_double2(0, 0)};
-  double2 D[3] = {make_double2(0, 0), make_double2(0, 0), make_double2(0, 0)};
+  const int j0 = blockIdx.y * chunk, j1 = min(g.n, j0 + chunk);
+  double2 S[NCLS], D[NCLS];
+#pragma unroll
+  for (int c = 0; c < NCLS; c++) S[c] = D[c] = make_double2(0, 0);
   for (int j = j0; j < j1; j++) {
     const double qj = d.q[j];
     if (qj == 0) continue;
-    const int m = d.mol_of[j];
-    const int c = m >= phantom ? 0 : (m < phantom / 2 ? 1 : 2);
+    const int cls = NCLS == 1 ? 0 : stretch_class(d.mol_of[j], phantom);
     const double xw = wrap_coord(d.x[j], g.L[0], g.inv_L[0]);
     const double yw = wrap_coord(d.y[j], g.L[1], g.inv_L[1]);
     const double nz = floor(d.z[j] * g.inv_L[2]);
     const double zw = d.z[j] - nz * g.L[2];
     const double zws = zs[j] - nz * Ls;
-    const double th = kx * xw + ky * yw + kz * zw;
-    const double dth = kzs * zws - kz * zw;
-    double sn, cs, sh, chh;
-    sincos(th, &sn, &cs);
-    sincos(th + 0.5 * dth, &sh, &chh);
-    const double s2 = 2.0 * sin(0.5 * dth);
-    S[c].x += qj * cs;
-    S[c].y += qj * sn;
+    double sn, cs, sh, ch;
+    sincos(kx * xw + ky * yw + kz * zw, &sn, &cs);
+    half_phase(0.5 * (kzs * zws - kz * zw), sh, ch);
     // 2 i sin(d/2) e^{i (th + d/2)}
-    D[c].x -= qj * s2 * sh;
-    D[c].y += qj * s2 * chh;
+    const double s2 = 2.0 * qj * sh;
+    const double dx = -s2 * (sn * ch + cs * sh), dy = s2 * (cs * ch - sn * sh);
+#pragma unroll
+    for (int c = 0; c < NCLS; c++)
+      if (c == cls) {
+        S[c].x += qj * cs;
+        S[c].y += qj * sn;
+        D[c].x += dx;
+        D[c].y += dy;
+      }
   }
-  for (int c = 0; c < 3; c++) {
-    part[((size_t)blockIdx.y * 6 + c) * nk + k] = S[c];
-    part[((size_t)blockIdx.y * 6 + 3 + c) * nk + k] = D[c];
+#pragma unroll
+  for (int c = 0; c < NCLS; c++) {
+    part[((size_t)blockIdx.y * 2 * NCLS + c) * nk + k] = S[c];
+    part[((size_t)blockIdx.y * 2 * NCLS + NCLS + c) * nk + k] = D[c];
   }
 }
 
@@ -152,6 +146,7 @@ __device__ __forceinline__ double re_conj(double2 a, double2 b) { return a.x * b
 // Q(S) = |S_M|^2 + 2 Re(S_A* S_B) + 2 Re(S_A* S_M) (the included pairs),
 // written as dc Q(S) + c' (Q(S + dS) - Q(S)) where l is in both lists
 // (dc = c' - c, evaluated on the host without cancellation); block partials.
+template <int NCLS>
 __global__ __launch_bounds__(kBlock) void k_vp_dsk_energy(const double2* __restrict__ part, int nchunk, int nk,
                                                           const double* __restrict__ c_old,
                                                           const double* __restrict__ c_new,
@@ -162,10 +157,12 @@ __global__ __launch_bounds__(kBlock) void k_vp_dsk_energy(const double2* __restr
   if (k < nk) {
     double2 S[3] = {make_double2(0, 0), make_double2(0, 0), make_double2(0, 0)};
     double2 D[3] = {make_double2(0, 0), make_double2(0, 0), make_double2(0, 0)};
+#pragma unroll 8
     for (int ch = 0; ch < nchunk; ch++)
-      for (int c = 0; c < 3; c++) {
-        const double2 v = part[((size_t)ch * 6 + c) * nk + k];
-        const double2 w = part[((size_t)ch * 6 + 3 + c) * nk + k];
+#pragma unroll
+      for (int c = 0; c < NCLS; c++) {
+        const double2 v = part[((size_t)ch * 2 * NCLS + c) * nk + k];
+        const double2 w = part[((size_t)ch * 2 * NCLS + NCLS + c) * nk + k];
         S[c].x += v.x;
         S[c].y += v.y;
         D[c].x += w.x;
@@ -184,55 +181,65 @@ __global__ __launch_bounds__(kBlock) void k_vp_dsk_energy(const double2* __restr
   if (threadIdx.x == 0) epart[blockIdx.x] = r;
 }
 
-// Walls (mobile beads), springs and the slab dipole, then every partial into
-// out[0..5] = Ewald pairs, LJ pairs, walls, springs, dipole, k space.
-__global__ __launch_bounds__(kBlock) void k_vp_small(Geo g, Dev d, const double* __restrict__ zs, int phantom,
-                                                     const double* __restrict__ ppart, int npb,
-                                                     const double* __restrict__ ekpart, int nkb, double* out) {
+// Walls (mobile beads), springs (each bond's change) and the dipole moments
+// before and after: block partials part[4 b ..].
+__global__ __launch_bounds__(kBlock) void k_vp_small(Geo g, Dev d, const double* __restrict__ zs,
+                                                     const double* __restrict__ disp, int phantom, double* part) {
   __shared__ double sh[kBlock / kWave];
   Geo gs = g;
   gs.Lsim[2] = g.Lsim[2] + kDz;
   double ew = 0, eb = 0, mo = 0, mn = 0;
-  for (int j = threadIdx.x; j < g.n; j += kBlock) {
-    if (g.use_ext && d.mol_of[j] >= phantom) {
+  for (int j = blockIdx.x * kBlock + threadIdx.x; j < g.n; j += gridDim.x * kBlock) {
+    const int m = d.mol_of[j];
+    if (g.use_ext && m >= phantom) {
       const WallType w = d.wall[d.type[j]];
       ew += wall_energy(zs[j], w, gs) - wall_energy(d.z[j], w, g);
     }
     mo += d.q[j] * d.z[j];
     mn += d.q[j] * zs[j];
-  }
-  if (g.use_bond) {
-    for (int m = threadIdx.x; m < g.n_mols; m += kBlock) {
-      const int a = d.mol_start[m], b = d.mol_start[m + 1];
-      double e = 0;
-      for (int i = a; i < b - 1; i++) {
-        const double dx = d.x[i] - d.x[i + 1], dy = d.y[i] - d.y[i + 1], dz = zs[i] - zs[i + 1];
-        const double r = sqrt(dx * dx + dy * dy + dz * dz);
-        e += 0.5 * g.k_bond * (r - g.r0) * (r - g.r0);
-      }
-      eb += e - d.bond_cur[m];
+    if (g.use_bond && j + 1 < d.mol_start[m + 1]) {
+      const double dx = d.x[j] - d.x[j + 1], dy = d.y[j] - d.y[j + 1], dz = d.z[j] - d.z[j + 1];
+      eb += spring_energy(g, dx, dy, dz + (disp[j] - disp[j + 1])) - spring_energy(g, dx, dy, dz);
     }
   }
-  double pe = 0, pl = 0, kk = 0;
-  for (int b = threadIdx.x; b < npb; b += kBlock) {
-    pe += ppart[2 * b];
-    pl += ppart[2 * b + 1];
+  const double v4[4] = {ew, eb, mo, mn};
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const double t = block_sum<kBlock>(v4[k], sh);
+    if (threadIdx.x == 0) part[4 * blockIdx.x + k] = t;
   }
-  for (int b = threadIdx.x; b < nkb; b += kBlock) kk += ekpart[b];
-  const double t_ew = block_sum<kBlock>(ew, sh);
-  const double t_eb = block_sum<kBlock>(eb, sh);
-  const double t_mo = block_sum<kBlock>(mo, sh);
-  const double t_mn = block_sum<kBlock>(mn, sh);
-  const double t_pe = block_sum<kBlock>(pe, sh);
-  const double t_pl = block_sum<kBlock>(pl, sh);
-  const double t_kk = block_sum<kBlock>(kk, sh);
+}
+
+// Every partial into out[0..5] = Ewald pairs, LJ pairs, walls, springs,
+// dipole, k space.
+__global__ __launch_bounds__(kFinalThreads) void k_vp_final(Geo g, const double2* __restrict__ ppart, int npp,
+                                                            const double* __restrict__ ekpart, int nkb,
+                                                            const double* __restrict__ opart, int nob, double* out) {
+  __shared__ double sh[kFinalThreads / kWave];
+  double pe = 0, pl = 0, kk = 0, vo[4] = {0, 0, 0, 0};
+#pragma unroll 4
+  for (int b = threadIdx.x; b < npp; b += kFinalThreads) {
+    pl += ppart[b].x;
+    pe += ppart[b].y;
+  }
+  for (int b = threadIdx.x; b < nkb; b += kFinalThreads) kk += ekpart[b];
+  for (int b = threadIdx.x; b < nob; b += kFinalThreads)
+#pragma unroll
+    for (int k = 0; k < 4; k++) vo[k] += opart[4 * b + k];
+  const double t_ew = block_sum<kFinalThreads>(vo[0], sh);
+  const double t_eb = block_sum<kFinalThreads>(vo[1], sh);
+  const double t_mo = block_sum<kFinalThreads>(vo[2], sh);
+  const double t_mn = block_sum<kFinalThreads>(vo[3], sh);
+  const double t_pe = block_sum<kFinalThreads>(pe, sh);
+  const double t_pl = block_sum<kFinalThreads>(pl, sh);
+  const double t_kk = block_sum<kFinalThreads>(kk, sh);
   if (threadIdx.x == 0) {
     double dip = 0;
     if (g.use_ewald && g.dipole) {
       const double* L = g.Lsim;
       dip = (g.lB * 2 * kPi) * (t_mn * t_mn / (L[0] * L[1] * (L[2] + kDz)) - t_mo * t_mo / (L[0] * L[1] * L[2]));
     }
-    out[0] = t_pe;
+    out[0] = g.use_ewald ? t_pe : 0.0;
     out[1] = g.use_pair ? t_pl : 0.0;
     out[2] = g.use_ext ? t_ew : 0.0;
     out[3] = g.use_bond ? t_eb : 0.0;

@@ -2,15 +2,18 @@
 // of the pressure estimator.  Included once, at the end of engine.hip.
 
 struct VpHost {
-  double* zs = nullptr;       // stretched z per bead
-  double* ppart = nullptr;    // pair partials (Ewald, LJ) per block
+  // stretched z per bead, its displacement, that of the image in the cell list
+  double *zs = nullptr, *dz = nullptr, *dw = nullptr;
+  double2* ppart = nullptr;   // pair partials (LJ, Ewald) per wave
+  size_t pcap = 0;            // their number allocated
+  double* opart = nullptr;    // walls, springs, dipole partials
   int4* kl_u = nullptr;       // half-space l vectors in the current or the stretched k list
   double *c_old = nullptr, *c_new = nullptr, *dc = nullptr;   // c_k of each box (0: not in its list), c' - c
   int nk_u = 0;
   double2* skpart = nullptr;  // S(k) and dS(k) partials [chunk][6][k]
   double *ekpart = nullptr, *out = nullptr;
   double* h_out = nullptr;    // pinned
-  int npb = 0, nchunk = 0, nkb = 0;
+  int nchunk = 0, chunk = 0, nkb = 0;
 };
 
 void vp_free(VpHost* h) {
@@ -72,14 +75,17 @@ int vp_setup(plum_ctx* c) {
         }
   }
   h->nk_u = (int)kl.size();
-  const long long n = g.n;
-  const long long npair = n * (n + 1) / 2;
-  h->npb = (int)std::max(1LL, std::min(8192LL, (npair + kBlock - 1) / kBlock));
-  h->nchunk = (g.n + kVpChunk - 1) / kVpChunk;
   const int nk = std::max(h->nk_u, 1);
   h->nkb = (nk + kBlock - 1) / kBlock;
+  // bead chunks of the S(k) sums: two blocks per CU over the k blocks, at most
+  // 64 chunks (their sum is a serial chain too), at least 16 beads
+  const int want = std::max(1, std::min(64, 512 / h->nkb));
+  h->chunk = std::max(16, (g.n + want - 1) / want);
+  h->nchunk = (g.n + h->chunk - 1) / h->chunk;
   CHK(dalloc(c, &h->zs, (size_t)g.n));
-  CHK(dalloc(c, &h->ppart, 2 * (size_t)h->npb));
+  CHK(dalloc(c, &h->dz, (size_t)g.n));
+  CHK(dalloc(c, &h->dw, (size_t)g.n));
+  CHK(dalloc(c, &h->opart, 4 * (size_t)kFullSmall));
   CHK(dalloc(c, &h->kl_u, (size_t)nk));
   CHK(dalloc(c, &h->c_old, (size_t)nk));
   CHK(dalloc(c, &h->c_new, (size_t)nk));
@@ -115,20 +121,34 @@ extern "C" int plum_vp_sample(plum_ctx* c, int phantom, plum_vp* out) {
   }
   VpHost* h = c->vp;
   const Geo& g = c->g;
-  hipLaunchKernelGGL(k_vp_scale, dim3((g.n_mols + kBlock - 1) / kBlock), dim3(kBlock), 0, c->st, g, c->d, h->zs);
-  const long long n = g.n;
-  hipLaunchKernelGGL(k_vp_pairs, dim3(h->npb), dim3(kBlock), 0, c->st, g, c->d, h->zs, phantom, n * (n + 1) / 2,
-                     h->ppart);
+  const size_t np = (size_t)g.ncell * c->full_groups * c->full_parts * kQWaves;
+  if (np > h->pcap) {
+    CHK(dalloc(c, &h->ppart, np));
+    h->pcap = np;
+  }
+  hipLaunchKernelGGL(k_vp_scale, dim3((g.n + kBlock - 1) / kBlock), dim3(kBlock), 0, c->st, g, c->d, h->zs,
+                     h->dz, h->dw);
+  hipLaunchKernelGGL(k_vp_pairs, dim3(g.ncell, c->full_groups, c->full_parts), dim3(kBlock), 0, c->st, g, c->d, h->dw,
+                     phantom, c->full_parts, h->ppart);
   int nkb = 0;
   if (g.use_ewald && h->nk_u > 0) {
-    hipLaunchKernelGGL(k_vp_dsk, dim3((h->nk_u + kBlock - 1) / kBlock, h->nchunk), dim3(kBlock), 0, c->st, g, c->d,
-                       h->kl_u, h->nk_u, h->zs, phantom, h->skpart);
-    hipLaunchKernelGGL(k_vp_dsk_energy, dim3(h->nkb), dim3(kBlock), 0, c->st, h->skpart, h->nchunk, h->nk_u,
-                       h->c_old, h->c_new, h->dc, h->ekpart);
     nkb = h->nkb;
+    if (phantom > 0) {
+      hipLaunchKernelGGL(k_vp_dsk<3>, dim3(nkb, h->nchunk), dim3(kBlock), 0, c->st, g, c->d, h->kl_u, h->nk_u, h->zs,
+                         phantom, h->chunk, h->skpart);
+      hipLaunchKernelGGL(k_vp_dsk_energy<3>, dim3(nkb), dim3(kBlock), 0, c->st, h->skpart, h->nchunk, h->nk_u,
+                         h->c_old, h->c_new, h->dc, h->ekpart);
+    } else {
+      hipLaunchKernelGGL(k_vp_dsk<1>, dim3(nkb, h->nchunk), dim3(kBlock), 0, c->st, g, c->d, h->kl_u, h->nk_u, h->zs,
+                         phantom, h->chunk, h->skpart);
+      hipLaunchKernelGGL(k_vp_dsk_energy<1>, dim3(nkb), dim3(kBlock), 0, c->st, h->skpart, h->nchunk, h->nk_u,
+                         h->c_old, h->c_new, h->dc, h->ekpart);
+    }
   }
-  hipLaunchKernelGGL(k_vp_small, dim3(1), dim3(kBlock), 0, c->st, g, c->d, h->zs, phantom, h->ppart, h->npb,
-                     h->ekpart, nkb, h->out);
+  hipLaunchKernelGGL(k_vp_small, dim3(kFullSmall), dim3(kBlock), 0, c->st, g, c->d, h->zs, h->dz, phantom,
+                     h->opart);
+  hipLaunchKernelGGL(k_vp_final, dim3(1), dim3(kFinalThreads), 0, c->st, g, h->ppart, (int)np, h->ekpart, nkb,
+                     h->opart, kFullSmall, h->out);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(h->h_out, h->out, 6 * sizeof(double), hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));

@@ -129,3 +129,23 @@ def test_spring_energy_has_one_set_of_bits():
         _, d = eng.delta(mol, idx, xyz[idx])
         eng.finalize(False)
         assert d["bond"] == 0.0
+
+
+@pytest.mark.parametrize("n_chains,chain_len,L,alpha", [(1, 2, 9.0, 0.2), (3, 7, 7.0, 0.06), (5, 11, 13.0, 0.5)])
+def test_volume_perturbation_sizes(n_chains, chain_len, L, alpha):
+    """The pressure sample by cluster queries and short bead chunks, from four
+    beads up, with up to two image shells, the chains outside the box so that
+    the listed images differ from the coordinates.  Bound of
+    test_gpu_pressure.py (1e-14 of the summed energies), ten times wider: the
+    oracle's stretched coordinates, up to 3.3 edges, round that much more."""
+    sd = systems.config("tiny")
+    xyz, q, ty, ms = systems.build_bulk(n_chains, chain_len, n_chains * chain_len, L, 31)
+    xyz = xyz + np.array([0.0, 0.0, 2.3 * L])      # wrapped images differ from the coordinates
+    sd.update(xyz=xyz, q=q, type=ty, mol_start=ms, box=[L, L, L], alpha=alpha)
+    eng = E.Engine(sd)
+    got = eng.vp_sample()
+    orc = O.Oracle(sd)
+    ref = orc.vp_sample(0)
+    scale = sum(abs(v) for v in orc.energy_full().values())
+    for k in ("el", "lj", "bond", "dU"):
+        assert abs(got[k] - ref[k]) <= 1e-13 * scale, (k, got[k], ref[k], scale)

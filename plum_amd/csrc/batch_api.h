@@ -67,7 +67,8 @@ struct SurHost {
   float *D3 = nullptr, *D2 = nullptr, *D1 = nullptr;
   double *T = nullptr, *loss = nullptr;
   int* N = nullptr;
-  float* part = nullptr;  // chunk partials of the weight gradients
+  float* part = nullptr;  // chunk partials of the gradient
+  double* loss_s = nullptr;  // squared error of each sample
   int step = 0;
   long long train_steps = 0;
   double last_loss = 0;

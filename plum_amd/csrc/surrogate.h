@@ -503,101 +503,266 @@ __global__ __launch_bounds__(kBlock) void k_mlp_spec(const NetBF16* __restrict__
 }
 
 // ------------------------------------------------------------ training (FP32)
-// C[M x N] = act(A[M x K] B[K x N] + bias), act 0 = identity, 1 = tanh.
-__global__ void k_gemm_ab(const float* __restrict__ A, const float* __restrict__ B, const float* __restrict__ bias,
-                          float* __restrict__ Cm, int M, int N, int K, int act) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= M * N) return;
-  const int i = idx / N, j = idx - (idx / N) * N;
-  float s = bias ? bias[j] : 0.f;
-  for (int k = 0; k < K; k++) s += A[(size_t)i * K + k] * B[(size_t)k * N + j];
-  Cm[idx] = act ? tanhf(s) : s;
-}
+// FP32 products and sums on v_mfma_f32_16x16x4f32: lane l supplies A[l % 16][l
+// / 16] and B[l / 16][l % 16] and receives D[4 (l / 16) + i][l % 16].  A layer
+// is kHid wide, so a block holds all of its weights in LDS and takes kLinRows
+// rows, a wave 16 of them by all columns; the weights are read once per block.
+// LDS rows are padded so that the 64 lanes of an operand read fall in
+// different banks (16 rows 4 banks apart, or 4 rows 16 banks apart).  One
+// thread per output over global memory took 430 us for a backward product of
+// 12,800 rows (each lane walking its own weight row), 1.8 ms for a whole loss
+// and gradient; the launches are now 8 instead of 18.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kLinRows = 64;
+constexpr int kPadK = 4;    // rows read along the inner index
+constexpr int kPadN = 16;   // rows read across
 
-// C[M x N] = (A[M x K] B^T) * (1 - H^2), B given as [N x K]... here B is the
-// weight W[N x K] (rows = layer input), so C = A W^T elementwise times the
-// tanh derivative of H[M x N].
-__global__ void k_gemm_abt_dtanh(const float* __restrict__ A, const float* __restrict__ W,
-                                 const float* __restrict__ H, float* __restrict__ Cm, int M, int N, int K) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= M * N) return;
-  const int i = idx / N, j = idx - (idx / N) * N;
-  float s = 0.f;
-  for (int k = 0; k < K; k++) s += A[(size_t)i * K + k] * W[(size_t)j * K + k];
-  const float h = H[idx];
-  Cm[idx] = s * (1.f - h * h);
-}
-
-// G[K1 x K2] = A^T B for A[M x K1], B[M x K2] (weight gradients) in two
-// passes: k_gemm_atb_part sums rows [c R, (c + 1) R) of chunk c into
-// part[c][K1 x K2 (+ K2 column sums of B)], k_gemm_atb_sum adds the chunks in
-// order.
-constexpr int kAtbRows = 128;
-
-__global__ void k_gemm_atb_part(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ part,
-                                int M, int K1, int K2) {
-  const int c = blockIdx.y;
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  const int nout = K1 * K2 + K2;
-  if (idx >= nout) return;
-  const int m0 = c * kAtbRows, m1 = min(M, m0 + kAtbRows);
-  float s = 0.f;
-  if (idx < K1 * K2) {
-    const int i = idx / K2, j = idx - (idx / K2) * K2;
-    for (int m = m0; m < m1; m++) s += A[(size_t)m * K1 + i] * B[(size_t)m * K2 + j];
-  } else {
-    const int j = idx - K1 * K2;
-    for (int m = m0; m < m1; m++) s += B[(size_t)m * K2 + j];
+// `n` floats in rows of `width`, from memory to LDS rows `ld` apart, 16 bytes
+// a load; rows past `rows` are zero.
+template <int WIDTH>
+__device__ __forceinline__ void stage_rows(const float* __restrict__ src, float* dst, int ld, int rows, int total) {
+  const float4* g4 = reinterpret_cast<const float4*>(src);
+  for (int c = threadIdx.x; c < total * (WIDTH / 4); c += kBlock) {
+    const int r = c / (WIDTH / 4), q = c % (WIDTH / 4);
+    const float4 v = r < rows ? g4[c] : make_float4(0.f, 0.f, 0.f, 0.f);
+    *reinterpret_cast<float4*>(dst + r * ld + 4 * q) = v;
   }
-  part[(size_t)c * nout + idx] = s;
 }
 
-__global__ void k_gemm_atb_sum(const float* __restrict__ part, int chunks, int K1, int K2, float* __restrict__ Gm,
-                               float* __restrict__ bias_g) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  const int nout = K1 * K2 + K2;
-  if (idx >= nout) return;
-  float s = 0.f;
-  for (int c = 0; c < chunks; c++) s += part[(size_t)c * nout + idx];
-  if (idx < K1 * K2) Gm[idx] = s;
-  else if (bias_g) bias_g[idx - K1 * K2] = s;
-}
-
-// Minibatch loss: sample i owns rows [i R, (i + 1) R) of f (R = 2 maxm: old
-// beads then new beads, n_i of each in use).  pred_i = sum(new) - sum(old);
-// loss = mean (pred_i - clip(target_i))^2; g[row] = dloss/df(row).
-__global__ void k_train_loss(const float* __restrict__ f, const double* __restrict__ target,
-                             const int* __restrict__ n, int samples, int maxm, double clip, float* __restrict__ g,
-                             double* __restrict__ loss_out) {
-  __shared__ double sh[kBlock / kWave];
-  double l = 0;
-  for (int i = threadIdx.x; i < samples; i += kBlock) {
-    const float* fo = f + (size_t)i * 2 * maxm;
-    const float* fn = fo + maxm;
-    double pred = 0;
-    for (int m = 0; m < n[i]; m++) pred += (double)fn[m] - (double)fo[m];
-    const double tgt = fmin(fmax(target[i], -clip), clip);
-    const double res = pred - tgt;
-    l += res * res;
-    const float gr = (float)(2.0 * res / samples);
-    float* go = g + (size_t)i * 2 * maxm;
-    for (int m = 0; m < maxm; m++) {
-      go[m] = m < n[i] ? -gr : 0.f;
-      go[maxm + m] = m < n[i] ? gr : 0.f;
+// H[M x kHid] = tanh(A[M x K] W + bias), W[K x kHid]; with w4 also the network
+// output F = H w4 + b4 per row.
+template <int K>
+__global__ __launch_bounds__(kBlock) void k_lin_fwd(const float* __restrict__ A, const float* __restrict__ W,
+                                                    const float* __restrict__ bias, float* __restrict__ H, int M,
+                                                    const float* __restrict__ w4, const float* __restrict__ b4,
+                                                    float* __restrict__ F) {
+  __shared__ __align__(16) float s_a[kLinRows * (K + kPadK)];
+  __shared__ __align__(16) float s_w[K * (kHid + kPadN)];
+  const int m0 = blockIdx.x * kLinRows;
+  stage_rows<K>(A + (size_t)m0 * K, s_a, K + kPadK, M - m0, kLinRows);
+  stage_rows<kHid>(W, s_w, kHid + kPadN, K, K);
+  __syncthreads();
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave, col = lane % 16, sub = lane / 16;
+  constexpr int NT = kHid / 16;
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const float* a = s_a + (16 * w + col) * (K + kPadK) + sub;
+  const float* b = s_w + sub * (kHid + kPadN) + col;
+#pragma unroll 4
+  for (int k = 0; k < K; k += 4) {
+    const float av = a[k];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+      acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b[k * (kHid + kPadN) + 16 * t], acc[t], 0, 0, 0);
+  }
+  float f[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < NT; t++) {
+    const int c = 16 * t + col;
+    const float bc = bias[c], wc = w4 ? w4[c] : 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int m = m0 + 16 * w + 4 * sub + i;
+      const float h = tanhf(acc[t][i] + bc);
+      if (m < M) H[(size_t)m * kHid + c] = h;
+      f[i] += h * wc;
     }
   }
-  const double t = block_sum<kBlock>(l, sh);
-  if (threadIdx.x == 0) *loss_out = t / samples;
+  if (!w4) return;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) f[i] += __shfl_xor(f[i], o, kWave);
+    const int m = m0 + 16 * w + 4 * sub + i;
+    if (col == 0 && m < M) F[m] = f[i] + *b4;
+  }
 }
 
-// delta3[M x 128] = g[m] w4 (1 - H3^2).
-__global__ void k_out_delta(const float* __restrict__ g, const float* __restrict__ w4, const float* __restrict__ H3,
-                            float* __restrict__ d3, int M) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= M * kHid) return;
-  const int m = idx / kHid, j = idx - (idx / kHid) * kHid;
-  const float h = H3[idx];
-  d3[idx] = g[m] * w4[j] * (1.f - h * h);
+// C[M x kHid] = (D W^T) (1 - H^2), W[kHid x kHid] (rows = layer input).  With
+// g the layer above is the output: D = g w4 (1 - Ht^2) from its activations
+// Ht, written to D too (the weight gradient reads it).
+__global__ __launch_bounds__(kBlock) void k_lin_bwd(float* __restrict__ D, const float* __restrict__ W,
+                                                    const float* __restrict__ H, float* __restrict__ C, int M,
+                                                    const float* __restrict__ g, const float* __restrict__ w4,
+                                                    const float* __restrict__ Ht) {
+  constexpr int LD = kHid + kPadK;
+  __shared__ __align__(16) float s_a[kLinRows * LD];
+  __shared__ __align__(16) float s_w[kHid * LD];
+  const int m0 = blockIdx.x * kLinRows;
+  if (g) {
+    for (int c = threadIdx.x; c < kLinRows * kHid; c += kBlock) {
+      const int r = c / kHid, k = c % kHid, m = m0 + r;
+      float v = 0.f;
+      if (m < M) {
+        const float h = Ht[(size_t)m * kHid + k];
+        v = g[m] * w4[k] * (1.f - h * h);
+        D[(size_t)m * kHid + k] = v;
+      }
+      s_a[r * LD + k] = v;
+    }
+  } else {
+    stage_rows<kHid>(D + (size_t)m0 * kHid, s_a, LD, M - m0, kLinRows);
+  }
+  stage_rows<kHid>(W, s_w, LD, kHid, kHid);
+  __syncthreads();
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave, col = lane % 16, sub = lane / 16;
+  constexpr int NT = kHid / 16;
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const float* a = s_a + (16 * w + col) * LD + sub;
+  const float* b = s_w + col * LD + sub;
+#pragma unroll 4
+  for (int k = 0; k < kHid; k += 4) {
+    const float av = a[k];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+      acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b[16 * t * LD + k], acc[t], 0, 0, 0);
+  }
+#pragma unroll
+  for (int t = 0; t < NT; t++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int m = m0 + 16 * w + 4 * sub + i;
+      if (m < M) {
+        const float h = H[(size_t)m * kHid + 16 * t + col];
+        C[(size_t)m * kHid + 16 * t + col] = acc[t][i] * (1.f - h * h);
+      }
+    }
+}
+
+// Weight gradients A^T B and bias gradients (column sums of B) of every layer
+// over rows [c kAtbRows, (c + 1) kAtbRows) of chunk c = blockIdx.x, layer
+// blockIdx.y, into part[c] laid out as the parameters; k_grad_sum adds the
+// chunks.
+constexpr int kAtbRows = 128, kAtbStage = 32;
+
+template <int K1>
+__device__ void atb_chunk(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ gw,
+                          float* __restrict__ gb, int rows, float* s_a, float* s_b) {
+  constexpr int LA = K1 + kPadN, LB = kHid + kPadN, IT = K1 / 64, NT = kHid / 16;
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave, col = lane % 16, sub = lane / 16;
+  f32x4 acc[IT][NT];
+#pragma unroll
+  for (int u = 0; u < IT; u++)
+#pragma unroll
+    for (int t = 0; t < NT; t++) acc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float bs = 0.f;
+  for (int r0 = 0; r0 < rows; r0 += kAtbStage) {
+    __syncthreads();
+    stage_rows<K1>(A + (size_t)r0 * K1, s_a, LA, rows - r0, kAtbStage);
+    stage_rows<kHid>(B + (size_t)r0 * kHid, s_b, LB, rows - r0, kAtbStage);
+    __syncthreads();
+#pragma unroll 2
+    for (int k = 0; k < kAtbStage; k += 4) {
+      float av[IT];
+#pragma unroll
+      for (int u = 0; u < IT; u++) av[u] = s_a[(k + sub) * LA + (w * IT + u) * 16 + col];
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        const float bv = s_b[(k + sub) * LB + 16 * t + col];
+#pragma unroll
+        for (int u = 0; u < IT; u++) acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u], bv, acc[u][t], 0, 0, 0);
+      }
+    }
+    if (threadIdx.x < kHid)
+      for (int k = 0; k < kAtbStage; k++) bs += s_b[k * LB + threadIdx.x];
+  }
+#pragma unroll
+  for (int u = 0; u < IT; u++)
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) gw[((w * IT + u) * 16 + 4 * sub + i) * kHid + 16 * t + col] = acc[u][t][i];
+  if (threadIdx.x < kHid) gb[threadIdx.x] = bs;
+}
+
+__global__ __launch_bounds__(kBlock) void k_grad_part(const float* __restrict__ X, const float* __restrict__ H1,
+                                                      const float* __restrict__ H2, const float* __restrict__ H3,
+                                                      const float* __restrict__ D1, const float* __restrict__ D2,
+                                                      const float* __restrict__ D3, const float* __restrict__ G, int M,
+                                                      float* __restrict__ part) {
+  __shared__ __align__(16) float s_a[kAtbStage * (kHid + kPadN)];
+  __shared__ __align__(16) float s_b[kAtbStage * (kHid + kPadN)];
+  const int m0 = blockIdx.x * kAtbRows, rows = min(kAtbRows, M - m0);
+  float* p = part + (size_t)blockIdx.x * kNParams;
+  const size_t h0 = (size_t)m0 * kHid;
+  if (blockIdx.y == 0) {
+    atb_chunk<kDescr>(X + (size_t)m0 * kDescr, D1 + h0, p + kOffW1, p + kOffB1, rows, s_a, s_b);
+  } else if (blockIdx.y == 1) {
+    atb_chunk<kHid>(H1 + h0, D2 + h0, p + kOffW2, p + kOffB2, rows, s_a, s_b);
+  } else if (blockIdx.y == 2) {
+    atb_chunk<kHid>(H2 + h0, D3 + h0, p + kOffW3, p + kOffB3, rows, s_a, s_b);
+  } else {
+    // output row: H3^T g and the sum of g, two halves of the rows
+    const int j = threadIdx.x % kHid, half = threadIdx.x / kHid;
+    float s = 0.f, b = 0.f;
+    for (int m = half; m < rows; m += 2) {
+      const float gm = G[m0 + m];
+      s += H3[h0 + (size_t)m * kHid + j] * gm;
+      b += gm;
+    }
+    if (half) s_a[j] = s, s_b[j] = b;
+    __syncthreads();
+    if (!half) {
+      p[kOffW4 + j] = s + s_a[j];
+      if (j == 0) p[kOffB4] = b + s_b[0];
+    }
+  }
+}
+static_assert(kBlock == 2 * kHid, "two halves of the rows");
+
+// grad = sum of the chunks' partials (four interleaved groups of chunks, then
+// the groups), kWave parameters per block; block 0 also sums the samples'
+// losses.
+__global__ __launch_bounds__(kBlock) void k_grad_sum(const float* __restrict__ part, int chunks,
+                                                     float* __restrict__ grad, const double* __restrict__ loss_s,
+                                                     int samples, double* __restrict__ loss) {
+  __shared__ float s_g[kBlock / kWave][kWave];
+  __shared__ double sh[kBlock / kWave];
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+  const int p = blockIdx.x * kWave + lane;
+  float s = 0.f;
+  if (p < kNParams) {
+#pragma unroll 8
+    for (int c = w; c < chunks; c += kBlock / kWave) s += part[(size_t)c * kNParams + p];
+  }
+  s_g[w][lane] = s;
+  __syncthreads();
+  if (w == 0 && p < kNParams) grad[p] = (s_g[0][lane] + s_g[1][lane]) + (s_g[2][lane] + s_g[3][lane]);
+  if (blockIdx.x == 0) {
+    double l = 0;
+    for (int i = threadIdx.x; i < samples; i += kBlock) l += loss_s[i];
+    const double t = block_sum<kBlock>(l, sh);
+    if (threadIdx.x == 0) *loss = t / samples;
+  }
+}
+
+// Minibatch loss, one wave per sample: sample i owns rows [i R, (i + 1) R) of
+// f (R = 2 maxm: old beads then new beads, n_i of each in use).  pred_i =
+// sum(new) - sum(old); loss = mean (pred_i - clip(target_i))^2 (the squares
+// summed by k_grad_sum); g[row] = dloss/df(row).
+__global__ __launch_bounds__(kBlock) void k_train_loss(const float* __restrict__ f, const double* __restrict__ target,
+                                                       const int* __restrict__ n, int samples, int maxm, double clip,
+                                                       float* __restrict__ g, double* __restrict__ loss_s) {
+  const int i = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  if (i >= samples) return;
+  const float* fo = f + (size_t)i * 2 * maxm;
+  const float* fn = fo + maxm;
+  const int ni = n[i];
+  double pred = 0;
+  for (int m = lane; m < ni; m += kWave) pred += (double)fn[m] - (double)fo[m];
+  pred = __shfl(wave_sum(pred), 0, kWave);
+  const double tgt = fmin(fmax(target[i], -clip), clip);
+  const double res = pred - tgt;
+  if (lane == 0) loss_s[i] = res * res;
+  const float gr = (float)(2.0 * res / samples);
+  float* go = g + (size_t)i * 2 * maxm;
+  for (int m = lane; m < maxm; m += kWave) {
+    go[m] = m < ni ? -gr : 0.f;
+    go[maxm + m] = m < ni ? gr : 0.f;
+  }
 }
 
 // Adam (Kingma & Ba 2015) on the FP32 master copy, then the BF16 inference

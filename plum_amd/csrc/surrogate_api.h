@@ -32,7 +32,8 @@ int sur_workspace(plum_ctx* c, int samples) {
   CHK(salloc(s, &s->G, M));
   CHK(salloc(s, &s->T, samples));
   CHK(salloc(s, &s->N, samples));
-  CHK(salloc(s, &s->part, ((M + kAtbRows - 1) / kAtbRows) * (size_t)(kHid * kHid + kHid)));
+  CHK(salloc(s, &s->loss_s, samples));
+  CHK(salloc(s, &s->part, ((M + kAtbRows - 1) / kAtbRows) * (size_t)kNParams));
   s->tb_cap = samples;
   return PLUM_OK;
 }
@@ -42,23 +43,13 @@ void sur_forward32(plum_ctx* c, hipStream_t st, size_t M) {
   SurHost* s = c->sur;
   const float* w = s->w32;
   const int m = (int)M;
-  hipLaunchKernelGGL(k_gemm_ab, dim3(nblocks(M * kHid)), dim3(kBlock), 0, st, s->X, w + kOffW1, w + kOffB1, s->H1, m,
-                     kHid, kDescr, 1);
-  hipLaunchKernelGGL(k_gemm_ab, dim3(nblocks(M * kHid)), dim3(kBlock), 0, st, s->H1, w + kOffW2, w + kOffB2, s->H2,
-                     m, kHid, kHid, 1);
-  hipLaunchKernelGGL(k_gemm_ab, dim3(nblocks(M * kHid)), dim3(kBlock), 0, st, s->H2, w + kOffW3, w + kOffB3, s->H3,
-                     m, kHid, kHid, 1);
-  hipLaunchKernelGGL(k_gemm_ab, dim3(nblocks(M)), dim3(kBlock), 0, st, s->H3, w + kOffW4, w + kOffB4, s->F, m, 1,
-                     kHid, 0);
-}
-
-// dW = A^T B (and the bias gradient, column sums of B) over M rows.
-void sur_atb(SurHost* s, hipStream_t st, const float* A, const float* B, float* Gm, float* bias_g, int M, int K1,
-             int K2) {
-  const int chunks = (M + kAtbRows - 1) / kAtbRows;
-  const int nout = K1 * K2 + K2;
-  hipLaunchKernelGGL(k_gemm_atb_part, dim3(nblocks(nout), chunks), dim3(kBlock), 0, st, A, B, s->part, M, K1, K2);
-  hipLaunchKernelGGL(k_gemm_atb_sum, dim3(nblocks(nout)), dim3(kBlock), 0, st, s->part, chunks, K1, K2, Gm, bias_g);
+  const dim3 grid((unsigned)((M + kLinRows - 1) / kLinRows));
+  hipLaunchKernelGGL(k_lin_fwd<kDescr>, grid, dim3(kBlock), 0, st, s->X, w + kOffW1, w + kOffB1, s->H1, m, nullptr,
+                     nullptr, nullptr);
+  hipLaunchKernelGGL(k_lin_fwd<kHid>, grid, dim3(kBlock), 0, st, s->H1, w + kOffW2, w + kOffB2, s->H2, m, nullptr,
+                     nullptr, nullptr);
+  hipLaunchKernelGGL(k_lin_fwd<kHid>, grid, dim3(kBlock), 0, st, s->H2, w + kOffW3, w + kOffB3, s->H3, m, w + kOffW4,
+                     w + kOffB4, s->F);
 }
 
 // Loss and gradient of the samples in s->X / s->T / s->N, then (update) one
@@ -71,20 +62,19 @@ int sur_train_step(plum_ctx* c, hipStream_t st, int samples, bool gather, bool u
     hipLaunchKernelGGL(k_gather_samples, dim3(16, samples), dim3(kBlock), 0, st, s->tr_x, s->tr_target, s->tr_n,
                        s->tr_ctl, samples, c->maxm, s->X, s->T, s->N);
   sur_forward32(c, st, M);
-  hipLaunchKernelGGL(k_train_loss, dim3(1), dim3(kBlock), 0, st, s->F, s->T, s->N, samples, c->maxm,
-                     s->p.target_clip, s->G, s->loss);
-  float* g = s->grad;
+  hipLaunchKernelGGL(k_train_loss, dim3((samples + kBlock / kWave - 1) / (kBlock / kWave)), dim3(kBlock), 0, st, s->F,
+                     s->T, s->N, samples, c->maxm, s->p.target_clip, s->G, s->loss_s);
   const float* w = s->w32;
-  const int m = (int)M;
-  sur_atb(s, st, s->H3, s->G, g + kOffW4, g + kOffB4, m, kHid, 1);
-  hipLaunchKernelGGL(k_out_delta, dim3(nblocks(M * kHid)), dim3(kBlock), 0, st, s->G, w + kOffW4, s->H3, s->D3, m);
-  sur_atb(s, st, s->H2, s->D3, g + kOffW3, g + kOffB3, m, kHid, kHid);
-  hipLaunchKernelGGL(k_gemm_abt_dtanh, dim3(nblocks(M * kHid)), dim3(kBlock), 0, st, s->D3, w + kOffW3, s->H2, s->D2,
-                     m, kHid, kHid);
-  sur_atb(s, st, s->H1, s->D2, g + kOffW2, g + kOffB2, m, kHid, kHid);
-  hipLaunchKernelGGL(k_gemm_abt_dtanh, dim3(nblocks(M * kHid)), dim3(kBlock), 0, st, s->D2, w + kOffW2, s->H1, s->D1,
-                     m, kHid, kHid);
-  sur_atb(s, st, s->X, s->D1, g + kOffW1, g + kOffB1, m, kDescr, kHid);
+  const int m = (int)M, chunks = (m + kAtbRows - 1) / kAtbRows;
+  const dim3 grid((unsigned)((M + kLinRows - 1) / kLinRows));
+  hipLaunchKernelGGL(k_lin_bwd, grid, dim3(kBlock), 0, st, s->D3, w + kOffW3, s->H2, s->D2, m, s->G, w + kOffW4,
+                     s->H3);
+  hipLaunchKernelGGL(k_lin_bwd, grid, dim3(kBlock), 0, st, s->D2, w + kOffW2, s->H1, s->D1, m, nullptr, nullptr,
+                     nullptr);
+  hipLaunchKernelGGL(k_grad_part, dim3(chunks, 4), dim3(kBlock), 0, st, s->X, s->H1, s->H2, s->H3, s->D1, s->D2,
+                     s->D3, s->G, m, s->part);
+  hipLaunchKernelGGL(k_grad_sum, dim3((kNParams + kWave - 1) / kWave), dim3(kBlock), 0, st, s->part, chunks, s->grad,
+                     s->loss_s, samples, s->loss);
   if (update) {
     s->step++;
     hipLaunchKernelGGL(k_adam, dim3(nblocks(kNParams)), dim3(kBlock), 0, st, s->w32, s->grad, s->m1, s->m2, kNParams,

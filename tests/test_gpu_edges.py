@@ -149,3 +149,62 @@ def test_volume_perturbation_sizes(n_chains, chain_len, L, alpha):
     scale = sum(abs(v) for v in orc.energy_full().values())
     for k in ("el", "lj", "bond", "dU"):
         assert abs(got[k] - ref[k]) <= 1e-13 * scale, (k, got[k], ref[k], scale)
+
+
+@pytest.mark.parametrize("samples,chain_len", [(1, 2), (3, 5), (2, 33), (17, 8)])
+def test_gradient_tiles(samples, chain_len):
+    """Loss and gradient with rows short of, at and past the 64-row and
+    128-row tiles, against the float64 reference; FP32 products and sums of up
+    to 272 rows and 128 inputs carry about sqrt(272 * 128) * 6e-8 of the
+    gradient's norm at most (bound 1e-4, that of test_gpu_surrogate.py)."""
+    sd = systems.config("tiny")
+    xyz, q, ty, ms = systems.build_bulk(2, chain_len, 2 * chain_len, 12.0, 41)
+    sd.update(xyz=xyz, q=q, type=ty, mol_start=ms, box=[12.0, 12.0, 12.0], alpha=0.2)
+    eng = E.Engine(sd)
+    eng.surrogate_enable(train_every=0, train_samples=1, ring=1, r_d=2.5, seed=3)
+    rng = np.random.default_rng(samples)
+    m = chain_len
+    x = np.abs(rng.normal(0, 0.3, (samples, 2 * m, 64))).astype(np.float32)
+    n = rng.integers(1, m + 1, samples).astype(np.int32)
+    t = rng.normal(0, 15.0, samples)
+    w = eng.surrogate_weights()
+    loss, grad = eng.surrogate_gradient(x.reshape(-1, 64), t, n)
+    ref_loss, ref = _reference_gradient(w, x, t, n)
+    assert abs(loss - ref_loss) <= 1e-5 * abs(ref_loss)
+    assert np.linalg.norm(grad - ref) <= 1e-4 * np.linalg.norm(ref)
+    f = eng.surrogate_forward(x.reshape(-1, 64), bf16=False)
+    assert np.max(np.abs(f - _reference_forward(w, x.reshape(-1, 64))[-1])) <= 1e-5 * max(1.0, np.max(np.abs(f)))
+
+
+def _layers(w):
+    o = np.cumsum([0, 64 * 128, 128, 128 * 128, 128, 128 * 128, 128, 128, 1])
+    w = np.asarray(w, dtype=np.float64)
+    p = [w[o[i]:o[i + 1]] for i in range(8)]
+    return [p[0].reshape(64, 128), p[1], p[2].reshape(128, 128), p[3], p[4].reshape(128, 128), p[5], p[6], p[7]]
+
+
+def _reference_forward(w, x):
+    p = _layers(w)
+    h1 = np.tanh(x @ p[0] + p[1])
+    h2 = np.tanh(h1 @ p[2] + p[3])
+    h3 = np.tanh(h2 @ p[4] + p[5])
+    return h1, h2, h3, h3 @ p[6] + p[7][0]
+
+
+def _reference_gradient(w, x, t, n, clip=20.0):
+    s, m2, _ = x.shape
+    m = m2 // 2
+    p = _layers(w)
+    X = x.reshape(-1, 64).astype(np.float64)
+    h1, h2, h3, f = _reference_forward(w, X)
+    f = f.reshape(s, 2, m)
+    used = np.arange(m)[None] < n[:, None]
+    res = ((f[:, 1] - f[:, 0]) * used).sum(1) - np.clip(t, -clip, clip)
+    g = np.zeros((s, 2, m))
+    g[:, 0], g[:, 1] = -2 * res[:, None] * used / s, 2 * res[:, None] * used / s
+    g = g.reshape(-1)
+    d3 = np.outer(g, p[6]) * (1 - h3 ** 2)
+    d2 = (d3 @ p[4].T) * (1 - h2 ** 2)
+    d1 = (d2 @ p[2].T) * (1 - h1 ** 2)
+    parts = [X.T @ d1, d1.sum(0), h1.T @ d2, d2.sum(0), h2.T @ d3, d3.sum(0), h3.T @ g, [g.sum()]]
+    return np.mean(res ** 2), np.concatenate([np.ravel(v) for v in parts])

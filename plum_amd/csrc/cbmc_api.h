@@ -4,13 +4,17 @@
 struct CbmcHost {
   // whole-chain growth: buffers for K trials x L steps, and the captured
   // launch sequence of one growth
-  int gK = 0, gL = 0, g_nkb = 0, g_prec = -1;
+  int gK = 0, gL = 0, g_prec = -1;
   GrowIn* g_in = nullptr;
   GrowOut* g_out = nullptr;
-  double *g_rnd = nullptr, *g_grown = nullptr, *g_kpart = nullptr;
-  double2 *g_Sx = nullptr, *g_cells = nullptr, *g_expl = nullptr;
+  double *g_rnd = nullptr, *g_grown = nullptr;
+  // two buffers each, used in turn by the steps
+  double* g_kpart[2] = {nullptr, nullptr};
+  double2 *g_Sx[2] = {nullptr, nullptr}, *g_cells[2] = {nullptr, nullptr}, *g_expl[2] = {nullptr, nullptr};
   char* gh_stage = nullptr;  // pinned: GrowIn, then the random numbers
   char* gh_out = nullptr;    // pinned: GrowOut, then the grown chain
+  const int* g_cells_of = nullptr;   // the cell list the graph was captured with
+  int g_gen = -1, g_cap = 0;
   hipGraph_t g_graph = nullptr;
   hipGraphExec_t g_exec = nullptr;
   int cap_k = 0, cap_g = 0, nkb = 0;
@@ -129,7 +133,9 @@ int grow_reserve(plum_ctx* c, int K, int L) {
   CbmcHost*& h = c->cbmc;
   if (!h) h = new CbmcHost();
   const int prec = c->p.precision;
-  if (K == h->gK && L == h->gL && prec == h->g_prec && h->g_exec) return PLUM_OK;
+  // (a re-gridded or enlarged cell list has other arrays than the ones captured)
+  const bool same_list = h->g_cells_of == c->d.cbead && h->g_gen == c->grid_gen && h->g_cap == c->g.cap;
+  if (K == h->gK && L == h->gL && prec == h->g_prec && same_list && h->g_exec) return PLUM_OK;
   if (h->g_exec) (void)hipGraphExecDestroy(h->g_exec);
   if (h->g_graph) (void)hipGraphDestroy(h->g_graph);
   h->g_exec = nullptr;
@@ -144,12 +150,14 @@ int grow_reserve(plum_ctx* c, int K, int L) {
     CHK(dalloc(c, &stage, grow_stage_bytes(k2, l2)));
     h->g_in = reinterpret_cast<GrowIn*>(stage);
     h->g_rnd = reinterpret_cast<double*>(stage + sizeof(GrowIn));
-    CHK(dalloc(c, &h->g_out, 1));
+    CHK(dalloc(c, &h->g_out, 2));
     CHK(dalloc(c, &h->g_grown, 6 * (size_t)l2));
-    CHK(dalloc(c, &h->g_Sx, (size_t)std::max(1, c->g.n_kh)));
-    CHK(dalloc(c, &h->g_cells, 2 * (size_t)k2 * c->nsplit));
-    CHK(dalloc(c, &h->g_expl, (size_t)k2));
-    CHK(dalloc(c, &h->g_kpart, (size_t)k2 * nkb));
+    for (int u = 0; u < 2; u++) {
+      CHK(dalloc(c, &h->g_Sx[u], (size_t)std::max(1, c->g.n_kh)));
+      CHK(dalloc(c, &h->g_cells[u], 2 * (size_t)k2 * kMaxGrowSplit * kQWaves));
+      CHK(dalloc(c, &h->g_expl[u], (size_t)k2));
+      CHK(dalloc(c, &h->g_kpart[u], (size_t)k2 * nkb));
+    }
     if (h->gh_stage) (void)hipHostFree(h->gh_stage);
     if (h->gh_out) (void)hipHostFree(h->gh_out);
     h->gh_stage = h->gh_out = nullptr;
@@ -160,27 +168,39 @@ int grow_reserve(plum_ctx* c, int K, int L) {
   h->gK = K;
   h->gL = L;
   h->g_prec = prec;
+  h->g_cells_of = c->d.cbead;
+  h->g_gen = c->grid_gen;
+  h->g_cap = c->g.cap;
   const Geo& g = c->g;
-  const int ns = c->nsplit;
   const int nkb = (g.use_ewald && g.n_kh > 0) ? (g.n_kh + kBlock - 1) / kBlock : 0;
-  h->g_nkb = nkb;
-  const int ncell = 2 * K * ns;
-  // one growth: upload, S_x, then two launches per step, download
+  // blocks per trial bead's query: about 512 in a step (two per CU), no fewer
+  // than 256 candidates, one per thread, each
+  const int ns = std::max(1, std::min(std::min(kMaxGrowSplit, 256 / K), (int)(c->cand / kBlock)));
+  GrowBuf B{};
+  B.in = h->g_in;
+  B.rnd = h->g_rnd;
+  B.grown = h->g_grown;
+  B.out = h->g_out;
+  for (int u = 0; u < 2; u++) {
+    B.Sx[u] = h->g_Sx[u];
+    B.cells[u] = h->g_cells[u];
+    B.expl[u] = h->g_expl[u];
+    B.kpart[u] = h->g_kpart[u];
+  }
+  // one growth: upload, S_x, then a launch per step and one for the last
+  // choice, download
   HIPCHK(hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
   (void)hipMemcpyAsync(h->g_in, h->gh_stage, grow_stage_bytes(K, L), hipMemcpyHostToDevice, c->st);
-  hipLaunchKernelGGL(k_grow_init, dim3(std::max(1, nkb)), dim3(kBlock), 0, c->st, g, c->d, h->g_in, h->g_Sx,
-                     h->g_out);
-  for (int s = 0; s < L; s++) {
+  hipLaunchKernelGGL(k_grow_init, dim3(std::max(1, (g.n_kh + kInitK - 1) / kInitK)), dim3(kBlock), 0, c->st, g, c->d,
+                     h->g_in, h->g_Sx[0], h->g_out);
+  for (int s = 0; s <= L; s++) {
+    const dim3 grid(s < L ? 2 * K * ns + K + K * nkb : 1);
     if (prec == PLUM_FP32_PAIR)
-      hipLaunchKernelGGL(k_grow_trials<1>, dim3(ncell + K + K * nkb), dim3(kBlock), 0, c->st, g, c->d, h->g_in,
-                         h->g_rnd, h->g_grown, h->g_Sx, h->g_out, s, ns, h->g_cells, h->g_expl, h->g_kpart);
+      hipLaunchKernelGGL(k_grow_step<1>, grid, dim3(kBlock), 0, c->st, g, c->d, B, s, ns, nkb);
     else
-      hipLaunchKernelGGL(k_grow_trials<0>, dim3(ncell + K + K * nkb), dim3(kBlock), 0, c->st, g, c->d, h->g_in,
-                         h->g_rnd, h->g_grown, h->g_Sx, h->g_out, s, ns, h->g_cells, h->g_expl, h->g_kpart);
-    hipLaunchKernelGGL(k_grow_select, dim3(1), dim3(kSelThreads), 0, c->st, g, c->d, h->g_in, h->g_rnd,
-                       h->g_grown, h->g_Sx, h->g_out, s, ns, nkb, h->g_cells, h->g_expl, h->g_kpart);
+      hipLaunchKernelGGL(k_grow_step<0>, grid, dim3(kBlock), 0, c->st, g, c->d, B, s, ns, nkb);
   }
-  (void)hipMemcpyAsync(h->gh_out, h->g_out, sizeof(GrowOut), hipMemcpyDeviceToHost, c->st);
+  (void)hipMemcpyAsync(h->gh_out, h->g_out + (L & 1), sizeof(GrowOut), hipMemcpyDeviceToHost, c->st);
   (void)hipMemcpyAsync(h->gh_out + sizeof(GrowOut), h->g_grown, sizeof(double) * 6 * (size_t)L,
                        hipMemcpyDeviceToHost, c->st);
   hipGraph_t gr = nullptr;

@@ -208,3 +208,79 @@ def _reference_gradient(w, x, t, n, clip=20.0):
     d1 = (d2 @ p[2].T) * (1 - h1 ** 2)
     parts = [X.T @ d1, d1.sum(0), h1.T @ d2, d2.sum(0), h2.T @ d3, d3.sum(0), h3.T @ g, [g.sum()]]
     return np.mean(res ** 2), np.concatenate([np.ravel(v) for v in parts])
+
+
+@pytest.mark.parametrize("K,L,mode,charged", [(1, 1, 0, True), (1, 5, 0, True), (3, 4, 1, True), (17, 6, 0, False),
+                                              (33, 3, 2, True), (300, 2, 0, True)])
+@pytest.mark.parametrize("precision", [E.PLUM_FP64, E.PLUM_FP32_PAIR])
+def test_growth_steps(K, L, mode, charged, precision):
+    """A whole growth (one launch a step, the choice repeated in every block)
+    against the single-step trial energies of plum_cbmc_trials with the same
+    draws: weight to 1e-10 (FP32 pairs: 1e-5, the exponent of the summed 1e-6
+    errors), chosen beads exactly."""
+    sd = systems.config("gc_small")
+    Lb = sd["box"][0]
+    rng = np.random.default_rng(K + L)
+    eng = E.Engine(sd, precision=precision)
+    first = np.array([[0.3, 0.4, 0.2], [7.0, 6.0, 5.0]])
+    d = first[:, None] - sd["xyz"][None]
+    d -= Lb * np.round(d / Lb)
+    while (d ** 2).sum(-1).min() < 0.81:
+        first = rng.uniform(0, Lb, (2, 3))
+        d = first[:, None] - sd["xyz"][None]
+        d -= Lb * np.round(d / Lb)
+    v = rng.normal(size=(L, K, 3))
+    disp = v / np.linalg.norm(v, axis=-1)[..., None]
+    ions = rng.uniform(0, Lb, (L, K, 3))
+    sel = rng.uniform(0, 1, L)
+    ms = sd["mol_start"]
+    kw = dict(type_ion=1, q_ion=1.0) if charged else {}
+    actual = exclude = None
+    if mode == 1:
+        exclude = (int(ms[0]), int(ms[7]) - 1)
+        actual = np.concatenate([sd["xyz"][:L], sd["xyz"][6:6 + L]])
+    for rep in range(2):   # the second growth replays the captured launches
+        w, stop, chain = eng.cbmc_grow(mode, L, K, 0, -1.0, first=first, disp=disp, ions=ions, sel=sel, actual=actual,
+                                       charged=charged, exclude=exclude, **kw)
+    beads, gi, W, end = np.zeros((0, 3)), np.zeros((0, 3)), 1.0, -1
+    for s in range(L):
+        if s == 0:
+            b, i = (actual[:1], actual[L:L + 1]) if mode == 1 else (first[:1], first[1:])
+        else:
+            b, i = beads[-1] + disp[s], ions[s].copy()
+            if mode == 1:
+                b[0], i[0] = actual[s], actual[L + s]
+        e = eng.cbmc_trials(b, 0, -1.0, grown=beads, ions=i if charged else None, type_ion=1, q_ion=1.0,
+                            grown_ions=gi if charged else None, exclude=exclude)
+        p = np.exp(-e)
+        W *= p.sum() / len(p)
+        if W == 0:   # every trial overlaps: the growth ends here
+            end = s
+            break
+        pick = 0
+        if s and mode != 1:
+            pick = min(int(np.searchsorted(np.cumsum(p), sel[s] * p.sum())), len(p) - 1)
+        beads, gi = np.vstack([beads, b[pick]]), np.vstack([gi, i[pick]])
+    assert stop == end
+    assert abs(w - W) <= (1e-10 if precision == E.PLUM_FP64 else 1e-5) * W
+    assert np.array_equal(chain[:len(beads)], beads)
+    if charged:
+        assert np.array_equal(chain[L:L + len(gi)], gi)
+
+
+def test_growth_after_a_regrid():
+    """The captured growth belongs to one cell list: after a re-grid it is
+    captured again, and gives the weight it gave before."""
+    sd = systems.config("gc_small")
+    rng = np.random.default_rng(4)
+    Lb = sd["box"][0]
+    kw = dict(first=np.array([[0.3, 0.4, 0.2], [7.0, 6.0, 5.0]]), disp=np.full((3, 4, 3), 0.58),
+              ions=rng.uniform(0, Lb, (3, 4, 3)), sel=np.full(3, 0.5), type_ion=1, q_ion=1.0)
+    eng = E.Engine(sd)
+    a = eng.cbmc_grow(2, 3, 4, 0, -1.0, **kw)
+    eng.set_tuning(cell_div=3)
+    eng.mc_run(40, sd["move_prob"], seed=3)
+    x = eng.positions()
+    b = eng.cbmc_grow(2, 3, 4, 0, -1.0, **kw)
+    c = E.Engine(dict(sd, xyz=x)).cbmc_grow(2, 3, 4, 0, -1.0, **kw)
+    assert abs(b[0] - c[0]) <= 1e-9 * abs(c[0]) and np.array_equal(b[2], c[2])

@@ -1,6 +1,8 @@
 // Device-resident state of one system (layout in HBM) and the small records
 // the host and the kernels exchange.
 #pragma once
+#include <stddef.h>
+
 #include "engine_dev.h"
 
 namespace plum {
@@ -105,6 +107,15 @@ struct Ctl {
   long long train_evals;   // first-stage rejections evaluated for training
   long long stale_cuts;    // batches ended early by a stale surrogate value
 };
+
+// The counters from `attempted` on are one array of this many (resolve_decide
+// adds to them a lane each).
+constexpr int kCtlCounters = 16;
+static_assert(offsetof(Ctl, stale_cuts) == offsetof(Ctl, attempted) + (kCtlCounters - 1) * sizeof(long long) &&
+                  offsetof(Ctl, valid_moves) == offsetof(Ctl, attempted) + 10 * sizeof(long long) &&
+                  offsetof(Ctl, skipped) == offsetof(Ctl, attempted) + 11 * sizeof(long long) &&
+                  offsetof(Ctl, s1_rejected) == offsetof(Ctl, attempted) + 12 * sizeof(long long),
+              "the counters are contiguous");
 
 struct Dev {
   // beads, index order

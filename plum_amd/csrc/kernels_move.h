@@ -425,29 +425,6 @@ __device__ double molecule_spring(const Geo& g, const Dev& d, int mol, bool tria
   return acc;  // valid in thread 0
 }
 
-// Spring energy of molecule `mol` with the beads lo..hi at mv_new[i - lo]
-// (a proposal's contiguous moved range) and the others at their current
-// positions; same fixed-order block tree as molecule_spring.
-__device__ double molecule_spring_range(const Geo& g, const Dev& d, int mol, int lo, int hi,
-                                        const double4* mv_new, double* sbuf) {
-  const int a = d.mol_start[mol], b = d.mol_start[mol + 1];
-  double acc = 0;
-  for (int base = a; base < b - 1; base += kBlock) {
-    const int i = base + threadIdx.x;
-    double e = 0;
-    if (i < b - 1) {
-      double p0[3] = {d.x[i], d.y[i], d.z[i]};
-      double p1[3] = {d.x[i + 1], d.y[i + 1], d.z[i + 1]};
-      if (i >= lo && i <= hi) { const double4 v = mv_new[i - lo]; p0[0] = v.x; p0[1] = v.y; p0[2] = v.z; }
-      if (i + 1 >= lo && i + 1 <= hi) { const double4 v = mv_new[i + 1 - lo]; p1[0] = v.x; p1[1] = v.y; p1[2] = v.z; }
-      const double dx = p0[0] - p1[0], dy = p0[1] - p1[1], dz = p0[2] - p1[2];
-      e = spring_energy(g, dx, dy, dz);
-    }
-    acc += block_sum<kBlock>(e, sbuf);
-  }
-  return acc;  // valid in thread 0
-}
-
 // Removes the tombstones of one cell, keeping slot order (one thread).
 __device__ void compact_cell(const Geo& g, const Dev& d, int cell) {
   const int cnt = d.ccount[cell];
@@ -846,54 +823,21 @@ __device__ MoveSel select_move(const Dev& d, const McDev& mc, unsigned long long
 
 // One proposal of Simulation::TranslationalMove (simulation.cc:241-312) with
 // the move generators of molecule.cc:103-312, drawing from Philox4x32-10
-// (counter = move number, streams: 1 move parameters, 2+i bead i).  `d` is
-// the view of one proposal slot (its rec / mv_* arrays); nothing shared per
-// bead is written, so two proposals of one molecule can coexist in a batch.
-struct PrSmem {
-  alignas(16) double s_b[kMaxChainDev][3];
-  int s_mol, s_type, s_valid, s_a, s_len;
-  double s_par[4];
-  int s_ipar[3];
+// (counter = move number, streams: 1 move parameters, 2+i bead i), by one
+// block: the new positions of the beads [lo, lo + n) (every generator moves a
+// contiguous range) in s_b, a = the molecule's first bead, len its length.
+// Every thread draws the move's parameters itself; returns lo and n in every
+// thread, s_b complete after a barrier.  A chain of dependent memory and LDS
+// round trips on one block, so the fewer of them the better.
+struct PropRange {
+  int lo, n;
 };
 
-__device__ void propose_block(const Geo& g, const Dev& d, const McDev& mc, unsigned long long ctr, MoveSel sel,
-                              PrSmem& sm) {
-  double (&s_b)[kMaxChainDev][3] = sm.s_b;
-  int& s_mol = sm.s_mol;
-  int& s_type = sm.s_type;
-  int& s_valid = sm.s_valid;
-  int& s_a = sm.s_a;
-  int& s_len = sm.s_len;
-  double* s_par = sm.s_par;
-  int* s_ipar = sm.s_ipar;
-  if (threadIdx.x == 0) {
-    const uint4 r1 = rnd(mc, ctr, 1, 0);
-    s_mol = sel.mol;
-    s_type = sel.mt;
-    s_valid = sel.valid;
-    s_a = d.mol_start[sel.mol];
-    s_len = d.mol_start[sel.mol + 1] - s_a;
-    s_par[0] = u01_32(r1.x);
-    s_par[1] = u01_32(r1.y);
-    s_par[2] = u01_32(r1.z);
-    s_par[3] = u01_32(r1.w);
-    s_ipar[0] = (int)(r1.w & 7u);
-  }
-  __syncthreads();
-  const int mol = s_mol, mt = s_type, a = s_a, len = s_len;
-  int nmv = 0;
-  if (!s_valid || len > kMaxChainDev) {
-    if (threadIdx.x == 0) {
-      d.rec->n_moved = 0;
-      d.rec->mol = mol;
-      d.rec->move_type = mt;
-      d.rec->valid = 0;
-      d.rec->contig = 1;
-      d.rec->lo = 0;
-      d.rec->hi = -1;
-    }
-    return;
-  }
+__device__ PropRange propose_positions(const Dev& d, const McDev& mc, unsigned long long ctr, int mt, int a, int len,
+                                       double (*s_b)[3]) {
+  const uint4 r1 = rnd(mc, ctr, 1, 0);
+  const double par[3] = {u01_32(r1.x), u01_32(r1.y), u01_32(r1.z)};
+  const unsigned ipar = r1.w & 7u;
   if (mt == 0) {
     // Molecule::BeadTranslate: 3 move_size along a random direction
     if (threadIdx.x == 0) {
@@ -901,34 +845,48 @@ __device__ void propose_block(const Geo& g, const Dev& d, const McDev& mc, unsig
       sphere(mc, ctr, 2, v);
       double vl = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
       if (vl > 0) vl = 3 * mc.move_size / vl;
-      d.mv_new[0] = make_double4(d.x[a] + vl * v[0], d.y[a] + vl * v[1], d.z[a] + vl * v[2], d.q[a]);
+      s_b[0][0] = d.x[a] + vl * v[0];
+      s_b[0][1] = d.y[a] + vl * v[1];
+      s_b[0][2] = d.z[a] + vl * v[2];
     }
-    nmv = 1;
-  } else if (mt == 1) {
+    return {a, 1};
+  }
+  if (mt == 1) {
     // Molecule::COMTranslate: each component U[0, move_size/2], random sign
     double v[3];
     for (int k = 0; k < 3; k++) {
-      v[k] = 0.5 * mc.move_size * s_par[k];
-      if (((s_ipar[0] >> k) & 1u) == 0) v[k] = -v[k];
+      v[k] = 0.5 * mc.move_size * par[k];
+      if (((ipar >> k) & 1u) == 0) v[k] = -v[k];
     }
-    for (int i = threadIdx.x; i < len; i += kBlock)
-      d.mv_new[i] = make_double4(d.x[a + i] + v[0], d.y[a + i] + v[1], d.z[a + i] + v[2], d.q[a + i]);
-    nmv = len;
-  } else if (mt == 2) {
+    for (int i = threadIdx.x; i < len; i += kBlock) {
+      s_b[i][0] = d.x[a + i] + v[0];
+      s_b[i][1] = d.y[a + i] + v[1];
+      s_b[i][2] = d.z[a + i] + v[2];
+    }
+    return {a, len};
+  }
+  if (mt == 2) {
     // Molecule::Pivot: each bond beyond the pivot gets a random kick of size
     // move_size*U, is renormalised to the (varied) bond length, and the
     // chain is rebuilt outward from the pivot bead.
-    int pivot = (int)floor(len * s_par[0]);
+    int pivot = (int)floor(len * par[0]);
     if (pivot == len) pivot--;
-    const double msr = mc.move_size * s_par[1];
+    const double msr = mc.move_size * par[1];
     for (int i = threadIdx.x; i < len; i += kBlock) {
-      if (i == pivot) continue;
+      const double x = d.x[a + i], y = d.y[a + i], z = d.z[a + i];
+      if (i == pivot) {
+        s_b[i][0] = x;
+        s_b[i][1] = y;
+        s_b[i][2] = z;
+        continue;
+      }
       const int nb = i > pivot ? i - 1 : i + 1;
+      const double xn = d.x[a + nb], yn = d.y[a + nb], zn = d.z[a + nb];
       double v[3];
       sphere(mc, ctr, 2 + (uint32_t)i, v);
-      double bx = d.x[a + i] - d.x[a + nb] + msr * v[0];
-      double by = d.y[a + i] - d.y[a + nb] + msr * v[1];
-      double bz = d.z[a + i] - d.z[a + nb] + msr * v[2];
+      double bx = x - xn + msr * v[0];
+      double by = y - yn + msr * v[1];
+      double bz = z - zn + msr * v[2];
       double bl = mc.bond_len;
       if (mc.vary_bond) {
         const uint4 rb = rnd(mc, ctr, 2 + (uint32_t)i, 0xB0u);
@@ -940,56 +898,44 @@ __device__ void propose_block(const Geo& g, const Dev& d, const McDev& mc, unsig
       s_b[i][2] = nrm * bz;
     }
     __syncthreads();
-    // the two halves outward from the pivot, one lane each, in LDS (each
-    // bond vector is replaced by the position it leads to), then written
-    // out in parallel
-    if (threadIdx.x < 2) {
-      const int dir = threadIdx.x == 0 ? 1 : -1;
-      double px = d.x[a + pivot], py = d.y[a + pivot], pz = d.z[a + pivot];
-      if (threadIdx.x == 0) {
-        s_b[pivot][0] = px;
-        s_b[pivot][1] = py;
-        s_b[pivot][2] = pz;
-      }
-      // eight bonds are read together, then summed in order: one LDS
-      // round trip per eight beads instead of one per bead, and no branch
-      // inside a group
+    // the two halves outward from the pivot, one lane per half and
+    // component, in the reference's summation order: each bond component is
+    // replaced by the coordinate it leads to.  Eight are read together, the
+    // next eight while these are summed.
+    if (threadIdx.x < 6) {
+      const int dir = threadIdx.x < 3 ? 1 : -1, c = threadIdx.x % 3;
       const int cnt = dir > 0 ? len - 1 - pivot : pivot;
+      double px = s_b[pivot][c];
+      double b[8], nx[8];
       int j = 0;
+      if (cnt >= 8) {
+#pragma unroll
+        for (int u = 0; u < 8; u++) b[u] = s_b[pivot + dir * (u + 1)][c];
+      }
       for (; j + 8 <= cnt; j += 8) {
-        double b[8][3];
+        const bool more = j + 16 <= cnt;
+#pragma unroll
+        for (int u = 0; u < 8; u++) nx[u] = more ? s_b[pivot + dir * (j + u + 9)][c] : 0.0;
 #pragma unroll
         for (int u = 0; u < 8; u++) {
-          const int i = pivot + dir * (j + u + 1);
-          b[u][0] = s_b[i][0];
-          b[u][1] = s_b[i][1];
-          b[u][2] = s_b[i][2];
+          px += b[u];
+          s_b[pivot + dir * (j + u + 1)][c] = px;
         }
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const int i = pivot + dir * (j + u + 1);
-          px += b[u][0]; py += b[u][1]; pz += b[u][2];
-          s_b[i][0] = px;
-          s_b[i][1] = py;
-          s_b[i][2] = pz;
-        }
+        for (int u = 0; u < 8; u++) b[u] = nx[u];
       }
       for (; j < cnt; j++) {
         const int i = pivot + dir * (j + 1);
-        px += s_b[i][0]; py += s_b[i][1]; pz += s_b[i][2];
-        s_b[i][0] = px;
-        s_b[i][1] = py;
-        s_b[i][2] = pz;
+        px += s_b[i][c];
+        s_b[i][c] = px;
       }
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < len; i += kBlock)
-      d.mv_new[i] = make_double4(s_b[i][0], s_b[i][1], s_b[i][2], d.q[a + i]);
-    nmv = len;
-  } else if (mt == 3) {
+    return {a, len};
+  }
+  if (mt == 3) {
     // Molecule::Crankshaft: rotate beads first+1..last-1 about first->last
-    int first = (int)floor((len - 2) * s_par[0]);
-    int last = (int)floor((len - first) * s_par[1]) + first;
+    const int first = (int)floor((len - 2) * par[0]);
+    int last = (int)floor((len - first) * par[1]) + first;
     if (last > len - 1) last = len - 1;
     double ax[3] = {d.x[a + last] - d.x[a + first], d.y[a + last] - d.y[a + first],
                     d.z[a + last] - d.z[a + first]};
@@ -998,7 +944,7 @@ __device__ void propose_block(const Geo& g, const Dev& d, const McDev& mc, unsig
       const double inv = sqrt(nn);
       ax[0] /= inv; ax[1] /= inv; ax[2] /= inv;
     }
-    const double angle = mc.move_size * (s_par[2] * 2 * M_PI - M_PI);
+    const double angle = mc.move_size * (par[2] * 2 * M_PI - M_PI);
     double sn, cs;
     sincos(angle, &sn, &cs);
     double R[3][3];
@@ -1008,55 +954,35 @@ __device__ void propose_block(const Geo& g, const Dev& d, const McDev& mc, unsig
     R[0][2] += sn * ax[1]; R[2][0] -= sn * ax[1];
     R[1][2] -= sn * ax[0]; R[2][1] += sn * ax[0];
     const double fx = d.x[a + first], fy = d.y[a + first], fz = d.z[a + first];
-    nmv = last - first - 1;
-    if (nmv < 0) nmv = 0;
-    for (int k = threadIdx.x; k < nmv; k += kBlock) {
+    const int n = max(0, last - first - 1);
+    for (int k = threadIdx.x; k < n; k += kBlock) {
       const int i = first + 1 + k;
       const double v0 = d.x[a + i] - fx, v1 = d.y[a + i] - fy, v2 = d.z[a + i] - fz;
-      d.mv_new[k] = make_double4(R[0][0] * v0 + R[0][1] * v1 + R[0][2] * v2 + fx,
-                                 R[1][0] * v0 + R[1][1] * v1 + R[1][2] * v2 + fy,
-                                 R[2][0] * v0 + R[2][1] * v1 + R[2][2] * v2 + fz, d.q[a + i]);
-      d.mv_idx[k] = a + i;
+      s_b[k][0] = R[0][0] * v0 + R[0][1] * v1 + R[0][2] * v2 + fx;
+      s_b[k][1] = R[1][0] * v0 + R[1][1] * v1 + R[1][2] * v2 + fy;
+      s_b[k][2] = R[2][0] * v0 + R[2][1] * v1 + R[2][2] * v2 + fz;
     }
-  } else {
-    // Molecule::RandomReptation: slide one slot, new end at the bond length
-    double bl = mc.bond_len;
-    if (mc.vary_bond) bl += (mc.bond_len / 5.0) * (s_par[0] - 0.5);
-    const int dir = (s_ipar[0] & 1u) ? 1 : -1;
-    const int end = dir == 1 ? len - 1 : 0;
-    for (int i = threadIdx.x; i < len; i += kBlock) {
-      if (i == end) {
-        double v[3];
-        sphere(mc, ctr, 2, v);
-        const double vl = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-        d.mv_new[i] = make_double4(d.x[a + i] + bl * v[0] / vl, d.y[a + i] + bl * v[1] / vl,
-                                   d.z[a + i] + bl * v[2] / vl, d.q[a + i]);
-      } else {
-        const int s = i + dir;
-        d.mv_new[i] = make_double4(d.x[a + s], d.y[a + s], d.z[a + s], d.q[a + i]);
-      }
+    return {a + first + 1, n};
+  }
+  // Molecule::RandomReptation: slide one slot, new end at the bond length
+  double bl = mc.bond_len;
+  if (mc.vary_bond) bl += (mc.bond_len / 5.0) * (par[0] - 0.5);
+  const int dir = (ipar & 1u) ? 1 : -1;
+  const int end = dir == 1 ? len - 1 : 0;
+  for (int i = threadIdx.x; i < len; i += kBlock) {
+    const int s = i == end ? i : i + dir;
+    double q[3] = {d.x[a + s], d.y[a + s], d.z[a + s]};
+    if (i == end) {
+      double v[3];
+      sphere(mc, ctr, 2, v);
+      const double vl = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+      for (int k = 0; k < 3; k++) q[k] = q[k] + bl * v[k] / vl;
     }
-    nmv = len;
+    s_b[i][0] = q[0];
+    s_b[i][1] = q[1];
+    s_b[i][2] = q[2];
   }
-  __syncthreads();
-  // moved list (crankshaft filled mv_idx itself)
-  for (int k = threadIdx.x; k < nmv; k += kBlock) {
-    const int i = (mt == 3) ? d.mv_idx[k] : a + k;
-    if (mt != 3) d.mv_idx[k] = i;
-    d.mv_old[k] = make_double4(d.x[i], d.y[i], d.z[i], d.q[i]);
-    d.mv_type[k] = d.type[i];
-  }
-  if (threadIdx.x == 0) {
-    d.rec->n_moved = nmv;
-    d.rec->mol = mol;
-    d.rec->move_type = mt;
-    d.rec->valid = 1;
-    // every generator moves a contiguous index range
-    const int lo = (mt == 3) ? a + (int)floor((len - 2) * s_par[0]) + 1 : a;
-    d.rec->contig = 1;
-    d.rec->lo = lo;
-    d.rec->hi = lo + nmv - 1;
-  }
+  return {a, len};
 }
 
 }  // namespace plum

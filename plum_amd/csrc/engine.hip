@@ -71,9 +71,11 @@ struct plum_ctx {
   double *epart_k = nullptr, *opart = nullptr;   // from-scratch k-space / springs, walls, self, dipole partials
   int *d_max = nullptr, *h_max = nullptr;        // largest cell count (device, pinned host)
   std::vector<int> mol_start;
-  char* h_in = nullptr;  // pinned staging of the move record
+  char* h_in = nullptr;  // pinned: trial coordinates, then bead indices of the caller's move
+  HostRes* h_res = nullptr;  // pinned: results of the host path
+  int seq = 0;               // its calls so far
   Ctl* h_ctl = nullptr;  // pinned copy of the control block
-  size_t in_bytes = 0, off_xyz = 0;
+  size_t off_idx = 0;
   char* d_in = nullptr;
   int drec_cap = 0;      // decision-record capacity allocated (plum_mc_record)
   hipEvent_t ev_idle = nullptr;  // marks the end of the work queued on st
@@ -307,7 +309,19 @@ int validate(const plum_params* p, int n, const double* xyz, const double* q, co
 
 int nmm_for(const plum_ctx*, int nm) { return nmm_blocks(nm); }
 
-// Blocks per real-space query: about 1.5 candidate slots per thread.
+// Waits until the kernel of host-path call `seq` has written its results to
+// c->h_res: polled for a while (a call takes tens of microseconds), then by
+// the stream, which also reports a kernel that failed.
+int host_wait(plum_ctx* c, int seq) {
+  const auto t0 = std::chrono::steady_clock::now();
+  for (int i = 1;; i++) {
+    if (__atomic_load_n(&c->h_res->seq, __ATOMIC_ACQUIRE) == seq) return PLUM_OK;
+    if (i % 64 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
+  }
+  HIPCHK(hipStreamSynchronize(c->st));
+  if (__atomic_load_n(&c->h_res->seq, __ATOMIC_ACQUIRE) != seq) return fail(PLUM_E_HIP, "trial-move kernel did not finish");
+  return PLUM_OK;
+}
 
 // k-space and real-space work of one trial move in one launch, once the
 // moved list (and, for the k space, the phase tables) exists on the device.
@@ -567,22 +581,22 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
   ALLOC(d.sk_part, (size_t)c->nchunk * std::max(1, g.n_kh));
   ALLOC(c->epart_k, c->nkb_full); ALLOC(c->opart, 4 * kFullSmall); ALLOC(c->d_max, 1);
   ALLOC(d.chain_ids, n_mols); ALLOC(d.ion_ids, n_mols);
-  // move record: header + idx[maxm] + pad + xyz[3 maxm], contiguous
-  c->off_xyz = sizeof(MoveRec) + sizeof(int) * maxm + ((sizeof(int) * maxm) % 8);
-  c->in_bytes = c->off_xyz + sizeof(double) * 3 * maxm;
   {
+    // move record of the host path: header, then the bead indices
     char* din = nullptr;
-    ALLOC(din, c->in_bytes);
+    ALLOC(din, sizeof(MoveRec) + sizeof(int) * maxm);
     c->d_in = din;
     d.rec = reinterpret_cast<MoveRec*>(din);
     d.mv_idx = reinterpret_cast<int*>(din + sizeof(MoveRec));
-    d.mv_xyz = reinterpret_cast<double*>(din + c->off_xyz);
   }
+  c->off_idx = sizeof(double) * 3 * maxm;
 #undef ALLOC
-  if (hipHostMalloc((void**)&c->h_in, c->in_bytes, hipHostMallocDefault) != hipSuccess ||
+  if (hipHostMalloc((void**)&c->h_in, c->off_idx + sizeof(int) * maxm, hipHostMallocCoherent) != hipSuccess ||
+      hipHostMalloc((void**)&c->h_res, sizeof(HostRes), hipHostMallocCoherent) != hipSuccess ||
       hipHostMalloc((void**)&c->h_max, sizeof(int), hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc((void**)&c->h_ctl, sizeof(Ctl), hipHostMallocDefault) != hipSuccess)
     return bail(fail(PLUM_E_NOMEM, "hipHostMalloc failed"));
+  std::memset(c->h_res, 0, sizeof(HostRes));
   auto up = [&](void* dst, const void* src, size_t bytes) -> int {
     if (bytes == 0) return PLUM_OK;
     HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->st));
@@ -607,7 +621,7 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
       hipMemsetAsync(d.ctl, 0, sizeof(Ctl), c->st) != hipSuccess ||
       hipMemsetAsync(d.plan, 0, sizeof(SpecPlan), c->st) != hipSuccess ||
       hipMemsetAsync(d.recs, 0, sizeof(MoveRec) * kMaxScreen, c->st) != hipSuccess ||
-      hipMemsetAsync(c->d_in, 0, c->in_bytes, c->st) != hipSuccess)
+      hipMemsetAsync(c->d_in, 0, sizeof(MoveRec) + sizeof(int) * maxm, c->st) != hipSuccess)
     return bail(fail(PLUM_E_HIP, "hipMemsetAsync failed"));
   if ((rc = build_cells(c, 0)) != PLUM_OK) return bail(rc);
   double f[8];
@@ -633,6 +647,7 @@ int plum_destroy(plum_ctx* c) {
   c->vp = nullptr;
   for (void* p : c->dev_allocs) (void)hipFree(p);
   if (c->h_in) (void)hipHostFree(c->h_in);
+  if (c->h_res) (void)hipHostFree(c->h_res);
   if (c->h_ctl) (void)hipHostFree(c->h_ctl);
   if (c->h_max) (void)hipHostFree(c->h_max);
   if (c->ev_idle) (void)hipEventDestroy(c->ev_idle);
@@ -671,43 +686,38 @@ int plum_energy_difference(plum_ctx* c, int mol, int n_moved, const int* idx, co
     for (int e = 0; e < 3; e++)
       if (!std::isfinite(trial_xyz[3 * k + e])) return fail(PLUM_E_ARG, "non-finite trial coordinate");
   }
-  MoveRec* r = reinterpret_cast<MoveRec*>(c->h_in);
-  r->n_moved = n_moved;
-  r->mol = mol;
-  r->move_type = -1;
-  r->valid = 1;
+  MoveRec r{};
+  r.n_moved = n_moved;
+  r.mol = mol;
+  r.move_type = -1;
+  r.valid = 1;
   int lo = b, hi = a - 1;
   for (int k = 0; k < n_moved; k++) {
     lo = std::min(lo, idx[k]);
     hi = std::max(hi, idx[k]);
   }
-  r->contig = (n_moved > 0 && hi - lo + 1 == n_moved) ? 1 : 0;
-  r->lo = lo;
-  r->hi = hi;
-  std::memcpy(c->h_in + sizeof(MoveRec), idx, sizeof(int) * n_moved);
-  std::memcpy(c->h_in + c->off_xyz, trial_xyz, sizeof(double) * 3 * n_moved);
-  HIPCHK(hipMemcpyAsync(c->d_in, c->h_in, sizeof(MoveRec) + sizeof(int) * n_moved, hipMemcpyHostToDevice,
-                        c->st));
-  if (n_moved > 0)
-    HIPCHK(hipMemcpyAsync(c->d_in + c->off_xyz, c->h_in + c->off_xyz, sizeof(double) * 3 * n_moved,
-                          hipMemcpyHostToDevice, c->st));
-  const Geo& g = c->g;
-  hipLaunchKernelGGL(k_host_moves, dim3(std::max(1, (n_moved + kBlock - 1) / kBlock)), dim3(kBlock), 0, c->st,
-                     g, c->d);
-  if (g.use_ewald && g.n_kh > 0 && n_moved > 0) {
-    const int tw = n_moved * 2 * std::max(1, g.tab_w);
-    hipLaunchKernelGGL(k_tables, dim3(std::max(1, std::min(2048, (tw + kBlock - 1) / kBlock))), dim3(kBlock), 0,
-                       c->st, g, c->d);
+  r.contig = (n_moved > 0 && hi - lo + 1 == n_moved) ? 1 : 0;
+  r.lo = lo;
+  r.hi = hi;
+  int* h_idx = reinterpret_cast<int*>(c->h_in + c->off_idx);
+  double* h_xyz = reinterpret_cast<double*>(c->h_in);
+  if (n_moved > 0) {
+    std::memcpy(h_idx, idx, sizeof(int) * n_moved);
+    std::memcpy(h_xyz, trial_xyz, sizeof(double) * 3 * n_moved);
   }
+  const Geo& g = c->g;
+  hipLaunchKernelGGL(k_host_move, dim3(std::max(1, (n_moved + kHostBeads - 1) / kHostBeads)), dim3(kBlock), 0, c->st,
+                     g, c->d, r, h_idx, h_xyz);
   launch_compute(c, n_moved);
+  const int seq = ++c->seq;
   hipLaunchKernelGGL(k_epilogue, dim3(1), dim3(kBlock), 0, c->st, g, c->d,
-                     (g.use_ewald && g.n_kh > 0) ? c->nkb : 0, 2 * n_moved * c->nsplit, nmm_for(c, n_moved));
+                     (g.use_ewald && g.n_kh > 0) ? c->nkb : 0, 2 * n_moved * c->nsplit, nmm_for(c, n_moved),
+                     c->h_res, seq);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(c->h_ctl, c->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
+  CHK(host_wait(c, seq));
   c->pending = true;
-  if (dE) to_terms(c->h_ctl->terms, dE);
-  if (total) *total = c->h_ctl->total;
+  if (dE) to_terms(c->h_res->terms, dE);
+  if (total) *total = c->h_res->total;
   return PLUM_OK;
 }
 
@@ -715,16 +725,16 @@ int plum_finalize(plum_ctx* c, int accept) {
   if (!c) return fail(PLUM_E_ARG, "null context");
   if (!c->pending) return fail(PLUM_E_STATE, "no pending trial move");
   const Geo& g = c->g;
-  hipLaunchKernelGGL(k_commit, dim3(1), dim3(kBlock), 0, c->st, g, c->d, accept ? 1 : 0);
-  if (g.use_ewald && g.n_kh > 0 && accept)
-    hipLaunchKernelGGL(k_commit_sk, dim3(c->nkb_full), dim3(kBlock), 0, c->st, g, c->d);
+  const int seq = accept ? ++c->seq : c->seq;
+  hipLaunchKernelGGL(k_commit, dim3(g.use_ewald && g.n_kh > 0 && accept ? 1 + c->nkb_full : 1), dim3(kBlock), 0, c->st,
+                     g, c->d, accept ? 1 : 0, c->h_res, seq);
   HIPCHK(hipGetLastError());
   c->pending = false;
   if (accept) {
-    HIPCHK(hipMemcpyAsync(c->h_ctl, c->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
-    if (c->h_ctl->overflow) {
+    CHK(host_wait(c, seq));
+    if (c->h_res->overflow) {
       // a cell ran out of slots: rebuild with twice the capacity
+      HIPCHK(hipStreamSynchronize(c->st));
       int zero = 0;
       HIPCHK(hipMemcpyAsync(&c->d.ctl->overflow, &zero, sizeof(int), hipMemcpyHostToDevice, c->st));
       CHK(build_cells(c, 2 * c->g.cap));

@@ -95,7 +95,6 @@ struct Ctl {
   int accept;           // decision of the pending move
   int overflow;         // a cell ran out of slots (cell list incomplete)
   int pending;          // a dE is waiting for commit/rollback
-  int sk_pending;       // S(k) += dS(k) still to be applied
   unsigned long long move_counter;   // Philox counter of the device loop
   long long attempted[5];
   long long accepted[5];
@@ -145,7 +144,6 @@ struct Dev {
   // pending move
   MoveRec* rec;
   int* mv_idx;
-  double* mv_xyz;         // caller's trial xyz (host path)
   double4 *mv_old, *mv_new;
   int* mv_type;
   Ctl* ctl;

@@ -11,42 +11,68 @@ constexpr int kKPerBlock = kBlock / kKGroups;
 constexpr int kMaxChainDev = 2048;      // longest molecule the device loop moves
 
 // ------------------------------------------------------------ move list
-// Host path: the caller's moved list -> old/new positions, masks.
-__global__ void k_host_moves(Geo g, Dev d) {
-  const int nm = d.rec->n_moved;
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nm; k += gridDim.x * blockDim.x) {
-    const int i = d.mv_idx[k];
+// Host path: the caller's move, read from pinned host memory -> moved list,
+// old/new positions, masks, and the phase tables e^{i k_l x} for l = 0..n_d of
+// each dimension d of every moved bead at its old and new position, with k_l
+// = (l*2) kPi / L exactly as potential_ewald_coul.cc:89-96 forms it (FP64
+// sincos; negative l is read as the conjugate, tab_phase).  One launch, a
+// block per kHostBeads beads: a move of 25 beads is 700 bytes, and two
+// uploads and two launches for them cost 14 us of the 62 a trial move took
+// (nine trial moves on 1,000 beads, two of them accepted, with the polled
+// results below: 562 -> 363 us).
+constexpr int kHostBeads = 8;
+__global__ __launch_bounds__(kBlock) void k_host_move(Geo g, Dev d, MoveRec rec, const int* __restrict__ idx,
+                                                      const double* __restrict__ xyz) {
+  __shared__ double s_p[2 * kHostBeads][3];
+  const int k0 = blockIdx.x * kHostBeads, nb = min(kHostBeads, rec.n_moved - k0);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *d.rec = rec;
+  if ((int)threadIdx.x < nb) {
+    const int k = k0 + threadIdx.x, i = idx[k];
+    const double x = xyz[3 * k], y = xyz[3 * k + 1], z = xyz[3 * k + 2];
+    const double qi = d.q[i], xo = d.x[i], yo = d.y[i], zo = d.z[i];
+    d.mv_idx[k] = i;
     d.moved[i] = 1;
     d.mv_slot[i] = k;
-    const double qi = d.q[i];
-    d.mv_old[k] = make_double4(d.x[i], d.y[i], d.z[i], qi);
-    d.mv_new[k] = make_double4(d.mv_xyz[3 * k], d.mv_xyz[3 * k + 1], d.mv_xyz[3 * k + 2], qi);
+    d.mv_old[k] = make_double4(xo, yo, zo, qi);
+    d.mv_new[k] = make_double4(x, y, z, qi);
     d.mv_type[k] = d.type[i];
+    double *po = s_p[2 * threadIdx.x], *pn = s_p[2 * threadIdx.x + 1];
+    po[0] = xo;
+    po[1] = yo;
+    po[2] = zo;
+    pn[0] = x;
+    pn[1] = y;
+    pn[2] = z;
   }
-}
-
-// Phase tables e^{i k_l x} for l = 0..n_d of each dimension d of every moved
-// bead at its old and new position, with k_l = (l*2) kPi / L exactly as
-// potential_ewald_coul.cc:89-96 forms it (FP64 sincos).  Negative l is read
-// as the conjugate (tab_phase).
-__global__ void k_tables(Geo g, Dev d) {
-  const int nm = d.rec->n_moved;
-  const int total = nm * 2 * g.tab_w;
-  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < total; e += gridDim.x * blockDim.x) {
+  if (!g.use_ewald || g.n_kh == 0) return;
+  __syncthreads();
+  for (int e = threadIdx.x; e < 2 * nb * g.tab_w; e += kBlock) {
     const int row = e / g.tab_w, off = e - row * g.tab_w;
-    const int m = row >> 1, on = row & 1;
     int dim, l;
     if (off <= g.nkx) { dim = 0; l = off; }
     else if (off <= g.nkx + 1 + g.nky) { dim = 1; l = off - (g.nkx + 1); }
     else { dim = 2; l = off - (g.nkx + 1) - (g.nky + 1); }
-    const double4 p = on ? d.mv_new[m] : d.mv_old[m];
-    const double xv = dim == 0 ? p.x : (dim == 1 ? p.y : p.z);
-    const double xw = wrap_coord(xv, g.L[dim], g.inv_L[dim]);
+    const double xw = wrap_coord(s_p[row][dim], g.L[dim], g.inv_L[dim]);
     const double kd = (double)(l * 2) * kPi / g.L[dim];
     double s, c;
     sincos(kd * xw, &s, &c);
-    d.tab[(size_t)row * g.tab_w + off] = make_double2(c, s);
+    d.tab[(size_t)(2 * k0 + row) * g.tab_w + off] = make_double2(c, s);
   }
+}
+
+// What the host path returns, in pinned host memory: the values, then (with
+// everything before it visible to the host) the number of the call, which the
+// host polls.  A copy back and a wait for the stream took 20 us.
+struct HostRes {
+  double terms[8];
+  double total;
+  int overflow;
+  int seq;
+};
+
+__device__ __forceinline__ void host_done(HostRes* res, int seq) {
+  __threadfence_system();
+  __hip_atomic_store(&res->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Table offsets of k vector l (x, y, z segments of l >= 0) and whether its y
@@ -77,9 +103,8 @@ __device__ __forceinline__ double2 tab_phase(const double2* t, const TabIdx& i) 
 // ------------------------------------------------------------ k space
 // dS(k) = sum_m q_m (e^{ik.r'_m} - e^{ik.r_m}); dE_k = c_k (|S+dS|^2 - |S|^2).
 // Block = 16 k vectors x 16 groups of moved beads; the groups are reduced in
-// LDS.  A still-pending S(k) += dS(k) of the previous accepted move is applied
-// first by the thread that owns k (device loop).  FP64 in both precision
-// modes: it is a small part of the per-move work and keeps S(k) exact.
+// LDS.  FP64 in both precision modes: it is a small part of the per-move work
+// and keeps S(k) exact.
 struct KSmem {
   double2 s_ds[kKGroups][kKPerBlock];
   double sh[kBlock / kWave];
@@ -112,48 +137,12 @@ __device__ void kspace_block(const Geo& g, const Dev& d, int blk, KSmem& sm) {
     double2 t = s_ds[0][kk];
 #pragma unroll
     for (int r = 1; r < kKGroups; r++) { t.x += s_ds[r][kk].x; t.y += s_ds[r][kk].y; }
-    double2 S = d.Sk[k];
-    if (d.ctl->sk_pending) {
-      const double2 prev = d.dS[k];
-      S.x += prev.x;
-      S.y += prev.y;
-      d.Sk[k] = S;
-    }
+    const double2 S = d.Sk[k];
     e = d.ck[k] * (2.0 * (S.x * t.x + S.y * t.y) + t.x * t.x + t.y * t.y);
     d.dS[k] = t;
   }
   const double r = block_sum<kBlock>(e, sh);
   if (threadIdx.x == 0) d.part_k[blk] = r;
-}
-
-// Applies a pending S(k) += dS(k) (end of a device run).
-__global__ void k_flush_sk(Geo g, Dev d) {
-  if (!d.ctl->sk_pending) return;
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < g.n_kh) {
-    double2 s = d.Sk[k];
-    const double2 ds = d.dS[k];
-    s.x += ds.x;
-    s.y += ds.y;
-    d.Sk[k] = s;
-  }
-}
-
-// Clears the pending S(k) flag after k_flush_sk (single thread).
-__global__ void k_clear_sk_pending(Dev d) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) d.ctl->sk_pending = 0;
-}
-
-// Host path: S(k) += dS(k) right away when the caller accepts.
-__global__ void k_commit_sk(Geo g, Dev d) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < g.n_kh) {
-    double2 s = d.Sk[k];
-    const double2 ds = d.dS[k];
-    s.x += ds.x;
-    s.y += ds.y;
-    d.Sk[k] = s;
-  }
 }
 
 // ------------------------------------------------------------ real space
@@ -748,21 +737,40 @@ __device__ void epilogue_block(const Geo& g, const Dev& d, int nkb, int nrb, int
     for (int k = 0; k < 8; k++) C->terms[k] = t[k];
     C->total = dE;
     C->pending = 1;
-    C->sk_pending = 0;
     C->accept = 0;
   }
   __syncthreads();
 }
 
-__global__ __launch_bounds__(kBlock) void k_epilogue(Geo g, Dev d, int nkb, int nrb, int nmmb) {
+__global__ __launch_bounds__(kBlock) void k_epilogue(Geo g, Dev d, int nkb, int nrb, int nmmb, HostRes* res,
+                                                     int seq) {
   __shared__ EpSmem sm;
   epilogue_block(g, d, nkb, nrb, nmmb, sm);
+  if (threadIdx.x != 0) return;
+  for (int k = 0; k < 8; k++) res->terms[k] = d.ctl->terms[k];
+  res->total = d.ctl->total;
+  host_done(res, seq);
 }
 
-// Host path: commit / roll back after the caller's decision.
-__global__ __launch_bounds__(kBlock) void k_commit(Geo g, Dev d, int accept) {
+// Host path: commit / roll back after the caller's decision; the blocks past
+// the first add the accepted dS(k) to S(k).
+__global__ __launch_bounds__(kBlock) void k_commit(Geo g, Dev d, int accept, HostRes* res, int seq) {
   __shared__ CommitSmem cs;
+  if (blockIdx.x > 0) {
+    const int k = (blockIdx.x - 1) * kBlock + threadIdx.x;
+    if (k < g.n_kh) {
+      double2 s = d.Sk[k];
+      const double2 ds = d.dS[k];
+      s.x += ds.x;
+      s.y += ds.y;
+      d.Sk[k] = s;
+    }
+    return;
+  }
   commit_block(g, d, accept && d.rec->valid, cs);
+  if (!accept || threadIdx.x != 0) return;
+  res->overflow = __hip_atomic_load(&d.ctl->overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  host_done(res, seq);
 }
 
 // ------------------------------------------------------------ proposals

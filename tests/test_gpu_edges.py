@@ -284,3 +284,30 @@ def test_growth_after_a_regrid():
     b = eng.cbmc_grow(2, 3, 4, 0, -1.0, **kw)
     c = E.Engine(dict(sd, xyz=x)).cbmc_grow(2, 3, 4, 0, -1.0, **kw)
     assert abs(b[0] - c[0]) <= 1e-9 * abs(c[0]) and np.array_equal(b[2], c[2])
+
+
+@pytest.mark.parametrize("n", [0, 1, 7, 8, 9, 17, 70])
+def test_host_moves_of_every_size(n):
+    """The caller's move read from pinned memory, eight beads a block: any
+    subset of a molecule's beads, three moves in a row, the second one
+    rejected, each against the oracle at the coordinates before it."""
+    sd = systems.config("tiny")
+    xyz, q, ty, ms = systems.build_bulk(2, 70, 6, 14.0, 3)
+    sd.update(xyz=xyz, q=q, type=ty, mol_start=ms, box=[14.0] * 3)
+    eng = E.Engine(sd)
+    rng = np.random.default_rng(n)
+    for step in range(3):
+        x = eng.positions()
+        idx = np.sort(rng.choice(np.arange(ms[0], ms[1]), n, replace=False)).astype(np.int32)
+        new = x[idx] + rng.normal(0, 0.02, (n, 3))
+        orc = O.Oracle(dict(sd, xyz=x))
+        orc.set_trial(0, idx, new)
+        t_ref, d_ref = orc.delta(0)
+        t, d = eng.delta(0, idx, new)
+        for k in E.TERMS:
+            assert abs(d[k] - d_ref[k]) <= 1e-10 * max(abs(d_ref[k]), 1e-2), (step, k, d[k], d_ref[k])
+        eng.finalize(step != 1)
+        x1 = x.copy()
+        if step != 1:
+            x1[idx] = new
+        assert np.array_equal(eng.positions(), x1)

@@ -23,6 +23,7 @@ constexpr int kMaxProp = 16;                                  // exactly evaluat
 constexpr int kMaxScreen = 32;                                // screened proposals per batch
 constexpr int kMaxPairs = kMaxProp * (kMaxProp - 1) / 2;       // exact-slot pairs
 constexpr int kKVals = kMaxProp + kMaxPairs;                   // k-space sums per batch
+constexpr int kGramParts = 32;                                // most blocks of the k-space cross sums
 constexpr int kDescr = 64;                                     // surrogate descriptor length
 
 // Pair slot of exact slots p != q.
@@ -64,7 +65,8 @@ struct SpecPlan {
   unsigned acc_mask;             // exact slots accepted by the last resolve: S(k) += dS pending
   int pad;
   double de_s[kMaxScreen];       // surrogate dE of each proposal (0 without it)
-  double ksum[kKVals];           // k space: dE per exact slot, then 2 sum c_k Re(dS_p* dS_q)
+  double ksum[kMaxProp];         // k-space dE per exact slot
+  double kx[kGramParts][kMaxPairs];   // parts of 2 sum c_k Re(dS_p* dS_q) per exact-slot pair
   double2 rsum[kMaxProp];        // (LJ, real) dE per exact slot against the unmoved state
   double2 xsum[kMaxPairs];       // (LJ, real) cross term per near pair
 };

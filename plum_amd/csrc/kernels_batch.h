@@ -26,8 +26,8 @@
 //                    slot, and cross blocks (LJ + real pairs between two
 //                    slots' moved beads, old/new combinations), spread over
 //                    one grid.
-//   k_reduce_spec    one block per sum and system, fixed order; the k-space
-//                    cross sums 2 c_k Re(dS_p* dS_q) formed from the dS rows.
+//   k_reduce_spec    the sums of every system, fixed order; the k-space cross
+//                    sums 2 c_k Re(dS_p* dS_q) as a Gram matrix of the dS rows.
 //   k_resolve_spec   grid R: the reference's sequential Metropolis chain over
 //                    the batch (simulation.cc:241-355), decided by one wave,
 //                    each dE corrected by the cross terms of the proposals
@@ -1205,25 +1205,42 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 }
 
 constexpr int kReduceThreads = 1024;
+constexpr int kReduceWaves = kReduceThreads / kWave;
+constexpr int kPairBlocks = (kMaxPairs + kReduceWaves - 1) / kReduceWaves;
+constexpr int kReduceBlocks = 2 * kMaxProp + kGramParts + kPairBlocks;
 
-// Sums of a batch, one block per (sum, system), fixed order: blockIdx.x in
-// [0, kMaxProp) the k-space dE per exact slot (the k tiles' partials), then
-// kMaxPairs k-space cross sums 2 sum_k c_k Re(dS_p* dS_q) of the slot pairs
-// p < q (pair_index order) from the dS rows, then kMaxProp (LJ, real) sums per
-// exact slot (real-space query blocks + moved-moved blocks), then kMaxPairs
-// real-space cross sums of the near pairs.
+// Blocks of a system's k-space cross sums: 384 k vectors are 96 KB of dS rows
+// a block, which a compute unit takes in about 2 us (10,170 k vectors, a launch:
+// 17 us by 4 blocks, 7.0 by 20, 5.9 by 27).
+__device__ __forceinline__ int gram_parts(int n_kh) { return max(1, min(kGramParts, (n_kh + 383) / 384)); }
+
+// Sums of a batch, fixed order, blocks of one system (blockIdx.y):
+//   [0, kMaxProp)   k-space dE per exact slot (the k tiles' partials)
+//   gram_parts      k-space cross sums 2 sum_k c_k Re(dS_p* dS_q) of all slot
+//                   pairs p < q, a part of the k vectors each (the resolve adds
+//                   the parts): a Gram matrix of the sixteen dS rows, so the
+//                   FP64 matrix cores read each row once (lane l holds row
+//                   l % 16 at k vector l / 16 of four, times c_k as A and
+//                   plain as B)
+//   kMaxProp        (LJ, real) sums per exact slot (query and moved-moved
+//                   blocks)
+//   kPairBlocks     real-space cross sums of the near pairs, a wave each
+// Launch and latency bound: a block per sum (272 a system, most of them with
+// nothing to do, each pair reading its two rows again) took 7.4 us for 16 slots of 10,170 k
+// vectors, now 5.9, and 38 us for 24 systems.
 __global__ __launch_bounds__(kReduceThreads) void k_reduce_spec(const Geo* __restrict__ G, const Dev* __restrict__ D,
                                                         const RepCfg* __restrict__ RC, int R) {
-  __shared__ double sh[kReduceThreads / kWave];
-  const int j = blockIdx.x, r = blockIdx.y;
+  __shared__ double sh[kReduceWaves];
+  __shared__ double s_g[kReduceWaves][kMaxProp * kMaxProp];
+  const int r = blockIdx.y, t = threadIdx.x, lane = t % kWave, wv = t / kWave;
+  int j = blockIdx.x;
   if (r >= R) return;
-  const Geo& g = G[r];
-  const Dev& d = D[r];
-  const RepCfg& rc = RC[r];
+  const Geo g = load_const(G, r);
+  const Dev d = load_const(D, r);
+  const RepCfg rc = load_const(RC, r);
   SpecPlan* plan = d.plan;
-  if (plan->n_prop == 0) return;
-  const int ne = plan->n_exact;
-  const int t = threadIdx.x;
+  const int np0 = plan->n_prop, ne = plan->n_exact;
+  if (np0 == 0) return;
   if (j < kMaxProp) {
     if (j >= ne) return;
     double s = 0;
@@ -1231,33 +1248,42 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce_spec(const Geo* __res
     for (int i = t; i < np; i += kReduceThreads) s += d.part_ks[(size_t)j * np + i];
     s = block_sum<kReduceThreads>(s, sh);
     if (t == 0) plan->ksum[j] = s;
-  } else if (j < kKVals) {
-    const int pj = j - kMaxProp;
-    int q = (int)((1.0 + sqrt(1.0 + 8.0 * pj)) * 0.5);
-    while (q * (q - 1) / 2 > pj) q--;
-    while ((q + 1) * q / 2 <= pj) q++;
-    const int p = pj - q * (q - 1) / 2;
-    if (q >= ne) return;
-    double s = 0;
+  } else if ((j -= kMaxProp) < kGramParts) {
+    if (ne < 2) return;
+    const int parts = gram_parts(g.n_kh);
+    if (j >= parts) return;
+    const int waves = parts * kReduceWaves, row = lane % 16, in = lane / 16;
+    const int ch = ((g.n_kh + waves - 1) / waves + 3) & ~3;
+    const int k0 = (j * kReduceWaves + wv) * ch, k1 = min(k0 + ch, g.n_kh);
+    f64x4 acc = {0, 0, 0, 0};
     if (rc.nkb_s > 0) {
-      const double2* a = d.dS + (size_t)p * g.n_kh;
-      const double2* b = d.dS + (size_t)q * g.n_kh;
+      const double2* a = d.dS + (size_t)min(row, ne - 1) * g.n_kh;
 #pragma unroll 4
-      for (int k = t; k < g.n_kh; k += kReduceThreads) {
-        const double2 u = a[k], v = b[k];
-        s += d.ck[k] * (u.x * v.x + u.y * v.y);
+      for (int k = k0; k < k1; k += 4) {
+        const int kk = k + in, kc = min(kk, g.n_kh - 1);
+        const double2 u = a[kc];
+        const double c = kk < k1 ? d.ck[kc] : 0.0;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(c * u.x, u.x, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(c * u.y, u.y, acc, 0, 0, 0);
       }
     }
-    s = block_sum<kReduceThreads>(s, sh);
-    if (t == 0) plan->ksum[j] = 2.0 * s;
-  } else if (j < kKVals + kMaxProp) {
-    const int e = j - kKVals;
-    if (e >= ne) return;
-    const int nm = d.recs[plan->screen_of[e]].n_moved;
+#pragma unroll
+    for (int v = 0; v < 4; v++) s_g[wv][(4 * v + in) * kMaxProp + row] = acc[v];
+    __syncthreads();
+    const int p = t / kMaxProp, q = t % kMaxProp;
+    if (p < q && q < ne) {
+      double s = 0;
+#pragma unroll
+      for (int w = 0; w < kReduceWaves; w++) s += s_g[w][t];
+      plan->kx[j][pair_index(p, q)] = 2.0 * s;
+    }
+  } else if ((j -= kGramParts) < kMaxProp) {
+    if (j >= ne) return;
+    const int nm = d.recs[plan->screen_of[j]].n_moved;
     if (nm == 0) return;
     const int nreal = query_blocks(nm, plan->qblk) * kQWaves, nmm = nmm_blocks(nm);
-    const double2* pr = d.part_r + (size_t)e * rc.rstride;
-    const double2* pm = d.part_mm + (size_t)e * rc.nmmb;
+    const double2* pr = d.part_r + (size_t)j * rc.rstride;
+    const double2* pm = d.part_mm + (size_t)j * rc.nmmb;
     double lj = 0, re = 0;
     for (int i = t; i < nreal; i += kReduceThreads) {
       lj += pr[i].x;
@@ -1269,19 +1295,20 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce_spec(const Geo* __res
     }
     lj = block_sum<kReduceThreads>(lj, sh);
     re = block_sum<kReduceThreads>(re, sh);
-    if (t == 0) plan->rsum[e] = make_double2(lj, re);
+    if (t == 0) plan->rsum[j] = make_double2(lj, re);
   } else {
-    const int jj = j - kKVals - kMaxProp;
+    const int jj = (j - kMaxProp) * kReduceWaves + wv;
     if (jj >= plan->n_near) return;
     const int off = plan->pair_off[jj], nblk = plan->pair_off[jj + 1] - off;
     double lj = 0, re = 0;
-    for (int i = t; i < nblk; i += kReduceThreads) {
-      lj += d.part_x[off + i].x;
-      re += d.part_x[off + i].y;
+    for (int i = lane; i < nblk; i += kWave) {
+      const double2 x = d.part_x[off + i];
+      lj += x.x;
+      re += x.y;
     }
-    lj = block_sum<kReduceThreads>(lj, sh);
-    re = block_sum<kReduceThreads>(re, sh);
-    if (t == 0) plan->xsum[jj] = make_double2(lj, re);
+    lj = wave_sum(lj);
+    re = wave_sum(re);
+    if (lane == 0) plan->xsum[jj] = make_double2(lj, re);
   }
 }
 
@@ -1590,7 +1617,23 @@ __global__ __launch_bounds__(kBlock) void k_resolve_spec(const Geo* __restrict__
                                 make_uint2((uint32_t)mc.seed, (uint32_t)(mc.seed >> 32)));
     sm.s_u[t] = u01_32(u.x);
   }
-  if (t >= 64 && t < 64 + kKVals) sm.s_ksum[t - 64] = plan->ksum[t - 64];
+  if (t >= 64 && t < 64 + kKVals) {
+    const int i = t - 64;
+    double v = 0;
+    if (i < kMaxProp) {
+      v = plan->ksum[i];
+    } else {
+      const int parts = gram_parts(g.n_kh);
+      for (int u0 = 0; u0 < parts; u0 += 16) {   // sixteen loads in flight
+        double x[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) x[u] = plan->kx[min(u0 + u, parts - 1)][i - kMaxProp];
+#pragma unroll
+        for (int u = 0; u < 16; u++) v += u0 + u < parts ? x[u] : 0.0;
+      }
+    }
+    sm.s_ksum[i] = v;
+  }
   if (t >= 128 && t < 128 + kMaxPairs) {
     const int j = t - 128;
     pp = plan->pair_p[j];

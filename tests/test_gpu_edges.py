@@ -311,3 +311,22 @@ def test_host_moves_of_every_size(n):
         if step != 1:
             x1[idx] = new
         assert np.array_equal(eng.positions(), x1)
+
+
+@pytest.mark.parametrize("pmax", [1, 2, 3, 15, 16])
+@pytest.mark.parametrize("alpha", [0.02, 0.9])   # fewer k vectors than waves; several steps a wave
+def test_cross_sums_of_a_batch(pmax, alpha):
+    """Cross terms of one to sixteen slots: the k-space Gram matrix with rows
+    and k vectors past the end, the near pairs a wave each."""
+    sd = systems.config("tiny")
+    xyz, q, ty, ms = systems.build_bulk(4, 40, 20, 14.0, 6)
+    sd.update(xyz=xyz, q=q, type=ty, mol_start=ms, box=[14.0] * 3, alpha=alpha, move_prob=[0.6, 0.1, 0.1, 0.1, 0.1])
+    eng, st, recs, _ = record_run(sd, 200, pmax, seed=pmax)
+    run, full = eng.totals(), eng.energy_full()
+    # dE_k is what is left of sums whose terms add up to about the k-space and
+    # self energies E (a hundred kT and more at alpha 0.9), each with phases of
+    # l <= 20 rounded factors: up to 20 x 2.2e-16 E each way, 1e-14 E together,
+    # which the scaled tolerance allows at a floor of 1e-4 E
+    scale = max(abs(full["kspace"]), abs(full["self"]))
+    replay(sd, recs, 1e-10, floor=max(1e-2, 1e-4 * scale))
+    assert abs(run["kspace"] - full["kspace"]) <= 1e-10 * max(1.0, abs(full["kspace"]))

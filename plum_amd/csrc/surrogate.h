@@ -802,7 +802,10 @@ __global__ void k_pack_bf16(const float* __restrict__ w, NetBF16* __restrict__ n
   if (i == 0) net->b4 = w[kOffB4];
 }
 
-// Minibatch gather: the `samples` most recent ring slots (newest last).
+// Minibatch gather: the `samples` most recent ring slots (newest last).  Rows
+// past a sample's beads are never written in the ring and come out as zeros:
+// their weight in the gradient is 0, but 0 times whatever the memory held
+// before (an infinity, a NaN) is not.
 __global__ void k_gather_samples(const float* __restrict__ tr_x, const double* __restrict__ tr_target,
                                  const int* __restrict__ tr_n, const int* __restrict__ tr_ctl, int samples,
                                  int maxm, float* __restrict__ X, double* __restrict__ target, int* __restrict__ n) {
@@ -811,11 +814,12 @@ __global__ void k_gather_samples(const float* __restrict__ tr_x, const double* _
   const int head = tr_ctl[0], ring = tr_ctl[1];
   const int slot = ((head - samples + i) % ring + ring) % ring;
   const size_t rowsz = (size_t)2 * maxm * kDescr;
+  const int ni = tr_n[slot];
   for (size_t k = blockIdx.x * blockDim.x + threadIdx.x; k < rowsz; k += (size_t)gridDim.x * blockDim.x)
-    X[(size_t)i * rowsz + k] = tr_x[(size_t)slot * rowsz + k];
+    X[(size_t)i * rowsz + k] = (int)(k / kDescr) % maxm < ni ? tr_x[(size_t)slot * rowsz + k] : 0.f;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     target[i] = tr_target[slot];
-    n[i] = tr_n[slot];
+    n[i] = ni;
   }
 }
 

@@ -783,22 +783,24 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
   const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
   const double rs = STR ? g.rs + kStretchMargin : g.rs, rs2 = STR ? rs * rs : g.rs2;
   QWaveSmem<P, MODE>& sm = sh.q[wv];
-  // each point as the image nearest the first point's wrapped position (an
-  // image of a point has the same pair images within the radius), and the
-  // points' bounding box
+  // each point as the image nearest the first point (an image of a point has
+  // the same pair images within the radius), and the points' bounding box.  The
+  // image is the point's own wrapped position plus a whole edge or none, as a
+  // candidate's is, so that a bead at the same coordinates is at distance 0 to
+  // the bit.
   const unsigned vm = (unsigned)__ballot(valid) & ((1u << kCluster) - 1u);
   const int np = ALL ? kCluster : __popc(vm);
   const int ref = __builtin_ctz(vm);
   double bl[3], bh[3];
   {
-    const double p0v[3] = {lane_double(p.x, ref), lane_double(p.y, ref), lane_double(p.z, ref)};
-    const double pv[3] = {p.x, p.y, p.z};
-    double qv[3];
+    const double pw[3] = {wrap_coord(p.x, g.L[0], g.inv_L[0]), wrap_coord(p.y, g.L[1], g.inv_L[1]),
+                          wrap_coord(p.z, g.L[2], g.inv_L[2])};
+    double qv[3], nv[3];
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-      double dk = valid ? pv[k] - p0v[k] : 0.0;
-      dk -= g.L[k] * rint(dk * g.inv_L[k]);
-      qv[k] = wrap_coord(p0v[k], g.L[k], g.inv_L[k]) + dk;
+      const double rk = lane_double(pw[k], ref);
+      nv[k] = -rint((pw[k] - rk) * g.inv_L[k]);
+      qv[k] = valid ? pw[k] + nv[k] * g.L[k] : rk;
     }
     if (threadIdx.x < kCluster) {
       // (a point that does not count is out of every candidate's reach)
@@ -806,9 +808,9 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
       sh.s_ptt[lane] = type;
       sh.s_own[lane] = own;
       if constexpr (STR) {
-        // the point's image is p's own: qv is p wrapped near the reference
+        // (p is a slot of the list: its own image is the wrapped one)
         const int jo = valid ? own : 0;
-        sh.s_ptd[lane] = valid ? st.dw[jo] + rint((qv[2] - p.z) * g.inv_L[2]) * st.dz : 0.0;
+        sh.s_ptd[lane] = valid ? st.dw[jo] + nv[2] * st.dz : 0.0;
         sh.s_cls[lane] = stretch_class(st.mol_of[jo], st.phantom);
       }
     }
@@ -1013,10 +1015,9 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
         }
         // FP64 queue: every charged pair (P = 0), the close ones (P = 1)
         // ALL: a pair counts from its lower index, a bead's own images by half
-        // (the bead itself is at zero, up to the rounding of the point's image)
         const int own = ALL ? sh.s_own[i] : -1;
         const bool self = ALL && j == own;
-        const bool in = r2 <= rcj2 && (!ALL || j > own || (self && r2 > 1e-6)) &&
+        const bool in = r2 <= rcj2 && (!ALL || j > own || (self && r2 > 0)) &&
                         (!STR || stretch_pair(sh.s_cls[i], cj));
         const bool near = in && (P == 0 || r2 < fp64_b2);
         const unsigned long long m = __ballot(near);

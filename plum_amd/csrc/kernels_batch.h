@@ -787,7 +787,8 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
   // the same pair images within the radius), and the points' bounding box.  The
   // image is the point's own wrapped position plus a whole edge or none, as a
   // candidate's is, so that a bead at the same coordinates is at distance 0 to
-  // the bit.
+  // the bit.  A z that is not periodic stays as wrapped: LJ counts the
+  // candidates of image 0 only, which is the image of the point's own z.
   const unsigned vm = (unsigned)__ballot(valid) & ((1u << kCluster) - 1u);
   const int np = ALL ? kCluster : __popc(vm);
   const int ref = __builtin_ctz(vm);
@@ -799,7 +800,7 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
 #pragma unroll
     for (int k = 0; k < 3; k++) {
       const double rk = lane_double(pw[k], ref);
-      nv[k] = -rint((pw[k] - rk) * g.inv_L[k]);
+      nv[k] = k < g.npbc ? -rint((pw[k] - rk) * g.inv_L[k]) : 0.0;
       qv[k] = valid ? pw[k] + nv[k] * g.L[k] : rk;
     }
     if (threadIdx.x < kCluster) {

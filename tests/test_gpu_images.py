@@ -11,7 +11,7 @@ import pytest
 
 from oracle import oracle as O
 from plum_amd import engine as E
-from plum_amd import systems
+from plum_amd import host, systems
 from test_gpu_record import record_run, replay
 
 pytestmark = pytest.mark.gpu
@@ -63,3 +63,40 @@ def test_coincident_beads(cell_div, precision):
         # a move within a chain cancels up to ten sentinels, 1e8 each rounded
         # to 1.5e-8 in both sums: 3e-7 at most, 1e-10 of a floor of 1e4
         replay(sd, recs, 1e-10, floor=1e4)
+
+
+def _slab(L, alpha, length, seed, dipole):
+    """Chains and ions between two walls, beads of some chains at both."""
+    sd = systems.config("slab_small")
+    box = [12.0, 12.0, L]
+    xyz, q, ty, ms = host.synth_system(6, length, 6 * length, 0, box, seed, npbc=2, z_range=(0.7, L - 0.7))
+    # chain 0 straight up, from wall to wall
+    a, b = int(ms[0]), int(ms[1])
+    xyz[a:b] = [0.3, 0.4, 0.0] + np.linspace(0.7, L - 0.7, b - a)[:, None] * [0.0, 0.0, 1.0]
+    sd.update(xyz=xyz, q=q, type=ty, mol_start=ms, box=box, alpha=alpha, dipole=dipole, grafted=0,
+              move_prob=[0.2, 0.2, 0.2, 0.2, 0.2])
+    return sd
+
+
+@pytest.mark.parametrize("L,length,dipole", [(8.0, 9, 0), (8.0, 20, 0), (10.0, 11, 0), (8.0, 9, 1)])
+@pytest.mark.parametrize("cell_div", [1, 2])
+def test_slab_thinner_than_the_cutoff(L, length, dipole, cell_div):
+    """Two periodic dimensions and no padding: one cell, and one cluster of a
+    chain's beads, spans more than half of the height.  LJ takes z as it is
+    (no image of z), the real-space sum has the period of the height."""
+    sd = _slab(L, (5.0 / 12.0) ** 2, length, 4, dipole)
+    orc = O.Oracle(sd)
+    eng = E.Engine(sd, cell_div=cell_div)
+    assert eng.info().real_cutoff > L / 2
+    ref = _full_matches(eng, orc)
+    _vp_matches(eng, orc, sum(abs(v) for v in ref.values()))
+    eng.close()
+    eng, _, recs, _ = record_run(sd, 150, 16, seed=6)
+    # a trial that leaves the slab is rejected by its wall term, its LJ (at a z
+    # that the cell list wraps) is not the reference's
+    out = [r for r in recs if r["dE"]["wall"] >= 0.9e8]
+    assert not any(r["accepted"] for r in out) and len(out) <= len(recs) // 2
+    for r in out:
+        r["evaluated"] = False
+    assert replay(sd, recs, 1e-10)[3] >= 50
+    _full_matches(eng, O.Oracle(dict(sd, xyz=eng.positions())))

@@ -126,6 +126,18 @@ extern "C" int plum_cbmc_trials(plum_ctx* c, const plum_cbmc_request* rq, const 
 
 namespace {
 
+// Whether every block of a growth step repeats the choice of the step before
+// (a launch less a step) or one block makes it in a launch between them.  The
+// repeated choice takes a block K / 16 passes over the trials' partial sums and
+// a serial sum of K weights, and every further round of blocks takes it again:
+// it pays for up to two passes and one round (four blocks on each of 256 compute
+// units).  A growth of 8 steps, repeated / one block: 160 / 169 us at K = 16 and
+// 570 blocks, 138 / 144 at K = 16 and 848, 185 / 189 at K = 32 and 576; 221 / 215
+// at K = 48 and 576, 198 / 169 at K = 24 and 1,272, 12.8 / 1.2 ms at K = 1,024 and
+// 19,456.
+constexpr int kFusedTrials = 32, kFusedBlocks = 1024;
+bool grow_fused(int K, int blocks) { return K <= kFusedTrials && blocks <= kFusedBlocks; }
+
 size_t grow_stage_bytes(int K, int L) { return sizeof(GrowIn) + sizeof(double) * grow_rnd_size(K, L); }
 size_t grow_out_bytes(int L) { return sizeof(GrowOut) + sizeof(double) * 6 * (size_t)L; }
 
@@ -187,18 +199,21 @@ int grow_reserve(plum_ctx* c, int K, int L) {
     B.expl[u] = h->g_expl[u];
     B.kpart[u] = h->g_kpart[u];
   }
-  // one growth: upload, S_x, then a launch per step and one for the last
-  // choice, download
+  // one growth: upload, S_x, then a launch per step (and one per choice where
+  // it is not fused) and one for the last choice, download
   HIPCHK(hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
   (void)hipMemcpyAsync(h->g_in, h->gh_stage, grow_stage_bytes(K, L), hipMemcpyHostToDevice, c->st);
   hipLaunchKernelGGL(k_grow_init, dim3(std::max(1, (g.n_kh + kInitK - 1) / kInitK)), dim3(kBlock), 0, c->st, g, c->d,
                      h->g_in, h->g_Sx[0], h->g_out);
-  for (int s = 0; s <= L; s++) {
-    const dim3 grid(s < L ? 2 * K * ns + K + K * nkb : 1);
+  const int blocks = 2 * K * ns + K + K * nkb;
+  const int fused = grow_fused(K, blocks) ? 1 : 0;
+  for (int s = 0; s < L; s++) {
     if (prec == PLUM_FP32_PAIR)
-      hipLaunchKernelGGL(k_grow_step<1>, grid, dim3(kBlock), 0, c->st, g, c->d, B, s, ns, nkb);
+      hipLaunchKernelGGL(k_grow_step<1>, dim3(blocks), dim3(kBlock), 0, c->st, g, c->d, B, s, ns, nkb, fused);
     else
-      hipLaunchKernelGGL(k_grow_step<0>, grid, dim3(kBlock), 0, c->st, g, c->d, B, s, ns, nkb);
+      hipLaunchKernelGGL(k_grow_step<0>, dim3(blocks), dim3(kBlock), 0, c->st, g, c->d, B, s, ns, nkb, fused);
+    if (!fused || s == L - 1)
+      hipLaunchKernelGGL(k_grow_select, dim3(1), dim3(kSelThreads), 0, c->st, g, c->d, B, s, ns, nkb);
   }
   (void)hipMemcpyAsync(h->gh_out, h->g_out + (L & 1), sizeof(GrowOut), hipMemcpyDeviceToHost, c->st);
   (void)hipMemcpyAsync(h->gh_out + sizeof(GrowOut), h->g_grown, sizeof(double) * 6 * (size_t)L,

@@ -2,24 +2,27 @@
 // step of an insertion, a deletion or a Widom test insertion (cbmc.cc:213-533)
 // is one launch, the trial draws made beforehand by the host in the
 // reference's order.
-//   k_grow_init  S_x(k) = S(k) - S_excluded(k), Rosenbluth weight 1
-//   k_grow_step  launch s = 0 .. L: every block first finishes step s - 1 (the
-//                trial energies from its partial sums, the weights, W *= W_s /
-//                K, the choice of the bead -- insertion: by the pre-drawn
-//                uniform; deletion: the existing bead, trial 0), then does its
-//                part of step s: part 1 (cell list, LJ + real space), parts
-//                2-4 (the grown chain, the bead-counterion pair, self images,
-//                walls; one block per trial) or the k-space sums of a trial
-//                bead and counterion, positions built from the bead just
-//                chosen.
-// The choice is a few hundred loads and K exponentials, so it is repeated in
-// every block rather than made by one in a launch between the steps: at 16
-// trials, 3,200 beads, an insertion and a deletion of 32 beads take 1543 ->
-// 1080 us, a step 24 -> 17 us; a step is latency (chains of dependent loads,
-// the queue of the query, a launch), not bytes or operations.  All blocks
-// compute the same bits.  What a launch reads and the next one's value
-// of (state, S_x, partial sums) live in two buffers used in turn; block 0
-// writes the state, the blocks of trial 0 write S_x.
+//   k_grow_init    S_x(k) = S(k) - S_excluded(k), Rosenbluth weight 1
+//   k_grow_step    launch s = 0 .. L - 1: every block first finishes step s - 1
+//                  (grow_select: the trial energies from its partial sums, the
+//                  weights, W *= W_s / K, the choice of the bead -- insertion:
+//                  by the pre-drawn uniform; deletion: the existing bead, trial
+//                  0), then does its part of step s: part 1 (cell list, LJ +
+//                  real space), parts 2-4 (the grown chain, the bead-counterion
+//                  pair, self images, walls; one block per trial) or the k-space
+//                  sums of a trial bead and counterion, positions built from the
+//                  bead just chosen.
+//   k_grow_select  the end of the last step, and of every step where repeating
+//                  it in each block costs more than a launch (many trials,
+//                  grow_fused): by one block.
+// With few trials the choice is a few hundred loads and K exponentials, so it
+// is repeated in every block rather than made by one in a launch between the
+// steps: at 16 trials, 3,200 beads, an insertion and a deletion of 32 beads take
+// 1543 -> 1080 us, a step 24 -> 15 us; a step is latency (chains of dependent
+// loads, the queue of the query, a launch), not bytes or operations.  All blocks
+// compute the same bits, and so does the one block.  What a launch reads and
+// the next one's value of (state, S_x, partial sums) live in two buffers used in
+// turn; block 0 writes the state, the blocks of trial 0 write S_x.
 // Step 0 is the first bead (and its counterion) alone, trial 0 of K.
 #pragma once
 #include "kernels_batch.h"
@@ -218,7 +221,7 @@ __device__ bool grow_select(const Geo& g, const GrowBuf& B, const GrowIn& in, co
   // 16 lanes per trial
   constexpr int G = 16;
   const int l16 = threadIdx.x % G;
-  for (int t = threadIdx.x / G; t < Kt; t += kBlock / G) {
+  for (int t = threadIdx.x / G; t < Kt; t += blockDim.x / G) {
     double elj = 0, ere = 0, ek = 0;
     const int np = nparts * kQWaves;
     for (int i = l16; i < np; i += G) {
@@ -302,10 +305,18 @@ __device__ bool grow_select(const Geo& g, const GrowBuf& B, const GrowIn& in, co
   return sm.s_go != 0;
 }
 
-// Launch s of a growth: step s - 1 finished, then (s < L) blocks [0, 2 K
-// nparts): part 1 of (bead b, trial t, split); then K blocks of parts 2-4, one
-// per trial; then K x nkb blocks of k space, (trial, 256 vectors) each.  Step
-// 0 evaluates trial 0 only.  A trial bead's query is a cluster query of one
+// The end of step s in a launch of its own (k_grow_step not fused).
+constexpr int kSelThreads = 1024;
+__global__ __launch_bounds__(kSelThreads) void k_grow_select(Geo g, Dev d, GrowBuf B, int s, int nparts, int nkb) {
+  __shared__ GrowSelSmem sm;
+  const GrowIn in = *B.in;
+  grow_select(g, B, in, grow_ptr(B.rnd, in.K, in.L), s, nparts, nkb, sm);
+}
+
+// Launch s of a growth: (fused) step s - 1 finished, then blocks [0, 2 K nparts):
+// part 1 of (bead b, trial t, split); then K blocks of parts 2-4, one per trial;
+// then K x nkb blocks of k space, (trial, 256 vectors) each.  Step 0 evaluates
+// trial 0 only.  A trial bead's query is a cluster query of one
 // point (its trials are close together, its counterions anywhere, and each
 // trial's energy is wanted): the pairs in range, a fifth of the candidates
 // where the cells are coarse, meet in the queue instead of leaving most lanes
@@ -313,7 +324,7 @@ __device__ bool grow_select(const Geo& g, const GrowBuf& B, const GrowIn& in, co
 template <int P>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_grow_step(Geo g, Dev d, GrowBuf B,
                                                                                               int s, int nparts,
-                                                                                              int nkb) {
+                                                                                              int nkb, int fused) {
   __shared__ union {
     QueryShare<P, Q_MOVED> q;
     GrowSelSmem sel;
@@ -324,11 +335,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
   const GrowPtr p = grow_ptr(B.rnd, in.K, in.L);
   const int K = in.K, Kt = s == 0 ? 1 : K;
   if (s > 0) {
-    if (!grow_select(g, B, in, p, s - 1, nparts, nkb, sm.sel)) return;
-    if (threadIdx.x < 6) s_prev[threadIdx.x] = sm.sel.s_pos[threadIdx.x];
+    if (fused) {
+      if (!grow_select(g, B, in, p, s - 1, nparts, nkb, sm.sel)) return;
+      if (threadIdx.x < 6) s_prev[threadIdx.x] = sm.sel.s_pos[threadIdx.x];
+    } else {
+      if (B.out[s & 1].stop >= 0) return;
+      if (threadIdx.x < 6) {
+        const size_t bead = threadIdx.x < 3 ? s - 1 : in.L + s - 1;
+        s_prev[threadIdx.x] = B.grown[3 * bead + threadIdx.x % 3];
+      }
+    }
     __syncthreads();
   }
-  if (s >= in.L) return;
   const int ncell = 2 * K * nparts, cur = s & 1;
   if ((int)blockIdx.x < ncell) {
     const int q = blockIdx.x / nparts, sp = blockIdx.x - q * nparts;

@@ -213,12 +213,14 @@ def _reference_gradient(w, x, t, n, clip=20.0):
 @pytest.mark.parametrize("K,L,mode,charged", [(1, 1, 0, True), (1, 5, 0, True), (3, 4, 1, True), (17, 6, 0, False),
                                               (33, 3, 2, True), (300, 2, 0, True)])
 @pytest.mark.parametrize("precision", [E.PLUM_FP64, E.PLUM_FP32_PAIR])
-def test_growth_steps(K, L, mode, charged, precision):
-    """A whole growth (one launch a step, the choice repeated in every block)
-    against the single-step trial energies of plum_cbmc_trials with the same
+def test_growth_steps(K, L, mode, charged, precision, alpha=None):
+    """A whole growth (the choice of a bead repeated in every block, or past 32
+    trials or 1,024 blocks made by one block) against the single-step trial energies of plum_cbmc_trials with the same
     draws: weight to 1e-10 (FP32 pairs: 1e-5, the exponent of the summed 1e-6
     errors), chosen beads exactly."""
     sd = systems.config("gc_small")
+    if alpha:
+        sd["alpha"] = alpha
     Lb = sd["box"][0]
     rng = np.random.default_rng(K + L)
     eng = E.Engine(sd, precision=precision)
@@ -266,6 +268,15 @@ def test_growth_steps(K, L, mode, charged, precision):
     assert np.array_equal(chain[:len(beads)], beads)
     if charged:
         assert np.array_equal(chain[L:L + len(gi)], gi)
+
+
+@pytest.mark.parametrize("K,L,mode,alpha", [(32, 4, 0, None), (33, 4, 1, None), (24, 4, 0, 1.6), (24, 3, 1, 1.6),
+                                            (1024, 2, 0, None)])
+def test_growth_on_both_sides_of_the_choice_rule(K, L, mode, alpha):
+    """The last number of trials whose choice every block repeats, the first
+    whose choice one block makes, the same below 32 trials with so many k
+    vectors that the step passes 1,024 blocks, and the largest number."""
+    test_growth_steps(K, L, mode, True, E.PLUM_FP64, alpha)
 
 
 def test_growth_after_a_regrid():

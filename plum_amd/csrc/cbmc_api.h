@@ -2,8 +2,9 @@
 // end of engine.hip.
 
 struct CbmcHost {
-  // whole-chain growth: buffers for K trials x L steps, and the captured
-  // launch sequence of one growth
+  // whole-chain growth: buffers for up to capK trials x capL steps, and the
+  // captured launch sequence of one growth of gK x gL
+  int capK = 0, capL = 0;
   int gK = 0, gL = 0, g_prec = -1;
   GrowIn* g_in = nullptr;
   GrowOut* g_out = nullptr;
@@ -152,11 +153,24 @@ int grow_reserve(plum_ctx* c, int K, int L) {
   if (h->g_graph) (void)hipGraphDestroy(h->g_graph);
   h->g_exec = nullptr;
   h->g_graph = nullptr;
-  if (K > h->gK || L > h->gL) {
-    // grow-only device buffers (older ones stay with the context until it
-    // is destroyed)
-    const int k2 = std::max(K, h->gK), l2 = std::max(L, h->gL);
+  if (K > h->capK || L > h->capL) {
+    // larger buffers in place of the ones there are (no growth is running: a
+    // call ends with its stream drained)
+    const int k2 = std::max(K, h->capK), l2 = std::max(L, h->capL);
     const int nkb = std::max(1, (c->g.n_kh + kBlock - 1) / kBlock);
+    h->capK = h->capL = 0;
+    dfree(c, &h->g_in);
+    dfree(c, &h->g_out);
+    dfree(c, &h->g_grown);
+    for (int u = 0; u < 2; u++) {
+      dfree(c, &h->g_Sx[u]);
+      dfree(c, &h->g_cells[u]);
+      dfree(c, &h->g_expl[u]);
+      dfree(c, &h->g_kpart[u]);
+    }
+    if (h->gh_stage) (void)hipHostFree(h->gh_stage);
+    if (h->gh_out) (void)hipHostFree(h->gh_out);
+    h->gh_stage = h->gh_out = nullptr;
     // GrowIn and the random numbers in one buffer, one upload
     char* stage = nullptr;
     CHK(dalloc(c, &stage, grow_stage_bytes(k2, l2)));
@@ -170,12 +184,11 @@ int grow_reserve(plum_ctx* c, int K, int L) {
       CHK(dalloc(c, &h->g_expl[u], (size_t)k2));
       CHK(dalloc(c, &h->g_kpart[u], (size_t)k2 * nkb));
     }
-    if (h->gh_stage) (void)hipHostFree(h->gh_stage);
-    if (h->gh_out) (void)hipHostFree(h->gh_out);
-    h->gh_stage = h->gh_out = nullptr;
     if (hipHostMalloc((void**)&h->gh_stage, grow_stage_bytes(k2, l2), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void**)&h->gh_out, grow_out_bytes(l2), hipHostMallocDefault) != hipSuccess)
       return fail(PLUM_E_NOMEM, "hipHostMalloc failed");
+    h->capK = k2;
+    h->capL = l2;
   }
   h->gK = K;
   h->gL = L;

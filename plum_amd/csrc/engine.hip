@@ -121,6 +121,18 @@ int dalloc(plum_ctx* c, T** ptr, size_t count) {
   return PLUM_OK;
 }
 
+// Gives back a buffer of dalloc's before the context is destroyed.
+template <typename T>
+void dfree(plum_ctx* c, T** ptr) {
+  auto& v = c->dev_allocs;
+  const auto it = std::find(v.begin(), v.end(), (void*)*ptr);
+  if (it != v.end()) {
+    (void)hipFree(*it);
+    v.erase(it);
+  }
+  *ptr = nullptr;
+}
+
 // potential_ewald_coul.cc:43-75: slab padding and the derived cutoffs.
 void derive_cutoffs(const plum_params& p, plum_info& info) {
   double box[3] = {p.box[0], p.box[1], p.box[2]};

@@ -270,12 +270,16 @@ def test_growth_steps(K, L, mode, charged, precision, alpha=None):
         assert np.array_equal(chain[L:L + len(gi)], gi)
 
 
-@pytest.mark.parametrize("K,L,mode,alpha", [(32, 4, 0, None), (33, 4, 1, None), (24, 4, 0, 1.6), (24, 3, 1, 1.6),
+@pytest.mark.parametrize("K,L,mode,alpha", [(32, 4, 0, None), (33, 4, 1, None), (32, 4, 0, 3.2), (30, 3, 1, 3.2),
                                             (1024, 2, 0, None)])
 def test_growth_on_both_sides_of_the_choice_rule(K, L, mode, alpha):
     """The last number of trials whose choice every block repeats, the first
     whose choice one block makes, the same below 32 trials with so many k
     vectors that the step passes 1,024 blocks, and the largest number."""
+    if alpha:
+        eng = E.Engine(dict(systems.config("gc_small"), alpha=alpha))
+        assert K * (3 + eng.info().n_k_half // 256) > 1024
+        eng.close()
     test_growth_steps(K, L, mode, True, E.PLUM_FP64, alpha)
 
 

@@ -69,6 +69,7 @@ struct SurHost {
   double *T = nullptr, *loss = nullptr;
   int* N = nullptr;
   float* part = nullptr;  // chunk partials of the gradient
+  int part_cap = 0;       // chunks allocated for
   double* loss_s = nullptr;  // squared error of each sample
   int step = 0;
   long long train_steps = 0;

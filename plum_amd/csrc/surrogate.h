@@ -637,6 +637,9 @@ __global__ __launch_bounds__(kBlock) void k_lin_bwd(float* __restrict__ D, const
 // blockIdx.y, into part[c] laid out as the parameters; k_grad_sum adds the
 // chunks.
 constexpr int kAtbRows = 128, kAtbStage = 32;
+// Chunks of one pass over the rows: a chunk's partials are all the parameters
+// (166 KB), so the passes keep them to 21 MB whatever the rows.
+constexpr int kGradChunks = 128;
 
 template <int K1>
 __device__ void atb_chunk(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ gw,
@@ -713,10 +716,10 @@ __global__ __launch_bounds__(kBlock) void k_grad_part(const float* __restrict__ 
 }
 static_assert(kBlock == 2 * kHid, "two halves of the rows");
 
-// grad = sum of the chunks' partials (four interleaved groups of chunks, then
-// the groups), kWave parameters per block; block 0 also sums the samples'
-// losses.
-__global__ __launch_bounds__(kBlock) void k_grad_sum(const float* __restrict__ part, int chunks,
+// grad = (add: grad +) the sum of the chunks' partials (four interleaved groups
+// of chunks, then the groups), kWave parameters per block; block 0 also sums the
+// samples' losses.
+__global__ __launch_bounds__(kBlock) void k_grad_sum(const float* __restrict__ part, int chunks, int add,
                                                      float* __restrict__ grad, const double* __restrict__ loss_s,
                                                      int samples, double* __restrict__ loss) {
   __shared__ float s_g[kBlock / kWave][kWave];
@@ -730,7 +733,10 @@ __global__ __launch_bounds__(kBlock) void k_grad_sum(const float* __restrict__ p
   }
   s_g[w][lane] = s;
   __syncthreads();
-  if (w == 0 && p < kNParams) grad[p] = (s_g[0][lane] + s_g[1][lane]) + (s_g[2][lane] + s_g[3][lane]);
+  if (w == 0 && p < kNParams) {
+    const float t = (s_g[0][lane] + s_g[1][lane]) + (s_g[2][lane] + s_g[3][lane]);
+    grad[p] = add ? grad[p] + t : t;
+  }
   if (blockIdx.x == 0) {
     double l = 0;
     for (int i = threadIdx.x; i < samples; i += kBlock) l += loss_s[i];

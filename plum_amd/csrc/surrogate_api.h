@@ -33,8 +33,22 @@ int sur_workspace(plum_ctx* c, int samples) {
   CHK(salloc(s, &s->T, samples));
   CHK(salloc(s, &s->N, samples));
   CHK(salloc(s, &s->loss_s, samples));
-  CHK(salloc(s, &s->part, ((M + kAtbRows - 1) / kAtbRows) * (size_t)kNParams));
   s->tb_cap = samples;
+  return PLUM_OK;
+}
+
+// Partials of the weight gradients of `chunks` chunks (a forward alone needs
+// none of them).
+int sur_grad_space(SurHost* s, int chunks) {
+  if (chunks <= s->part_cap) return PLUM_OK;
+  s->part_cap = 0;
+  const auto it = std::find(s->allocs.begin(), s->allocs.end(), (void*)s->part);
+  if (it != s->allocs.end()) {
+    (void)hipFree(*it);
+    s->allocs.erase(it);
+  }
+  CHK(salloc(s, &s->part, (size_t)chunks * kNParams));
+  s->part_cap = chunks;
   return PLUM_OK;
 }
 
@@ -66,15 +80,20 @@ int sur_train_step(plum_ctx* c, hipStream_t st, int samples, bool gather, bool u
                      s->T, s->N, samples, c->maxm, s->p.target_clip, s->G, s->loss_s);
   const float* w = s->w32;
   const int m = (int)M, chunks = (m + kAtbRows - 1) / kAtbRows;
+  CHK(sur_grad_space(s, std::min(chunks, kGradChunks)));
   const dim3 grid((unsigned)((M + kLinRows - 1) / kLinRows));
   hipLaunchKernelGGL(k_lin_bwd, grid, dim3(kBlock), 0, st, s->D3, w + kOffW3, s->H2, s->D2, m, s->G, w + kOffW4,
                      s->H3);
   hipLaunchKernelGGL(k_lin_bwd, grid, dim3(kBlock), 0, st, s->D2, w + kOffW2, s->H1, s->D1, m, nullptr, nullptr,
                      nullptr);
-  hipLaunchKernelGGL(k_grad_part, dim3(chunks, 4), dim3(kBlock), 0, st, s->X, s->H1, s->H2, s->H3, s->D1, s->D2,
-                     s->D3, s->G, m, s->part);
-  hipLaunchKernelGGL(k_grad_sum, dim3((kNParams + kWave - 1) / kWave), dim3(kBlock), 0, st, s->part, chunks, s->grad,
-                     s->loss_s, samples, s->loss);
+  for (int c0 = 0; c0 < chunks; c0 += kGradChunks) {
+    const int nc = std::min(kGradChunks, chunks - c0);
+    const size_t r0 = (size_t)c0 * kAtbRows, h0 = r0 * kHid;
+    hipLaunchKernelGGL(k_grad_part, dim3(nc, 4), dim3(kBlock), 0, st, s->X + r0 * kDescr, s->H1 + h0, s->H2 + h0,
+                       s->H3 + h0, s->D1 + h0, s->D2 + h0, s->D3 + h0, s->G + r0, m - (int)r0, s->part);
+    hipLaunchKernelGGL(k_grad_sum, dim3((kNParams + kWave - 1) / kWave), dim3(kBlock), 0, st, s->part, nc, c0 > 0,
+                       s->grad, s->loss_s, samples, s->loss);
+  }
   if (update) {
     s->step++;
     hipLaunchKernelGGL(k_adam, dim3(nblocks(kNParams)), dim3(kBlock), 0, st, s->w32, s->grad, s->m1, s->m2, kNParams,

@@ -176,6 +176,12 @@ def test_gradient_tiles(samples, chain_len):
     assert np.max(np.abs(f - _reference_forward(w, x.reshape(-1, 64))[-1])) <= 1e-5 * max(1.0, np.max(np.abs(f)))
 
 
+def test_gradient_in_several_passes():
+    """155 chunks of 128 rows, a second pass of the weight gradients over 27 of
+    them, the last one short."""
+    test_gradient_tiles(300, 33)
+
+
 def _layers(w):
     o = np.cumsum([0, 64 * 128, 128, 128 * 128, 128, 128 * 128, 128, 128, 1])
     w = np.asarray(w, dtype=np.float64)

@@ -43,3 +43,25 @@ def test_growth_buffers_of_alternating_shapes():
             grow(*s)
     assert _used() - before < 16 * MIB, (_used() - before) / MIB
     eng.close()
+
+
+def test_training_workspace():
+    """The FP32 forward allocates the rows and activations (3.3 KB a row, 652
+    MiB), not the partials of a gradient (1.3 KB a row more if every chunk of 128
+    rows had its own, 253 MiB); a gradient of as many rows then adds at most the
+    21 MB of 128 chunks."""
+    sd = systems.config("tiny")
+    xyz, q, ty, ms = systems.build_bulk(1, 200, 0, 40.0, 3)
+    sd.update(xyz=xyz, q=q * 0.0, type=ty, mol_start=ms, box=[40.0] * 3, alpha=0.05)
+    eng = E.Engine(sd)
+    eng.surrogate_enable(train_every=0, train_samples=1, ring=1, r_d=2.5, seed=3)
+    samples, m = 512, eng.max_mol_len()
+    rows = 2 * m * samples
+    x = np.zeros((rows, 64), np.float32)
+    before = _used()
+    eng.surrogate_forward(x, bf16=False)
+    mid = _used()
+    assert mid - before < rows * (64 + 6 * 128 + 2) * 4 + 64 * MIB, (mid - before) / MIB
+    eng.surrogate_gradient(x.reshape(samples, 2 * m, 64), np.zeros(samples), np.full(samples, m, np.int32))
+    assert _used() - mid < 48 * MIB, (_used() - mid) / MIB
+    eng.close()

@@ -283,9 +283,13 @@ void launch_batch(plum_batch* b, hipEvent_t* ev = nullptr) {
   if (ev) (void)hipEventRecord(ev[7], b->st);
 }
 
+// A wave per cell up to 65,536 cells (eight rounds of the waves the chip holds),
+// then as many cells a wave as keep to that number of waves.
 void launch_compact(plum_batch* b) {
-  hipLaunchKernelGGL(k_compact_batch, dim3((b->total_cells + kQWaves - 1) / kQWaves), dim3(kBlock), 0, b->st, b->dG,
-                     b->dD, b->d_cell_off, b->R);
+  const int per = std::max(1, std::min(kWave, (b->total_cells + 65535) / 65536));
+  const int waves = (b->total_cells + per - 1) / per;
+  hipLaunchKernelGGL(k_compact_batch, dim3((waves + kQWaves - 1) / kQWaves), dim3(kBlock), 0, b->st, b->dG, b->dD,
+                     b->d_cell_off, b->R, per);
 }
 
 void launch_status(plum_batch* b) {

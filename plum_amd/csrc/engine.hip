@@ -55,8 +55,11 @@ struct plum_ctx {
   int nmmb = 1;          // blocks of the moved-moved pair work
   int nchunk = 1;        // bead chunks of the S(k) build
   int chunk = 512;
-  int full_groups = 1, full_parts = 1;   // slot groups and cell shares of the full real-space kernel
+  int full_cells = 1, full_groups = 1, full_parts = 1;   // grid of the full real-space kernel
   size_t fpart_cap = 0;  // its partials allocated
+  int *cell_list = nullptr, *cell_cnt = nullptr;   // its cells, where a block takes several (k_cell_scan)
+  int cell_per = 0;      // list entries of a block (0: a block per cell)
+  size_t list_cap = 0;
   int nsplit = 1;        // blocks per real-space query
   double cand = 0;       // expected candidate pair-images per query
   int cell_div = 2;      // cells per search radius and dimension
@@ -160,6 +163,18 @@ void derive_cutoffs(const plum_params& p, plum_info& info) {
   for (int i = 0; i < 3; i++) info.repl_cell[i] = (int)ceil(sqrt(repl_cutoff) * box[i] / (2 * kPi));
 }
 
+// Most blocks of the full real-space kernel with a block per cell, and blocks
+// where each takes several.
+constexpr int kFullBlocks = 65536, kListBlocks = 8192;
+
+// The cells of each block of the full real-space kernel (listed by scan_cells).
+CellList full_cells(const plum_ctx* c) { return CellList{c->cell_list, c->cell_cnt, c->cell_per, c->full_cells}; }
+
+// Partials of the full real-space kernel.
+size_t full_partials(const plum_ctx* c) {
+  return (size_t)c->full_cells * c->full_groups * c->full_parts * kQWaves;
+}
+
 // Builds the cell list from the current device positions, each cell's beads in
 // index order (k_cell_*).  The largest count comes back to the host, which
 // sizes the slots.
@@ -184,14 +199,31 @@ int build_cells(plum_ctx* c, int min_cap) {
     CHK(dalloc(c, &c->d.ctype, slots));
     c->g.cap = cap;
   }
-  // from-scratch real space: block (cell, group of kCluster slots, share of
-  // the query's cells).  Groups for the counts the list holds now (a fuller
-  // cell's blocks take several), shares where few cells hold many beads
+  // from-scratch real space: block (residue of the cells, group of kCluster
+  // slots, share of the query's cells).  Groups for the counts the list holds
+  // now (a fuller cell's blocks take several), shares where few cells hold many
+  // beads.  A block takes one cell while that needs no more than kFullBlocks
+  // blocks and, past 1,024, two blocks a bead; else the cells are listed without
+  // the empty ones and dealt to fewer blocks: a block for each of 2.1 million
+  // cells, and its partials in the final sum, took 2.1 ms for 800 beads, 63 us now.
   c->full_groups = std::max(1, std::min((maxc + kCluster - 1) / kCluster, 65535));
-  const long long blocks = (long long)g.ncell * c->full_groups;
+  const long long most = std::max(1024LL, 2LL * g.n);
+  c->full_cells = g.ncell;
+  if (g.ncell > most || (long long)g.ncell * c->full_groups > kFullBlocks)
+    c->full_cells = (int)std::min({(long long)g.ncell, most, std::max(1024LL, (long long)kListBlocks / c->full_groups)});
+  const long long blocks = (long long)c->full_cells * c->full_groups;
   c->full_parts = (int)std::max(1LL, std::min<long long>(kMaxQBlock, std::min<long long>(
                       4096 / blocks, (long long)(c->cand / kQShare))));
-  const size_t fp = (size_t)blocks * c->full_parts * kQWaves;
+  c->cell_per = c->full_cells < g.ncell ? (g.ncell + c->full_cells - 1) / c->full_cells : 0;
+  const size_t nl = (size_t)c->full_cells * (c->cell_per + 1);
+  if (c->cell_per && nl > c->list_cap) {
+    c->list_cap = 0;
+    dfree(c, &c->cell_list);
+    CHK(dalloc(c, &c->cell_list, nl));
+    c->list_cap = nl;
+  }
+  c->cell_cnt = c->cell_per ? c->cell_list + (size_t)c->full_cells * c->cell_per : nullptr;
+  const size_t fp = full_partials(c);
   if (fp > c->fpart_cap) {
     CHK(dalloc(c, &c->d.fpart, fp));
     c->fpart_cap = fp;
@@ -260,8 +292,10 @@ constexpr int kFullSmall = 128;   // blocks of k_full_small
 // dipole state and the per-molecule spring cache are reset to it.
 int run_full(plum_ctx* c, int set_running, double out[8]) {
   const Geo& g = c->g;
-  hipLaunchKernelGGL(k_full_real, dim3(g.ncell, c->full_groups, c->full_parts), dim3(kBlock), 0, c->st, g, c->d,
-                     c->full_parts);
+  const CellList cl = full_cells(c);
+  if (cl.per) hipLaunchKernelGGL(k_cell_scan, dim3(c->full_cells), dim3(kBlock), 0, c->st, g, c->d, cl);
+  hipLaunchKernelGGL(k_full_real, dim3(c->full_cells, c->full_groups, c->full_parts), dim3(kBlock), 0, c->st, g, c->d,
+                     cl, c->full_parts);
   const bool ksp = g.use_ewald && g.n_kh > 0;
   if (ksp) {
     // by tiles where a step of four beads' tables fits the LDS stage
@@ -273,10 +307,9 @@ int run_full(plum_ctx* c, int set_running, double out[8]) {
     hipLaunchKernelGGL(k_full_sk_reduce, dim3(c->nkb_full), dim3(kBlock), 0, c->st, g, c->d, c->nchunk,
                        c->epart_k);
   }
-  hipLaunchKernelGGL(k_full_small, dim3(kFullSmall), dim3(kBlock), 0, c->st, g, c->d, c->opart);
-  hipLaunchKernelGGL(k_full_final, dim3(1), dim3(kFinalThreads), 0, c->st, g, c->d,
-                     g.ncell * c->full_groups * c->full_parts * kQWaves, ksp ? c->nkb_full : 0, kFullSmall,
-                     c->epart_k, c->opart, set_running);
+  hipLaunchKernelGGL(k_full_small, dim3(kFullSmall), dim3(kBlock), 0, c->st, g, c->d, (int)full_partials(c), c->opart);
+  hipLaunchKernelGGL(k_full_final, dim3(1), dim3(kFinalThreads), 0, c->st, g, c->d, ksp ? c->nkb_full : 0,
+                     kFullSmall, c->epart_k, c->opart, set_running);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(c->h_ctl, c->d.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
@@ -591,7 +624,7 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
   ALLOC(d.part_k, c->nkb); ALLOC(d.part_r, (size_t)kMaxProp * std::max(query_blocks(maxm, kMaxQBlock) * kQWaves, 2 * maxm * kMaxSplit));
   ALLOC(d.part_mm, (size_t)kMaxProp * c->nmmb);
   ALLOC(d.sk_part, (size_t)c->nchunk * std::max(1, g.n_kh));
-  ALLOC(c->epart_k, c->nkb_full); ALLOC(c->opart, 4 * kFullSmall); ALLOC(c->d_max, 1);
+  ALLOC(c->epart_k, c->nkb_full); ALLOC(c->opart, kSmallSums * kFullSmall); ALLOC(c->d_max, 1);
   ALLOC(d.chain_ids, n_mols); ALLOC(d.ion_ids, n_mols);
   {
     // move record of the host path: header, then the bead indices

@@ -85,28 +85,80 @@ __global__ __launch_bounds__(kBlock) void k_cell_order(Geo g, Dev d) {
 // with weight 1/2), which costs more distance tests than one thread per slot
 // that walks the cells around it, and none of its waits: 2.6 ms for 40,000
 // beads, and 8.5 ms for 3,200 beads in a box of 1.4 r_c, that way.
-// Block (cell, slot group, share of the query's cells).
+// Block (cells, slot group, share of the query's cells); its cells are cell
+// blockIdx.x, or where most cells are empty the ones scan_cells listed for it.
+struct CellList {
+  int *cell, *count;
+  int per;      // list entries of a block (0: a block per cell)
+  int blocks;   // blocks that share the cells
+};
+
+// List of block b: the occupied ones of cells b, b + blocks, .. in that order,
+// 256 counts read at a time (one block).
+__device__ void scan_cells(const Geo& g, const Dev& d, const CellList& cl, int b) {
+  __shared__ int s_wave[kQWaves];
+  const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
+  int* out = cl.cell + (size_t)b * cl.per;
+  int n = 0;
+  for (int base = 0; base < cl.per; base += kBlock) {
+    const long long c = b + (long long)(base + threadIdx.x) * cl.blocks;
+    const bool has = c < g.ncell && d.ccount[c] > 0;
+    const unsigned long long m = __ballot(has);
+    __syncthreads();   // the last counts are read
+    if (lane == 0) s_wave[wv] = __popcll(m);
+    __syncthreads();
+    int at = n + lanes_below(m);
+#pragma unroll
+    for (int w = 0; w < kQWaves; w++) {
+      if (w < wv) at += s_wave[w];
+      n += s_wave[w];
+    }
+    if (has) out[at] = (int)c;
+  }
+  if (threadIdx.x == 0) cl.count[b] = n;
+}
+
+__global__ __launch_bounds__(kBlock) void k_cell_scan(Geo g, Dev d, CellList cl) { scan_cells(g, d, cl, blockIdx.x); }
+
+// Sum over every bead pair of what real_query_cluster<0, MODE> evaluates, one
+// partial per wave.  Of the blocks of 40,000 beads 85% lie past their cell's
+// count, so what such a block does counts: with the set-up of the queries before
+// the test 232 us, with it after 206.
+template <int MODE>
+__device__ __forceinline__ void all_pairs(const Geo& g, const Dev& d, const CellList& cl, int nparts,
+                                          QueryShare<0, MODE>& sm, double2* out,
+                                          const StretchArgs& st = StretchArgs{nullptr, nullptr, 0, 0}) {
+  const int lane = threadIdx.x % kWave;
+  const size_t b = ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+  const int nc = cl.per ? uload(cl.count + blockIdx.x) : (int)blockIdx.y * kCluster < uload(d.ccount + blockIdx.x);
+  if (nc == 0) {   // before the set-up of the queries
+    if (threadIdx.x < kQWaves) out[b * kQWaves + threadIdx.x] = make_double2(0, 0);
+    return;
+  }
+  double elj = 0, ere = 0;
+  for (int i = 0; i < nc; i++) {
+    const int cell = cl.per ? uload(cl.cell + (size_t)blockIdx.x * cl.per + i) : (int)blockIdx.x;
+    const int cnt = uload(d.ccount + cell);
+    for (int s0 = blockIdx.y * kCluster; s0 < cnt; s0 += gridDim.y * kCluster) {
+      const int s = s0 + lane % kCluster;
+      const size_t si = (size_t)cell * g.cap + min(s, cnt - 1);
+      const int own = s < cnt ? d.cbead[si] : -1;
+      if (!__ballot(own >= 0)) continue;
+      const double2 e = real_query_cluster<0, MODE>(g, d, d.cpos[si], d.ctype[si], own >= 0, own, 0, -1, blockIdx.z,
+                                                    nparts, sm, st);
+      elj += e.x;
+      ere += e.y;
+      __syncthreads();   // the next group rewrites the points
+    }
+  }
+  if (lane == 0) out[b * kQWaves + threadIdx.x / kWave] = make_double2(elj, ere);
+}
+
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_full_real(Geo g, Dev d,
+                                                                                              CellList cl,
                                                                                               int nparts) {
   __shared__ QueryShare<0, Q_ALL> sm;
-  const int cell = blockIdx.x, part = blockIdx.z, lane = threadIdx.x % kWave;
-  const int cnt = d.ccount[cell];
-  double elj = 0, ere = 0;
-  for (int s0 = blockIdx.y * kCluster; s0 < cnt; s0 += gridDim.y * kCluster) {
-    const int s = s0 + lane % kCluster;
-    const size_t si = (size_t)cell * g.cap + min(s, cnt - 1);
-    const int own = s < cnt ? d.cbead[si] : -1;
-    if (!__ballot(own >= 0)) continue;
-    const double2 e = real_query_cluster<0, Q_ALL>(g, d, d.cpos[si], d.ctype[si], own >= 0, own, 0, -1, part, nparts,
-                                                  sm);
-    elj += e.x;
-    ere += e.y;
-    __syncthreads();   // the next group rewrites the points
-  }
-  if (lane == 0) {
-    const size_t b = ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
-    d.fpart[b * kQWaves + threadIdx.x / kWave] = make_double2(elj, ere);
-  }
+  all_pairs<Q_ALL>(g, d, cl, nparts, sm, d.fpart);
 }
 
 // S(k) from scratch, bead chunk `blockIdx.y`: direct FP64 sincos per (k,
@@ -243,10 +295,13 @@ __device__ double molecule_spring_wave(const Geo& g, const Dev& d, int a, int b)
   return acc;
 }
 
-// Springs per molecule (a wave each, grid-stride) and wall, self and dipole
-// sums over the beads: block partials opart[4 b ..] = springs, wall, self,
-// M_z.  (One block over all molecules in turn: 3.7 ms for 20,200 molecules.)
-__global__ __launch_bounds__(kBlock) void k_full_small(Geo g, Dev d, double* opart) {
+// Springs per molecule (a wave each, grid-stride), wall, self and dipole sums
+// over the beads and the sum of k_full_real's partials: block partials opart[6 b
+// ..] = springs, wall, self, M_z, LJ, real space.  (One block over all molecules
+// in turn: 3.7 ms for 20,200 molecules; one block over 68,000 partials: 25 us of
+// the 32 of k_full_final.)
+constexpr int kSmallSums = 6;
+__global__ __launch_bounds__(kBlock) void k_full_small(Geo g, Dev d, int nrealp, double* opart) {
   __shared__ double sh[kBlock / kWave];
   const int lane = threadIdx.x % kWave;
   double eb = 0;
@@ -266,38 +321,38 @@ __global__ __launch_bounds__(kBlock) void k_full_small(Geo g, Dev d, double* opa
     es += g.self_coef * qi * qi;
     mz += qi * d.z[i];
   }
-  const double v4[4] = {eb, ew, es, mz};
+  double el = 0, er = 0;
+#pragma unroll 4
+  for (int b = blockIdx.x * kBlock + threadIdx.x; b < nrealp; b += gridDim.x * kBlock) {
+    const double2 e = d.fpart[b];
+    el += e.x;
+    er += e.y;
+  }
+  const double v[kSmallSums] = {eb, ew, es, mz, el, er};
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const double t = block_sum<kBlock>(v4[k], sh);
-    if (threadIdx.x == 0) opart[4 * blockIdx.x + k] = t;
+  for (int k = 0; k < kSmallSums; k++) {
+    const double t = block_sum<kBlock>(v[k], sh);
+    if (threadIdx.x == 0) opart[kSmallSums * blockIdx.x + k] = t;
   }
 }
 
 // The final reduction of all from-scratch partials into the control block.
 constexpr int kFinalThreads = 1024;
-__global__ __launch_bounds__(kFinalThreads) void k_full_final(Geo g, Dev d, int nrealp, int nkb, int nob,
-                                                              const double* epart_k, const double* opart,
-                                                              int set_running) {
+__global__ __launch_bounds__(kFinalThreads) void k_full_final(Geo g, Dev d, int nkb, int nob, const double* epart_k,
+                                                              const double* opart, int set_running) {
   __shared__ double sh[kFinalThreads / kWave];
   Ctl* C = d.ctl;
-  double vl = 0, vr = 0, vk = 0, vo[4] = {0, 0, 0, 0};
-#pragma unroll 4
-  for (int b = threadIdx.x; b < nrealp; b += kFinalThreads) {
-    const double2 e = d.fpart[b];
-    vl += e.x;
-    vr += e.y;
-  }
+  double vk = 0, vo[kSmallSums] = {0, 0, 0, 0, 0, 0};
   for (int b = threadIdx.x; b < nkb; b += kFinalThreads) vk += epart_k[b];
   for (int b = threadIdx.x; b < nob; b += kFinalThreads)
 #pragma unroll
-    for (int k = 0; k < 4; k++) vo[k] += opart[4 * b + k];
+    for (int k = 0; k < kSmallSums; k++) vo[k] += opart[kSmallSums * b + k];
   const double ebt = block_sum<kFinalThreads>(vo[0], sh);
   const double ewt = block_sum<kFinalThreads>(vo[1], sh);
   const double est = block_sum<kFinalThreads>(vo[2], sh);
   const double mzt = block_sum<kFinalThreads>(vo[3], sh);
-  const double lt = block_sum<kFinalThreads>(vl, sh);
-  const double rt = block_sum<kFinalThreads>(vr, sh);
+  const double lt = block_sum<kFinalThreads>(vo[4], sh);
+  const double rt = block_sum<kFinalThreads>(vo[5], sh);
   const double kt = block_sum<kFinalThreads>(vk, sh);
   if (threadIdx.x == 0) {
     double f[8] = {0, 0, 0, 0, 0, 0, 0, 0};

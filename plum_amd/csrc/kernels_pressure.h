@@ -13,35 +13,65 @@ namespace plum {
 
 constexpr double kDz = 0.00001;   // utilities/constants.h:55
 
-// Stretched z of every bead (zs), its displacement (dz), and the displacement
-// of the image the cell list holds (dw).  A bead that moves with its molecule
-// sums the molecule's centre of mass itself, in the reference's bead order
-// (beads of the spring potential do not: the common case is one pass over the
-// beads).
-__global__ void k_vp_scale(Geo g, Dev d, double* zs, double* dz, double* dw) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= g.n) return;
+// Stretched z of bead j.  A bead that moves with its molecule sums the
+// molecule's centre of mass itself, in the reference's bead order (beads of the
+// spring potential do not).
+__device__ double vp_z(const Geo& g, const Dev& d, int j) {
   const double Lz = g.Lsim[2], z = d.z[j];
-  double zn;
-  if (g.use_bond && d.wall[d.type[j]].kind == 0) {
-    zn = z * (1.0 + kDz / Lz);
-  } else {
-    const int m = d.mol_of[j], a = d.mol_start[m], b = d.mol_start[m + 1];
-    const int k0 = d.wall[d.type[a]].kind;
-    double dcz = k0 == 2 ? kDz : 0.0;
-    if (k0 == 0) {
-      double com = 0;
-      for (int i = a; i < b; i++) com += d.z[i];
-      com /= (b - a);
-      dcz = kDz * (com / Lz);
-    }
-    zn = z + dcz;
+  if (g.use_bond && d.wall[d.type[j]].kind == 0) return z * (1.0 + kDz / Lz);
+  const int m = d.mol_of[j], a = d.mol_start[m], b = d.mol_start[m + 1];
+  const int k0 = d.wall[d.type[a]].kind;
+  double dcz = k0 == 2 ? kDz : 0.0;
+  if (k0 == 0) {
+    double com = 0;
+    for (int i = a; i < b; i++) com += d.z[i];
+    com /= (b - a);
+    dcz = kDz * (com / Lz);
   }
-  // the displacement of the rounded z', exactly: z and z' are close
-  const double disp = zn - z;
-  zs[j] = zn;
-  dz[j] = disp;
-  dw[j] = disp - rint((z - wrap_coord(z, g.L[2], g.inv_L[2])) * g.inv_L[2]) * kDz;
+  return z + dcz;
+}
+
+// Everything that goes over the beads, in one launch (a sample of a small
+// system is launches): stretched z (zs), the displacement of the image that the
+// cell list holds (dw), and block partials part[4 b ..] of the walls (mobile
+// beads), the springs (each bond's change) and the dipole moments before and
+// after.  Blocks past kVpBeadBlocks list the cells of k_vp_pairs.
+constexpr int kVpBeadBlocks = 128;
+__global__ __launch_bounds__(kBlock) void k_vp_beads(Geo g, Dev d, CellList cl, double* zs, double* dw, int phantom,
+                                                     double* part) {
+  __shared__ double sh[kBlock / kWave];
+  if (blockIdx.x >= kVpBeadBlocks) {
+    scan_cells(g, d, cl, blockIdx.x - kVpBeadBlocks);
+    return;
+  }
+  Geo gs = g;
+  gs.Lsim[2] = g.Lsim[2] + kDz;
+  double ew = 0, eb = 0, mo = 0, mn = 0;
+  for (int j = blockIdx.x * kBlock + threadIdx.x; j < g.n; j += kVpBeadBlocks * kBlock) {
+    const int m = d.mol_of[j];
+    const double z = d.z[j], zn = vp_z(g, d, j);
+    // the displacement of the rounded z', exactly: z and z' are close
+    const double disp = zn - z;
+    zs[j] = zn;
+    dw[j] = disp - rint((z - wrap_coord(z, g.L[2], g.inv_L[2])) * g.inv_L[2]) * kDz;
+    if (g.use_ext && m >= phantom) {
+      const WallType w = d.wall[d.type[j]];
+      ew += wall_energy(zn, w, gs) - wall_energy(z, w, g);
+    }
+    mo += d.q[j] * z;
+    mn += d.q[j] * zn;
+    if (g.use_bond && j + 1 < d.mol_start[m + 1]) {
+      const double dx = d.x[j] - d.x[j + 1], dy = d.y[j] - d.y[j + 1], dz = z - d.z[j + 1];
+      const double disp1 = vp_z(g, d, j + 1) - d.z[j + 1];
+      eb += spring_energy(g, dx, dy, dz + (disp - disp1)) - spring_energy(g, dx, dy, dz);
+    }
+  }
+  const double v4[4] = {ew, eb, mo, mn};
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const double t = block_sum<kBlock>(v4[k], sh);
+    if (threadIdx.x == 0) part[4 * blockIdx.x + k] = t;
+  }
 }
 
 // Ewald real-space and LJ pairs, stretched minus current: the from-scratch
@@ -50,27 +80,9 @@ __global__ void k_vp_scale(Geo g, Dev d, double* zs, double* dz, double* dw) {
 // 2 bead pairs, the pair index decoded per pair and both image sums explicit,
 // 250 us (432 us with all 27 images), quadratic in N.
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_vp_pairs(
-    Geo g, Dev d, const double* __restrict__ dw, int phantom, int nparts, double2* part_out) {
+    Geo g, Dev d, CellList cl, const double* __restrict__ dw, int phantom, int nparts, double2* part_out) {
   __shared__ QueryShare<0, Q_STRETCH> sm;
-  const StretchArgs st = {dw, d.mol_of, kDz, phantom};
-  const int cell = blockIdx.x, part = blockIdx.z, lane = threadIdx.x % kWave;
-  const int cnt = d.ccount[cell];
-  double dlj = 0, del = 0;
-  for (int s0 = blockIdx.y * kCluster; s0 < cnt; s0 += gridDim.y * kCluster) {
-    const int s = s0 + lane % kCluster;
-    const size_t si = (size_t)cell * g.cap + min(s, cnt - 1);
-    const int own = s < cnt ? d.cbead[si] : -1;
-    if (!__ballot(own >= 0)) continue;
-    const double2 e = real_query_cluster<0, Q_STRETCH>(g, d, d.cpos[si], d.ctype[si], own >= 0, own, 0, -1, part,
-                                                       nparts, sm, st);
-    dlj += e.x;
-    del += e.y;
-    __syncthreads();   // the next group rewrites the points
-  }
-  if (lane == 0) {
-    const size_t b = ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
-    part_out[b * kQWaves + threadIdx.x / kWave] = make_double2(dlj, del);
-  }
+  all_pairs<Q_STRETCH>(g, d, cl, nparts, sm, part_out, StretchArgs{dw, d.mol_of, kDz, phantom});
 }
 
 // k space of the stretch, per half-space l vector of the current or the
@@ -179,35 +191,6 @@ __global__ __launch_bounds__(kBlock) void k_vp_dsk_energy(const double2* __restr
   }
   const double r = block_sum<kBlock>(e, sh);
   if (threadIdx.x == 0) epart[blockIdx.x] = r;
-}
-
-// Walls (mobile beads), springs (each bond's change) and the dipole moments
-// before and after: block partials part[4 b ..].
-__global__ __launch_bounds__(kBlock) void k_vp_small(Geo g, Dev d, const double* __restrict__ zs,
-                                                     const double* __restrict__ disp, int phantom, double* part) {
-  __shared__ double sh[kBlock / kWave];
-  Geo gs = g;
-  gs.Lsim[2] = g.Lsim[2] + kDz;
-  double ew = 0, eb = 0, mo = 0, mn = 0;
-  for (int j = blockIdx.x * kBlock + threadIdx.x; j < g.n; j += gridDim.x * kBlock) {
-    const int m = d.mol_of[j];
-    if (g.use_ext && m >= phantom) {
-      const WallType w = d.wall[d.type[j]];
-      ew += wall_energy(zs[j], w, gs) - wall_energy(d.z[j], w, g);
-    }
-    mo += d.q[j] * d.z[j];
-    mn += d.q[j] * zs[j];
-    if (g.use_bond && j + 1 < d.mol_start[m + 1]) {
-      const double dx = d.x[j] - d.x[j + 1], dy = d.y[j] - d.y[j + 1], dz = d.z[j] - d.z[j + 1];
-      eb += spring_energy(g, dx, dy, dz + (disp[j] - disp[j + 1])) - spring_energy(g, dx, dy, dz);
-    }
-  }
-  const double v4[4] = {ew, eb, mo, mn};
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const double t = block_sum<kBlock>(v4[k], sh);
-    if (threadIdx.x == 0) part[4 * blockIdx.x + k] = t;
-  }
 }
 
 // Every partial into out[0..5] = Ewald pairs, LJ pairs, walls, springs,

@@ -2,8 +2,8 @@
 // of the pressure estimator.  Included once, at the end of engine.hip.
 
 struct VpHost {
-  // stretched z per bead, its displacement, that of the image in the cell list
-  double *zs = nullptr, *dz = nullptr, *dw = nullptr;
+  // stretched z per bead, displacement of its image in the cell list
+  double *zs = nullptr, *dw = nullptr;
   double2* ppart = nullptr;   // pair partials (LJ, Ewald) per wave
   size_t pcap = 0;            // their number allocated
   double* opart = nullptr;    // walls, springs, dipole partials
@@ -83,9 +83,8 @@ int vp_setup(plum_ctx* c) {
   h->chunk = std::max(16, (g.n + want - 1) / want);
   h->nchunk = (g.n + h->chunk - 1) / h->chunk;
   CHK(dalloc(c, &h->zs, (size_t)g.n));
-  CHK(dalloc(c, &h->dz, (size_t)g.n));
   CHK(dalloc(c, &h->dw, (size_t)g.n));
-  CHK(dalloc(c, &h->opart, 4 * (size_t)kFullSmall));
+  CHK(dalloc(c, &h->opart, 4 * (size_t)kVpBeadBlocks));
   CHK(dalloc(c, &h->kl_u, (size_t)nk));
   CHK(dalloc(c, &h->c_old, (size_t)nk));
   CHK(dalloc(c, &h->c_new, (size_t)nk));
@@ -121,15 +120,16 @@ extern "C" int plum_vp_sample(plum_ctx* c, int phantom, plum_vp* out) {
   }
   VpHost* h = c->vp;
   const Geo& g = c->g;
-  const size_t np = (size_t)g.ncell * c->full_groups * c->full_parts * kQWaves;
+  const size_t np = full_partials(c);
   if (np > h->pcap) {
     CHK(dalloc(c, &h->ppart, np));
     h->pcap = np;
   }
-  hipLaunchKernelGGL(k_vp_scale, dim3((g.n + kBlock - 1) / kBlock), dim3(kBlock), 0, c->st, g, c->d, h->zs,
-                     h->dz, h->dw);
-  hipLaunchKernelGGL(k_vp_pairs, dim3(g.ncell, c->full_groups, c->full_parts), dim3(kBlock), 0, c->st, g, c->d, h->dw,
-                     phantom, c->full_parts, h->ppart);
+  const CellList cl = full_cells(c);
+  hipLaunchKernelGGL(k_vp_beads, dim3(kVpBeadBlocks + (cl.per ? cl.blocks : 0)), dim3(kBlock), 0, c->st, g, c->d, cl,
+                     h->zs, h->dw, phantom, h->opart);
+  hipLaunchKernelGGL(k_vp_pairs, dim3(c->full_cells, c->full_groups, c->full_parts), dim3(kBlock), 0, c->st, g, c->d,
+                     cl, h->dw, phantom, c->full_parts, h->ppart);
   int nkb = 0;
   if (g.use_ewald && h->nk_u > 0) {
     nkb = h->nkb;
@@ -145,10 +145,8 @@ extern "C" int plum_vp_sample(plum_ctx* c, int phantom, plum_vp* out) {
                          h->c_old, h->c_new, h->dc, h->ekpart);
     }
   }
-  hipLaunchKernelGGL(k_vp_small, dim3(kFullSmall), dim3(kBlock), 0, c->st, g, c->d, h->zs, h->dz, phantom,
-                     h->opart);
   hipLaunchKernelGGL(k_vp_final, dim3(1), dim3(kFinalThreads), 0, c->st, g, h->ppart, (int)np, h->ekpart, nkb,
-                     h->opart, kFullSmall, h->out);
+                     h->opart, kVpBeadBlocks, h->out);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(h->h_out, h->out, 6 * sizeof(double), hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));

@@ -116,6 +116,31 @@ def test_from_scratch_energy_and_cell_order(n_chains, chain_len, salt, L, alpha,
     _full_matches(eng, orc)
 
 
+@pytest.mark.parametrize("L,cell_div", [(100.0, 2), (60.0, 2), (100.0, 1)])
+def test_mostly_empty_cells(L, cell_div):
+    """Neutral chains in a box of up to 512,000 cells, several hundred to a block
+    of the from-scratch sums and several to a wave of the compaction: energy
+    and pressure sample against the oracle, fresh and after moves (tombstones,
+    two compactions)."""
+    from plum_amd import host
+    sd = systems.config("tiny")
+    xyz, q, ty, ms = host.synth_system(5, 40, 0, 0, [L, L, L], 5, bead_q=0.0)
+    xyz[80:120] = xyz[:40] + [0.4, 0.4, 0.4]     # two chains in the same cells
+    sd.update(xyz=xyz, q=q, type=ty, mol_start=ms, box=[L, L, L], use_ewald=0)
+    eng = E.Engine(sd, cell_div=cell_div)
+    for moves in (0, 900):
+        if moves:
+            eng.mc_run(moves, sd["move_prob"], move_size=1.0, seed=3)
+        orc = O.Oracle(dict(sd, xyz=eng.positions()))
+        _full_matches(eng, orc)
+        got, ref = eng.vp_sample(), orc.vp_sample(0)
+        scale = sum(abs(v) for v in orc.energy_full().values())
+        for k in ("lj", "bond", "dU"):
+            assert abs(got[k] - ref[k]) <= 1e-14 * scale, (k, got[k], ref[k], scale)
+        run, full = eng.totals(), eng.energy_full()
+        assert abs(run["lj"] - full["lj"]) <= 1e-10 * scale
+
+
 def test_spring_energy_has_one_set_of_bits():
     """The molecule springs of the from-scratch pass equal the trial path's
     bit for bit: a move that changes nothing has a spring dE of exactly 0."""

@@ -1,15 +1,18 @@
-"""The FP64 erfc of the pair kernels (erfc_nodes in engine_dev.h): Taylor
+"""The FP64 erfc of the pair kernels (erfc_from_node in engine_dev.h): Taylor
 series about tabulated nodes x_i = i/128 with the Hermite-polynomial
-derivatives of erfc (Abramowitz & Stegun 7.1.19), eight terms.
+derivatives of erfc (Abramowitz & Stegun 7.1.19), regrouped by powers of t^2;
+and their square root and reciprocal (sqrt_rsqrt).
 
-The same steps in double precision are checked here against erfc at 40
-digits (mpmath): the method's error over [0, 8) is a few ulp, so the device
-real-space terms carry FP64 rounding only.  The device code itself is pinned
-end to end by the GPU parity tests (every real-space dE within 1e-10 of the
-oracle's libm erfc).  The FP32 pair path's erfc_nodes32 (the same nodes in
-float32, four terms) is checked the same way at float32 precision.
+The device's steps, fused operations rounded once, are checked here against
+40 digits (mpmath): erfc over [0, 8) is within a few ulp, r and 1 / r within
+one, so the device real-space terms carry FP64 rounding only.  The device code
+itself is pinned end to end by the GPU parity tests (every real-space dE within
+1e-10 of the oracle's libm erfc).  The FP32 pair path's erfc_from_node32 (the
+same nodes in float32, four terms) is checked the same way at float32
+precision.
 """
 import math
+from fractions import Fraction
 
 import numpy as np
 import pytest
@@ -29,6 +32,17 @@ def _nodes():
     return out
 
 
+def _fma(a, b, c):
+    return float(Fraction(a) * Fraction(b) + Fraction(c))
+
+
+def _horner(y, first, *rest):
+    p = first
+    for c in rest:
+        p = _fma(p, y, c)
+    return p
+
+
 def _erfc_nodes(x, nodes):
     if not x < X_MAX:
         return 0.0
@@ -36,18 +50,39 @@ def _erfc_nodes(x, nodes):
     xi = i * (1.0 / PER_UNIT)
     t = x - xi
     a, e = nodes[i]
-    m2x = -2.0 * xi
-    qm, q = 1.0, m2x
-    w = t
-    s = w
-    w *= t * 0.5
-    s += q * w
-    for n in range(1, 7):
-        qn = m2x * q - (2.0 * n) * qm
-        qm, q = q, qn
-        w *= t * (1.0 / (n + 2))
-        s += q * w
-    return a - e * s
+    y, t2 = -2.0 * xi * t, t * t
+    p0 = _horner(y, 1 / 40320.0, 1 / 5040.0, 1 / 720.0, 1 / 120.0, 1 / 24.0, 1 / 6.0, 0.5)
+    p1 = _horner(y, 1 / 960.0, 1 / 168.0, 1 / 36.0, 0.1, 0.25, 1 / 3.0)
+    p2 = _horner(y, 1 / 14.0, 1 / 6.0, 0.2)
+    r = _fma(t2, _fma(0.5 * t2, p2, -p1), p0 * y)
+    return _fma(-e, _fma(t, r, t), a)
+
+
+def _sqrt_rsqrt(r2, y):
+    """r and 1 / r from the estimate y of 1 / r."""
+    g, h = r2 * y, 0.5 * y
+    for _ in range(2):
+        e = _fma(-h, g, 0.5)
+        g, h = _fma(g, e, g), _fma(h, e, h)
+    g = _fma(_fma(-g, g, r2), h, g)
+    z = h + h
+    return g, _fma(_fma(-g, z, 1.0), z, z)
+
+
+def test_square_root_and_reciprocal_within_an_ulp():
+    """Both results, from estimates as far off as 2^-15 either way (the hardware
+    estimate of 64-bit reciprocal square roots is good to some 2^-23), over the
+    squared distances of a query: 1e-32 (beads that miss each other by rounding)
+    to 1e6."""
+    mpmath.mp.dps = 40
+    rng = np.random.default_rng(5)
+    worst = 0.0
+    for r2 in np.concatenate([10.0 ** rng.uniform(-32, 6, 1500), rng.uniform(0.5, 400.0, 1500), [1.0, 4.0, 2.0]]):
+        ref = mpmath.sqrt(mpmath.mpf(float(r2)))
+        for off in (2.0 ** -15, -2.0 ** -15, 2.0 ** -23 * rng.uniform(-1, 1)):
+            r, rinv = _sqrt_rsqrt(float(r2), float((1 + off) / ref))
+            worst = max(worst, abs(float((r - ref) / ref)), abs(float((rinv - 1 / ref) * ref)))
+    assert worst <= 2.0 ** -52, worst * 2.0 ** 52
 
 
 def test_erfc_nodes_within_four_ulp_on_0_to_8():
@@ -73,7 +108,7 @@ def test_erfc_nodes_exact_at_the_nodes_and_zero_beyond_range():
 
 
 def _erfc_nodes32(x, nodes32):
-    """erfc_nodes32 (engine_dev.h) step by step in float32."""
+    """erfc_from_node32 (engine_dev.h) step by step in float32."""
     f = np.float32
     x = f(x)
     if not x < f(X_MAX):

@@ -85,6 +85,36 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
   all_pairs<Q_STRETCH>(g, d, cl, nparts, sm, part_out, StretchArgs{dw, d.mol_of, kDz, phantom});
 }
 
+// The same for up to kVpDirect beads without Ewald, over the bead pairs a < b in
+// turn: a query is some 15 us of dependent steps however few its candidates, and
+// LJ has one image a pair.  A sample of neutral chains, pairs / queries: 27 / 41
+// us at 100 beads, 32 / 57 at 1,020, 45 / 66 at 2,000.
+constexpr int kVpDirect = 2048;
+__global__ __launch_bounds__(kBlock) void k_vp_pairs_lj(Geo g, Dev d, const double* __restrict__ zs, int phantom,
+                                                        double2* part_out) {
+  const long long npair = (long long)g.n * g.n;
+  const double cw = sqrt(g.lj2_max) + kStretchMargin, lj2 = cw * cw;
+  double dlj = 0;
+  for (long long p = blockIdx.x * (long long)kBlock + threadIdx.x; p < npair; p += (long long)gridDim.x * kBlock) {
+    const int a = (int)(p / g.n), b = (int)(p - (long long)a * g.n);
+    if (b <= a || !g.use_pair || d.mol_of[a] < phantom || d.mol_of[b] < phantom) continue;
+    double s[3] = {d.x[b] - d.x[a], d.y[b] - d.y[a], d.z[b] - d.z[a]}, m[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      m[k] = k < g.npbc ? rint(s[k] * g.inv_L[k]) : 0.0;
+      s[k] -= m[k] * g.L[k];
+    }
+    const double r2 = s[0] * s[0] + s[1] * s[1] + s[2] * s[2];
+    if (!(r2 < lj2)) continue;
+    const double sn = s[2] + ((zs[b] - d.z[b]) - (zs[a] - d.z[a]) - m[2] * kDz);
+    const LJPair lp = d.lj[d.type[a] * g.n_types + d.type[b]];
+    dlj += lj_energy(sqrt(s[0] * s[0] + s[1] * s[1] + sn * sn), lp) - lj_energy(sqrt(r2), lp);
+  }
+  dlj = wave_sum(dlj);
+  if (threadIdx.x % kWave == 0)
+    part_out[(size_t)blockIdx.x * kQWaves + threadIdx.x / kWave] = make_double2(dlj, 0.0);
+}
+
 // k space of the stretch, per half-space l vector of the current or the
 // stretched k list (their union): S_c(k) of the three bead sets the pair rule
 // separates -- mobile beads, the first and the second half of the phantom

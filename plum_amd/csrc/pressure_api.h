@@ -120,16 +120,22 @@ extern "C" int plum_vp_sample(plum_ctx* c, int phantom, plum_vp* out) {
   }
   VpHost* h = c->vp;
   const Geo& g = c->g;
-  const size_t np = full_partials(c);
+  const bool direct = !g.use_ewald && g.n <= kVpDirect;
+  const int dblocks = (int)std::min<long long>(512, ((long long)g.n * g.n + kBlock - 1) / kBlock);
+  const size_t np = direct ? (size_t)dblocks * kQWaves : full_partials(c);
   if (np > h->pcap) {
     CHK(dalloc(c, &h->ppart, np));
     h->pcap = np;
   }
-  const CellList cl = full_cells(c);
+  CellList cl = full_cells(c);
+  if (direct) cl.per = 0;   // no cells to list
   hipLaunchKernelGGL(k_vp_beads, dim3(kVpBeadBlocks + (cl.per ? cl.blocks : 0)), dim3(kBlock), 0, c->st, g, c->d, cl,
                      h->zs, h->dw, phantom, h->opart);
-  hipLaunchKernelGGL(k_vp_pairs, dim3(c->full_cells, c->full_groups, c->full_parts), dim3(kBlock), 0, c->st, g, c->d,
-                     cl, h->dw, phantom, c->full_parts, h->ppart);
+  if (direct)
+    hipLaunchKernelGGL(k_vp_pairs_lj, dim3(dblocks), dim3(kBlock), 0, c->st, g, c->d, h->zs, phantom, h->ppart);
+  else
+    hipLaunchKernelGGL(k_vp_pairs, dim3(c->full_cells, c->full_groups, c->full_parts), dim3(kBlock), 0, c->st, g, c->d,
+                       cl, h->dw, phantom, c->full_parts, h->ppart);
   int nkb = 0;
   if (g.use_ewald && h->nk_u > 0) {
     nkb = h->nkb;

@@ -116,15 +116,15 @@ def test_from_scratch_energy_and_cell_order(n_chains, chain_len, salt, L, alpha,
     _full_matches(eng, orc)
 
 
-@pytest.mark.parametrize("L,cell_div", [(100.0, 2), (60.0, 2), (100.0, 1)])
-def test_mostly_empty_cells(L, cell_div):
+@pytest.mark.parametrize("L,cell_div,chains", [(100.0, 2, 5), (60.0, 2, 55), (100.0, 1, 5), (100.0, 2, 55)])
+def test_mostly_empty_cells(L, cell_div, chains):
     """Neutral chains in a box of up to 512,000 cells, several hundred to a block
     of the from-scratch sums and several to a wave of the compaction: energy
-    and pressure sample against the oracle, fresh and after moves (tombstones,
-    two compactions)."""
+    and pressure sample (over the pairs up to 2,048 beads, by cells beyond)
+    against the oracle, fresh and after moves (tombstones, two compactions)."""
     from plum_amd import host
     sd = systems.config("tiny")
-    xyz, q, ty, ms = host.synth_system(5, 40, 0, 0, [L, L, L], 5, bead_q=0.0)
+    xyz, q, ty, ms = host.synth_system(chains, 40, 0, 0, [L, L, L], 5, bead_q=0.0)
     xyz[80:120] = xyz[:40] + [0.4, 0.4, 0.4]     # two chains in the same cells
     sd.update(xyz=xyz, q=q, type=ty, mol_start=ms, box=[L, L, L], use_ewald=0)
     eng = E.Engine(sd, cell_div=cell_div)
@@ -139,6 +139,32 @@ def test_mostly_empty_cells(L, cell_div):
             assert abs(got[k] - ref[k]) <= 1e-14 * scale, (k, got[k], ref[k], scale)
         run, full = eng.totals(), eng.energy_full()
         assert abs(run["lj"] - full["lj"]) <= 1e-10 * scale
+
+
+@pytest.mark.parametrize("npbc,phantom,use_bond", [(3, 0, 1), (2, 6, 1), (3, 4, 0)])
+@pytest.mark.parametrize("length", [10, 130])   # 60 and 780 beads
+def test_volume_perturbation_without_charges(npbc, phantom, use_bond, length):
+    """The LJ part of a pressure sample over the bead pairs: with images, surface
+    sites (which take no part), rigid molecules, beads far outside the box."""
+    from plum_amd import host
+    box = [20.0, 20.0, 14.0]
+    sd = systems.config("slab_small" if npbc == 2 else "tiny")
+    xyz, q, ty, ms = host.synth_system(6, length, 0, 0, box, 5, bead_q=0.0, npbc=npbc, min_sep=0.7,
+                                       z_range=(0.8, box[2] - 0.8) if npbc == 2 else None)
+    if npbc == 3:
+        xyz = xyz + np.array([0.0, 0.0, 2.3 * box[2]])
+    sites = np.c_[np.linspace(1, 19, phantom), np.linspace(1, 19, phantom), np.full(phantom, 7.0)]
+    ms = np.r_[np.arange(phantom), ms + phantom].astype(np.int32)
+    sd.update(xyz=np.r_[sites, xyz], q=np.r_[np.zeros(phantom), q], type=np.r_[np.zeros(phantom), ty].astype(np.int32),
+              mol_start=ms, box=box, use_ewald=0, use_bond=use_bond, dipole=0, grafted=0, phantom=phantom)
+    eng, orc = E.Engine(sd), O.Oracle(sd)
+    got, ref = eng.vp_sample(phantom), orc.vp_sample(phantom)
+    # 1e-14 of the energies, ten times that for coordinates 2.3 edges out (as
+    # in test_volume_perturbation_sizes)
+    scale = 1e-13 * sum(abs(v) for v in orc.energy_full().values())
+    assert abs(ref["lj"]) > 1e3 * scale
+    for k in ("lj", "wall", "bond", "dU"):
+        assert abs(got[k] - ref[k]) <= scale, (k, got[k], ref[k], scale)
 
 
 def test_spring_energy_has_one_set_of_bits():

@@ -175,6 +175,8 @@ int plum_surrogate_enable(plum_ctx* c, const plum_surrogate_params* p) {
       hipMemsetAsync(s->m2, 0, sizeof(float) * kNParams, st) != hipSuccess ||
       hipMemsetAsync(s->sur_x, 0, sizeof(float) * rows * kDescr, st) != hipSuccess ||
       hipMemsetAsync(s->sur_f, 0, sizeof(float) * rows, st) != hipSuccess ||
+      // the ring starts as NaN, so that a row read before it was written shows
+      hipMemsetAsync(s->tr_x, 0xff, sizeof(float) * (size_t)p->ring * 2 * c->maxm * kDescr, st) != hipSuccess ||
       hipMemcpyAsync(s->tr_ctl, ctl, sizeof(ctl), hipMemcpyHostToDevice, st) != hipSuccess)
     return bail(fail(PLUM_E_HIP, "surrogate upload failed"));
   hipLaunchKernelGGL(k_pack_bf16, dim3(nblocks(kHid * kHid)), dim3(kBlock), 0, st, s->w32, s->net);

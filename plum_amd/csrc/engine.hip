@@ -71,6 +71,7 @@ struct plum_ctx {
   CbmcHost* cbmc = nullptr;    // configurational-bias trial buffers
   VpHost* vp = nullptr;        // volume-perturbation pressure buffers
   int screen_cap = kMaxProp;   // proposal slots allocated
+  double self_img = 0;   // real-space energy of a unit charge and its own images
   double *epart_k = nullptr, *opart = nullptr;   // from-scratch k-space / springs, walls, self, dipole partials
   int *d_max = nullptr, *h_max = nullptr;        // largest cell count (device, pinned host)
   std::vector<int> mol_start;
@@ -161,6 +162,25 @@ void derive_cutoffs(const plum_params& p, plum_info& info) {
     repl_cutoff += alpha;
   info.repl_cutoff = repl_cutoff;
   for (int i = 0; i < 3; i++) info.repl_cell[i] = (int)ceil(sqrt(repl_cutoff) * box[i] / (2 * kPi));
+}
+
+// Real-space energy of a unit charge with its own images (half of each pair;
+// potential_ewald_coul.cc:134-164 at separation 0) where the period along z is
+// Lz: whole edges, exactly, since an edge may equal the cutoff (both are often
+// whole numbers).
+long double self_images(const plum_ctx* c, double Lz) {
+  const Geo& g = c->g;
+  if (!g.use_ewald) return 0;
+  const long double sa = g.sqrt_alpha;
+  long double e = 0;
+  for (int i = -g.real_cell[0]; i <= g.real_cell[0]; i++)
+    for (int j = -g.real_cell[1]; j <= g.real_cell[1]; j++)
+      for (int k = -g.real_cell[2]; k <= g.real_cell[2]; k++) {
+        const double x = i * g.L[0], y = j * g.L[1], z = k * Lz;
+        const double r = sqrt(x * x + y * y + z * z);
+        if (r > 0 && r <= g.rc) e += erfcl(sa * r) / r;
+      }
+  return 0.5L * g.lB * e;
 }
 
 // Most blocks of the full real-space kernel with a block per cell, and blocks
@@ -307,7 +327,8 @@ int run_full(plum_ctx* c, int set_running, double out[8]) {
     hipLaunchKernelGGL(k_full_sk_reduce, dim3(c->nkb_full), dim3(kBlock), 0, c->st, g, c->d, c->nchunk,
                        c->epart_k);
   }
-  hipLaunchKernelGGL(k_full_small, dim3(kFullSmall), dim3(kBlock), 0, c->st, g, c->d, (int)full_partials(c), c->opart);
+  hipLaunchKernelGGL(k_full_small, dim3(kFullSmall), dim3(kBlock), 0, c->st, g, c->d, (int)full_partials(c),
+                     c->self_img, c->opart);
   hipLaunchKernelGGL(k_full_final, dim3(1), dim3(kFinalThreads), 0, c->st, g, c->d, ksp ? c->nkb_full : 0,
                      kFullSmall, c->epart_k, c->opart, set_running);
   HIPCHK(hipGetLastError());
@@ -498,6 +519,7 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
   if (g.rs <= 0) g.rs = 1.0;
   g.rs2 = g.rs * g.rs;
   g.lj2_max = lj_max * lj_max * (1 + 1e-12);
+  c->self_img = (double)self_images(c, g.L[2]);
 
   // cell grid: edge ~ rs / div
   set_cell_grid(c, p.cell_div > 0 ? p.cell_div : 2);

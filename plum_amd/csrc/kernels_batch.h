@@ -768,7 +768,9 @@ struct QueryShare {
 // skipping the index range [mlo, mhi] (the device loop's moves are
 // contiguous), over share `part` of `nparts` of the query's cells.  Not
 // Q_MOVED: the points are beads of the list themselves, own their indices, and
-// each pair counts once (LJ needs no self images: they lie beyond its cutoff).
+// each pair counts once; a bead's own images are left to the caller (theirs are
+// whole edges away, and an edge may be the cutoff itself, where the rounding of
+// a position would decide).
 // Q_STRETCH: each pair's stretched minus current energy, over the pairs within
 // the cutoff in either (the search reaches kStretchMargin further, more than
 // a separation changes).  Each wave's part of the result valid in its lane 0.
@@ -1015,16 +1017,14 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
           n2 = dx * dx + dy * dy + dn * dn;
         }
         // FP64 queue: every charged pair (P = 0), the close ones (P = 1)
-        // ALL: a pair counts from its lower index, a bead's own images by half
+        // ALL: a pair counts from its lower index
         const int own = ALL ? sh.s_own[i] : -1;
-        const bool self = ALL && j == own;
-        const bool in = r2 <= rcj2 && (!ALL || j > own || (self && r2 > 0)) &&
-                        (!STR || stretch_pair(sh.s_cls[i], cj));
+        const bool in = r2 <= rcj2 && (!ALL || j > own) && (!STR || stretch_pair(sh.s_cls[i], cj));
         const bool near = in && (P == 0 || r2 < fp64_b2);
         const unsigned long long m = __ballot(near);
         if (m) {
           if (near) {
-            sm.s_q[qn + lanes_below(m)] = make_double2(r2, self ? 0.5 * (qp.w * qj) : qp.w * qj);
+            sm.s_q[qn + lanes_below(m)] = make_double2(r2, qp.w * qj);
             if constexpr (STR) sm.s_qn[qn + lanes_below(m)] = n2;
           }
           qn += __popcll(m);

@@ -81,8 +81,7 @@ __global__ __launch_bounds__(kBlock) void k_cell_order(Geo g, Dev d) {
 // ============================================================ from scratch
 // Real space + LJ over all pairs: the cluster queries of the device loop with
 // the beads of a cell, kCluster slots at a time, as the points.  Every ordered
-// pair is tested and a pair counted from its lower index (a bead's own images
-// with weight 1/2), which costs more distance tests than one thread per slot
+// pair is tested and a pair counted from its lower index, which costs more distance tests than one thread per slot
 // that walks the cells around it, and none of its waits: 2.6 ms for 40,000
 // beads, and 8.5 ms for 3,200 beads in a box of 1.4 r_c, that way.
 // Block (cells, slot group, share of the query's cells); its cells are cell
@@ -296,12 +295,13 @@ __device__ double molecule_spring_wave(const Geo& g, const Dev& d, int a, int b)
 }
 
 // Springs per molecule (a wave each, grid-stride), wall, self and dipole sums
-// over the beads and the sum of k_full_real's partials: block partials opart[6 b
-// ..] = springs, wall, self, M_z, LJ, real space.  (One block over all molecules
+// over the beads, the real-space sum of a bead's own images (self_img q^2) and
+// the sum of k_full_real's partials: block partials opart[6 b ..] = springs,
+// wall, self, M_z, LJ, real space.  (One block over all molecules
 // in turn: 3.7 ms for 20,200 molecules; one block over 68,000 partials: 25 us of
 // the 32 of k_full_final.)
 constexpr int kSmallSums = 6;
-__global__ __launch_bounds__(kBlock) void k_full_small(Geo g, Dev d, int nrealp, double* opart) {
+__global__ __launch_bounds__(kBlock) void k_full_small(Geo g, Dev d, int nrealp, double self_img, double* opart) {
   __shared__ double sh[kBlock / kWave];
   const int lane = threadIdx.x % kWave;
   double eb = 0;
@@ -314,14 +314,14 @@ __global__ __launch_bounds__(kBlock) void k_full_small(Geo g, Dev d, int nrealp,
         eb += e;
       }
     }
-  double ew = 0, es = 0, mz = 0;
+  double ew = 0, es = 0, mz = 0, el = 0, er = 0;
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < g.n; i += gridDim.x * kBlock) {
     const double qi = d.q[i];
     if (g.use_ext) ew += wall_energy(d.z[i], d.wall[d.type[i]], g);
     es += g.self_coef * qi * qi;
+    er += self_img * qi * qi;
     mz += qi * d.z[i];
   }
-  double el = 0, er = 0;
 #pragma unroll 4
   for (int b = blockIdx.x * kBlock + threadIdx.x; b < nrealp; b += gridDim.x * kBlock) {
     const double2 e = d.fpart[b];

@@ -33,12 +33,12 @@ __device__ double vp_z(const Geo& g, const Dev& d, int j) {
 
 // Everything that goes over the beads, in one launch (a sample of a small
 // system is launches): stretched z (zs), the displacement of the image that the
-// cell list holds (dw), and block partials part[4 b ..] of the walls (mobile
-// beads), the springs (each bond's change) and the dipole moments before and
-// after.  Blocks past kVpBeadBlocks list the cells of k_vp_pairs.
-constexpr int kVpBeadBlocks = 128;
+// cell list holds (dw), and block partials part[5 b ..] of the walls (mobile
+// beads), the springs (each bond's change), the dipole moments before and after
+// and the change of the mobile beads' own images (dself q^2).  Blocks past kVpBeadBlocks list the cells of k_vp_pairs.
+constexpr int kVpBeadBlocks = 128, kVpSums = 5;
 __global__ __launch_bounds__(kBlock) void k_vp_beads(Geo g, Dev d, CellList cl, double* zs, double* dw, int phantom,
-                                                     double* part) {
+                                                     double dself, double* part) {
   __shared__ double sh[kBlock / kWave];
   if (blockIdx.x >= kVpBeadBlocks) {
     scan_cells(g, d, cl, blockIdx.x - kVpBeadBlocks);
@@ -46,7 +46,7 @@ __global__ __launch_bounds__(kBlock) void k_vp_beads(Geo g, Dev d, CellList cl, 
   }
   Geo gs = g;
   gs.Lsim[2] = g.Lsim[2] + kDz;
-  double ew = 0, eb = 0, mo = 0, mn = 0;
+  double ew = 0, eb = 0, mo = 0, mn = 0, es = 0;
   for (int j = blockIdx.x * kBlock + threadIdx.x; j < g.n; j += kVpBeadBlocks * kBlock) {
     const int m = d.mol_of[j];
     const double z = d.z[j], zn = vp_z(g, d, j);
@@ -58,19 +58,21 @@ __global__ __launch_bounds__(kBlock) void k_vp_beads(Geo g, Dev d, CellList cl, 
       const WallType w = d.wall[d.type[j]];
       ew += wall_energy(zn, w, gs) - wall_energy(z, w, g);
     }
-    mo += d.q[j] * z;
-    mn += d.q[j] * zn;
+    const double q = d.q[j];
+    if (m >= phantom) es += dself * q * q;
+    mo += q * z;
+    mn += q * zn;
     if (g.use_bond && j + 1 < d.mol_start[m + 1]) {
       const double dx = d.x[j] - d.x[j + 1], dy = d.y[j] - d.y[j + 1], dz = z - d.z[j + 1];
       const double disp1 = vp_z(g, d, j + 1) - d.z[j + 1];
       eb += spring_energy(g, dx, dy, dz + (disp - disp1)) - spring_energy(g, dx, dy, dz);
     }
   }
-  const double v4[4] = {ew, eb, mo, mn};
+  const double v[kVpSums] = {ew, eb, mo, mn, es};
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const double t = block_sum<kBlock>(v4[k], sh);
-    if (threadIdx.x == 0) part[4 * blockIdx.x + k] = t;
+  for (int k = 0; k < kVpSums; k++) {
+    const double t = block_sum<kBlock>(v[k], sh);
+    if (threadIdx.x == 0) part[kVpSums * blockIdx.x + k] = t;
   }
 }
 
@@ -229,7 +231,7 @@ __global__ __launch_bounds__(kFinalThreads) void k_vp_final(Geo g, const double2
                                                             const double* __restrict__ ekpart, int nkb,
                                                             const double* __restrict__ opart, int nob, double* out) {
   __shared__ double sh[kFinalThreads / kWave];
-  double pe = 0, pl = 0, kk = 0, vo[4] = {0, 0, 0, 0};
+  double pe = 0, pl = 0, kk = 0, vo[kVpSums] = {0, 0, 0, 0, 0};
 #pragma unroll 4
   for (int b = threadIdx.x; b < npp; b += kFinalThreads) {
     pl += ppart[b].x;
@@ -238,12 +240,12 @@ __global__ __launch_bounds__(kFinalThreads) void k_vp_final(Geo g, const double2
   for (int b = threadIdx.x; b < nkb; b += kFinalThreads) kk += ekpart[b];
   for (int b = threadIdx.x; b < nob; b += kFinalThreads)
 #pragma unroll
-    for (int k = 0; k < 4; k++) vo[k] += opart[4 * b + k];
+    for (int k = 0; k < kVpSums; k++) vo[k] += opart[kVpSums * b + k];
   const double t_ew = block_sum<kFinalThreads>(vo[0], sh);
   const double t_eb = block_sum<kFinalThreads>(vo[1], sh);
   const double t_mo = block_sum<kFinalThreads>(vo[2], sh);
   const double t_mn = block_sum<kFinalThreads>(vo[3], sh);
-  const double t_pe = block_sum<kFinalThreads>(pe, sh);
+  const double t_pe = block_sum<kFinalThreads>(pe + vo[4], sh);
   const double t_pl = block_sum<kFinalThreads>(pl, sh);
   const double t_kk = block_sum<kFinalThreads>(kk, sh);
   if (threadIdx.x == 0) {

@@ -10,6 +10,7 @@ struct VpHost {
   int4* kl_u = nullptr;       // half-space l vectors in the current or the stretched k list
   double *c_old = nullptr, *c_new = nullptr, *dc = nullptr;   // c_k of each box (0: not in its list), c' - c
   int nk_u = 0;
+  double dself = 0;           // stretched minus current energy of a unit charge and its own images
   double2* skpart = nullptr;  // S(k) and dS(k) partials [chunk][6][k]
   double *ekpart = nullptr, *out = nullptr;
   double* h_out = nullptr;    // pinned
@@ -74,6 +75,7 @@ int vp_setup(plum_ctx* c) {
           dcv.push_back(d);
         }
   }
+  h->dself = (double)(self_images(c, g.L[2] + kDz) - self_images(c, g.L[2]));
   h->nk_u = (int)kl.size();
   const int nk = std::max(h->nk_u, 1);
   h->nkb = (nk + kBlock - 1) / kBlock;
@@ -84,7 +86,7 @@ int vp_setup(plum_ctx* c) {
   h->nchunk = (g.n + h->chunk - 1) / h->chunk;
   CHK(dalloc(c, &h->zs, (size_t)g.n));
   CHK(dalloc(c, &h->dw, (size_t)g.n));
-  CHK(dalloc(c, &h->opart, 4 * (size_t)kVpBeadBlocks));
+  CHK(dalloc(c, &h->opart, kVpSums * (size_t)kVpBeadBlocks));
   CHK(dalloc(c, &h->kl_u, (size_t)nk));
   CHK(dalloc(c, &h->c_old, (size_t)nk));
   CHK(dalloc(c, &h->c_new, (size_t)nk));
@@ -130,7 +132,7 @@ extern "C" int plum_vp_sample(plum_ctx* c, int phantom, plum_vp* out) {
   CellList cl = full_cells(c);
   if (direct) cl.per = 0;   // no cells to list
   hipLaunchKernelGGL(k_vp_beads, dim3(kVpBeadBlocks + (cl.per ? cl.blocks : 0)), dim3(kBlock), 0, c->st, g, c->d, cl,
-                     h->zs, h->dw, phantom, h->opart);
+                     h->zs, h->dw, phantom, h->dself, h->opart);
   if (direct)
     hipLaunchKernelGGL(k_vp_pairs_lj, dim3(dblocks), dim3(kBlock), 0, c->st, g, c->d, h->zs, phantom, h->ppart);
   else

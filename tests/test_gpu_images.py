@@ -100,3 +100,20 @@ def test_slab_thinner_than_the_cutoff(L, length, dipole, cell_div):
         r["evaluated"] = False
     assert replay(sd, recs, 1e-10)[3] >= 50
     _full_matches(eng, O.Oracle(dict(sd, xyz=eng.positions())))
+
+
+@pytest.mark.parametrize("box,npbc", [([6.0, 6.0, 6.0], 3), ([12.0, 12.0, 12.0], 3), ([9.0, 13.0, 18.0], 3),
+                                      ([9.0, 9.0, 9.0], 2)])
+def test_box_edge_equal_to_the_cutoff(box, npbc):
+    """The derived cutoff is a whole number, and so are many boxes: a bead's own
+    images then lie at the cutoff exactly, inside it (r <= r_c) in the energy,
+    and the ones along z outside it in the stretched box."""
+    sd = systems.config("slab_small" if npbc == 2 else "tiny")
+    xyz, q, ty, ms = host.synth_system(4, 5, 20, 0, box, 3, npbc=npbc,
+                                       z_range=(0.8, box[2] - 0.8) if npbc == 2 else None)
+    sd.update(xyz=xyz, q=q, type=ty, mol_start=ms, box=box, alpha=systems.alpha_for_cutoff(box[0]), dipole=0,
+              grafted=0)
+    eng, orc = E.Engine(sd), O.Oracle(sd)
+    assert eng.info().real_cutoff == box[0]
+    ref = _full_matches(eng, orc)
+    _vp_matches(eng, orc, sum(abs(v) for v in ref.values()))

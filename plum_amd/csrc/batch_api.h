@@ -201,7 +201,6 @@ int batch_upload_state(plum_batch* b) {
     q.qfill = b->n_cu * std::min(b->comp_occ, b->tune.blocks_per_cu) * kQWaves;
     q.qmax = query_split(c->cand, kQShare, b->tune.split_div);
     q.qfine = query_split(c->cand, kQFine, b->tune.split_div);
-    q.ncell = c->g.ncell;
     q.pmax = b->tune.pmax;
     q.maxm = c->maxm;
     const int ncl = std::min(kMaxProp, q.pmax) * query_clusters(c->maxm);
@@ -209,7 +208,6 @@ int batch_upload_state(plum_batch* b) {
     b->work += 2LL * ncl * query_spread(q.qmax, q.qfine, ncl, q.qfill) + std::min(kMaxProp, q.pmax) * (long long)q.nkb_s;
     q.nmmb = c->nmmb;
     q.rstride = query_blocks(c->maxm, kMaxQBlock) * kQWaves;
-    q.xcap = c->xcap;
     q.da = b->da ? 1 : 0;
     q.train = (b->da && r == 0) ? 1 : 0;
     q.fill = q.train ? b->reps[0]->sur->p.fill : 0;

@@ -65,7 +65,6 @@ struct plum_ctx {
   int cell_div = 2;      // cells per search radius and dimension
   int grid_gen = 0;      // bumped by every re-grid (batches re-upload their copies)
   int nkb_s = 0;         // k-space tiles of the speculative loop
-  int xcap = 0;          // cross-term partial capacity
   plum_batch* self = nullptr;  // this system as a batch of one (device loop)
   SurHost* sur = nullptr;      // delayed-acceptance surrogate (null when off)
   CbmcHost* cbmc = nullptr;    // configurational-bias trial buffers
@@ -530,9 +529,7 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
   info.n_k_full = 0;
   if (p.use_ewald) {
     const int* n3 = info.repl_cell;
-    // (the z tables always hold l_z = 1, the step of the speculative
-    // k-space's z recurrence)
-    g.nkx = n3[0]; g.nky = n3[1]; g.nkz = std::max(n3[2], 1);
+    g.nkx = n3[0]; g.nky = n3[1]; g.nkz = n3[2];
     const double pref0 = p.lB / (kPi * info.vol_e) * (4 * kPi * kPi);
     for (int lx = -n3[0]; lx <= n3[0]; lx++)
       for (int ly = -n3[1]; ly <= n3[1]; ly++)
@@ -638,8 +635,7 @@ int plum_create(const plum_params* params, int n, const double* xyz, const doubl
   ALLOC(erfc32_d, kErfcNodes);
   g.erfc_tab32 = erfc32_d;
   ALLOC(d.part_ks, (size_t)kMaxProp * std::max(1, c->nkb_s) * kQWaves);
-  c->xcap = kMaxPairs * cross_blocks(maxm, maxm);
-  ALLOC(d.part_x, c->xcap);
+  ALLOC(d.part_x, kMaxPairs * cross_blocks(maxm, maxm));
   ALLOC(d.ctl, 1);
   set_cand(c);
   // room for any split (the batch autotuner may change it)

@@ -54,7 +54,7 @@ struct Geo {
   double fp64_below;    // FP32 path: pairs closer than this use FP64 math
   int single_image;     // only the minimum image can lie within rc (real_pair)
   const double2* erfc_tab;  // erfc nodes (erfc_nodes), kErfcNodes entries
-  const float2* erfc_tab32;  // the same nodes rounded to FP32 (erfc_nodes32)
+  const float2* erfc_tab32;  // the same nodes rounded to FP32 (erfc_from_node32)
 };
 
 // FP64 erfc(x), x >= 0, by the Taylor series about the nearest tabulated
@@ -146,11 +146,6 @@ __device__ __forceinline__ float erfc_from_node32(float x, int i, float2 node) {
   return node.x - node.y * s;
 }
 
-__device__ __forceinline__ float erfc_nodes32(const Geo& g, float x) {
-  const int i = erfc_node_index32(x);
-  return erfc_from_node32(x, i, g.erfc_tab32[i]);
-}
-
 // LJ pair table entry for (ti, tj): sigma, epsilon, cutoff distance (strict
 // r < cut), energy shift; computed on the host with the reference's own
 // expressions (potential_truncated_lj.cc:49-85).
@@ -222,18 +217,6 @@ __device__ __forceinline__ void wave_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// The reference's minimum-image difference vector b - a
-// (GetDistVector, misc.cc:43-56).
-__device__ __forceinline__ void min_image(const double* a, const double* b,
-                                          const double* L, int npbc, double* d) {
-#pragma unroll
-  for (int i = 0; i < 3; i++) {
-    double di = b[i] - a[i];
-    if (i < npbc) di -= L[i] * round(di / L[i]);
-    d[i] = di;
-  }
 }
 
 // Bead::BBDist (bead.cc:162-176).
@@ -310,10 +293,11 @@ __device__ __forceinline__ void sqrt_rsqrt(double r2, double& r, double& rinv) {
   rinv = fma(fma(-g, z, 1.0), z, z);
 }
 
-// Minimum-image separation b - a in the Ewald box (x, y and, with three
-// periodic dimensions, z), the quotient taken with the reciprocal edge: it
-// differs from min_image only where |d| is half an edge to the last bit, and
-// there both images are in the image sum or both are beyond every cutoff.
+// Minimum-image separation b - a in the Ewald box (GetDistVector, misc.cc:43-56:
+// x, y and, with three periodic dimensions, z), the quotient taken with the
+// reciprocal edge: it differs from the reference's only where |d| is half an
+// edge to the last bit, and there both images are in the image sum or both are
+// beyond every cutoff.
 __device__ __forceinline__ void min_image_inv(const double* a, const double* b, const double* L, const double* inv_L,
                                               int npbc, double* d) {
 #pragma unroll
@@ -331,9 +315,8 @@ __device__ __forceinline__ void min_image_inv(const double* a, const double* b, 
 // rc are visited (the test widened by a rounding margin), in the order of the
 // full loop, so the sum is the full loop's: the others add
 // nothing.  In a box with 2 rc > L (27 images) one or two offsets a dimension
-// remain, and a pair costs its in-range images instead of 27 square roots (the
-// pressure sample of 3,200 beads with r_c = 42 and L = 60, 5.1 million pairs:
-// 824 -> 645 us).
+// remain, and a pair costs its in-range images instead of 27 square roots (5.1
+// million pairs with r_c = 42 and L = 60: 432 -> 250 us).
 __device__ inline double real_images(const double* d, const double* L, const double* inv_L, const Geo& g) {
   const double rcw = g.rc * (1 + 1e-9), rc2w = rcw * rcw;
   int lo[3], hi[3];

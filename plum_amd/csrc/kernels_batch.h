@@ -22,7 +22,7 @@
 //                    S(k).
 //   k_compute_spec   all systems' k-space blocks (dS_e(k) of every exact slot
 //                    and its dE_k per k tile), real-space query blocks
-//                    (cluster queries by waves) and moved-moved blocks per
+//                    (cluster queries by blocks) and moved-moved blocks per
 //                    slot, and cross blocks (LJ + real pairs between two
 //                    slots' moved beads, old/new combinations), spread over
 //                    one grid.
@@ -54,12 +54,10 @@ constexpr int kKTile = 16;             // rows and l_z of a speculative k-space 
 struct RepCfg {
   int nkb_s;    // k-space tiles (0 without Ewald)
   int qmax, qfine;   // blocks of a real-space query, ordinary and on an idle chip (query_split)
-  int ncell;    // cells
   int pmax;     // proposals per batch (<= kMaxProp, <= kMaxScreen with the surrogate)
   int maxm;     // moved-list capacity per proposal (longest molecule)
   int nmmb;     // moved-moved block capacity per exact slot
   int rstride;  // real-space partials per exact slot
-  int xcap;     // cross-term partial capacity
   int da;       // delayed acceptance on
   int fill;     // exact slots given to first-stage rejections (training data)
   float r_d;    // descriptor radius of the surrogate

@@ -116,6 +116,30 @@ def test_from_scratch_energy_and_cell_order(n_chains, chain_len, salt, L, alpha,
     _full_matches(eng, orc)
 
 
+def test_from_scratch_kspace_of_long_phase_rows():
+    """A box 200 times as long as wide: a bead's phase table has 839 entries, four
+    of which do not fit the LDS stage of the S(k) tiles, so S(k) is summed a
+    thread per vector; and the trial move's k space with such rows."""
+    sd = systems.config("tiny")
+    box = [6.0, 6.0, 1300.0]
+    xyz, q, ty, ms = systems.build_bulk(4, 5, 20, None, 3, box=box)
+    sd.update(xyz=xyz, q=q, type=ty, mol_start=ms, box=box, alpha=0.4)
+    eng, orc = E.Engine(sd), O.Oracle(sd)
+    assert sum(eng.info().repl_cell) + 3 > 768
+    _full_matches(eng, orc)
+    idx = np.arange(ms[0], ms[1], dtype=np.int32)
+    orc.set_trial(0, idx, xyz[idx] + 0.3)
+    t_ref, d_ref = orc.delta(0)
+    _, d = eng.delta(0, idx, xyz[idx] + 0.3)
+    eng.finalize(True)
+    for k in E.TERMS:
+        assert abs(d[k] - d_ref[k]) <= 1e-10 * max(abs(d_ref[k]), 1e-2), (k, d[k], d_ref[k])
+    eng.mc_run(64, sd["move_prob"], move_size=1.0, seed=3)
+    run = eng.totals()
+    _full_matches(eng, O.Oracle(dict(sd, xyz=eng.positions())))
+    assert abs(run["kspace"] - eng.energy_full()["kspace"]) <= 1e-10 * abs(run["kspace"])
+
+
 @pytest.mark.parametrize("L,cell_div,chains", [(100.0, 2, 5), (60.0, 2, 55), (100.0, 1, 5), (100.0, 2, 55)])
 def test_mostly_empty_cells(L, cell_div, chains):
     """Neutral chains in a box of up to 512,000 cells, several hundred to a block

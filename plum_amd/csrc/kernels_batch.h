@@ -787,8 +787,11 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
   // the same pair images within the radius), and the points' bounding box.  The
   // image is the point's own wrapped position plus a whole edge or none, as a
   // candidate's is, so that a bead at the same coordinates is at distance 0 to
-  // the bit.  A z that is not periodic stays as wrapped: LJ counts the
-  // candidates of image 0 only, which is the image of the point's own z.
+  // the bit.  Along a z that is not periodic all points move with the first one,
+  // by the edges that wrap it (none inside the slab): LJ counts the candidates of
+  // image 0 only, and a chain may span more than half of the height.  (Each
+  // wrapped on its own, a trial bead behind a wall would stretch the box over
+  // the height: 90 us for the brush's launch instead of 66.)
   const unsigned vm = (unsigned)__ballot(valid) & ((1u << kCluster) - 1u);
   const int np = ALL ? kCluster : __popc(vm);
   const int ref = __builtin_ctz(vm);
@@ -800,8 +803,13 @@ __device__ double2 real_query_cluster(const Geo& g, const Dev& d, const double4&
 #pragma unroll
     for (int k = 0; k < 3; k++) {
       const double rk = lane_double(pw[k], ref);
-      nv[k] = k < g.npbc ? -rint((pw[k] - rk) * g.inv_L[k]) : 0.0;
-      qv[k] = valid ? pw[k] + nv[k] * g.L[k] : rk;
+      double from = pw[k];
+      nv[k] = -rint((pw[k] - rk) * g.inv_L[k]);
+      if (k == 2 && g.npbc < 3) {
+        from = p.z;
+        nv[k] = rint((rk - lane_double(p.z, ref)) * g.inv_L[k]);
+      }
+      qv[k] = valid ? from + nv[k] * g.L[k] : rk;
     }
     if (threadIdx.x < kCluster) {
       // (a point that does not count is out of every candidate's reach)
